@@ -3,39 +3,48 @@
  *
  * Traversal (tg_svo_traverse, tg_sparse_voxel_octree.c:558-740). The
  * reference's node stack is exactly the path from the root to the current
- * node, so a lane keeps only the current node, its level and its integer
- * coordinates; popping walks parent links, and every node box is recomputed
- * from (level, coordinates) with the values the reference's stack holds
- * (integers below 2^24, exact in fp32). Slab quotient pairs (box min, box
- * max) are reduced to the one quotient that min/max would pick, chosen by
- * the sign of the direction component: subtraction and IEEE division are
- * monotone, so the value is the same and half of the divisions disappear.
+ * node, and every node box is an aligned power of two of integers below 2^24,
+ * exact in fp32. So a lane keeps only its leaf-grid cell and the current
+ * node's size, and a move (from one empty child slot or leaf to the next) pops
+ * and descends by comparing cell coordinates (lane_step), with the positions,
+ * advances and step counts of the reference's loop. Slab quotient pairs (box
+ * min, box max) are reduced to the one quotient that min/max would pick,
+ * chosen by the sign of the direction component: subtraction and IEEE division
+ * are monotone, so the value is the same and half of the divisions disappear.
  * The pop test (exit distance > FLT_EPSILON) needs no division at all
  * (axis_exit_gt_eps), and the DDA step lengths 1/|d| are computed once per
  * ray.
  *
  * Layout read by the traversal (written by the SVO build):
- *   inner[n_inner]   uint2 per inner node: first child, parent | valid << 24.
- *                    Held in LDS with the brick masks when both fit.
- *                    Leaves follow the inner nodes in node order, so leaf
- *                    index = node - n_inner,
- *                    and a child is a leaf exactly at the leaf level.
+ *   grid[8^leaf_level] u32 per 32^3 cell of the root: its leaf, or the size of
+ *                    the empty child slot it lies in (SVO_GRID_EMPTY).
  *   bricks[n_leaves] u64 per leaf: one bit per 8^3 brick holding a solid
- *                    voxel. The 32^3 DDA tests the brick bit before it
- *                    loads a bit word, and keeps the last word, so most DDA
- *                    iterations read no memory. Voxels tested and their
- *                    order are the reference's; only loads are skipped.
+ *                    voxel, held in LDS when they fit. The 32^3 DDA tests the
+ *                    brick bit before it loads a bit word, and keeps the last
+ *                    word, so most DDA iterations read no memory. Voxels
+ *                    tested and their order are the reference's; only loads
+ *                    are skipped.
+ * Leaves follow the inner nodes in node order, so a leaf's node is n_inner +
+ * leaf.
  *
  * gi_trace_k is persistent: each lane runs one ray as a state machine
- * whose steps are up to `node_iters` node iterations of the reference's
- * loop while the lane descends, then up to `burst` iterations of the leaf
- * DDA, so lanes of a wave stay busy while they are in different phases
- * (both tuning). In the uncounted DDA, once enough of a wave's walking
- * lanes are in 8^3 bricks without solid voxels, those lanes cross their
- * bricks in one exact step (brick_cross). Whenever `refill` (tuning) lanes
- * of a wave have finished, the wave hands that many new rays to them
- * (ballot + lane rank), from a slice of the queue it took with one atomic
- * (`chunk` rays, tuning).
+ * whose steps are up to `node_iters` moves while the ray is outside the
+ * leaves, then up to `burst` iterations of the leaf DDA, so lanes of a wave
+ * stay busy while they are in different phases (both tuning). In the uncounted
+ * DDA, once enough of a wave's walking lanes are in 8^3 bricks without solid
+ * voxels, those lanes cross their bricks in one exact step (brick_cross).
+ * Whenever `refill` (tuning) lanes of a wave have finished, the wave hands
+ * that many new rays to them (ballot + lane rank), from a slice of the queue
+ * it took with one atomic (`chunk` rays, tuning).
+ *
+ * The kernel is bound by instruction issue: a wave issues what any of its lanes
+ * needs, and a phase runs for 20 to 40 of 64 lanes. Walking the tree took about
+ * 125 instructions per node of a descent and 35 per pop, both in loops as long
+ * as the slowest lane's; a move takes about 165 in all. 512 noise objects at
+ * 1080p, 4 samples a pixel: 3.99 -> 2.97 ms, the 4096-object 16-camera frame
+ * 92.5 -> 58.3 ms (2 moves and a 12-iteration burst a step, brick crossing from
+ * half of the walking lanes; 1, 3 moves 3.16, 3.04 ms, bursts of 8 and 16 3.06
+ * and 2.95 ms against 2.93).
  *
  * GI frame (estimator documented at tgx_gi_params in tgx.h):
  *   gi_gen_k     surface of each visible pixel, spp bounce rays at
@@ -63,21 +72,19 @@
 
 #define TRACE_BLOCK 1024
 #define DDA_BURST 8u
-#define TRACE_ADV_MIN 16u   /* lanes of a wave that make it run the advances */
-#define TRACE_LDS_NODES_MAX 8000u   /* inner nodes + leaf brick masks in LDS (64000 B) */
+#define TRACE_LDS_LEAVES_MAX 8000u  /* leaf brick masks in LDS (64000 B) */
 
 /* ------------------------------------------------------------------------ */
 /* Traversal                                                                */
 /* ------------------------------------------------------------------------ */
 
 struct trace_params {
-    const uint2*              inner;
+    const uint32_t*           grid;
     const unsigned long long* bricks;
     const uint32_t*           leaf_bits;
-    uint32_t                  n_inner;
+    uint32_t                  n_inner;       /* index of the first leaf node */
     uint32_t                  n_leaves;
-    uint32_t                  depth;
-    uint32_t                  leaf_level;
+    uint32_t                  leaf_level;    /* 2^leaf_level cells per axis */
     float                     mnx, mny, mnz;
     float                     half;          /* 2^depth / 2 */
     float                     cx, cy, cz;    /* root centre, min + half */
@@ -123,11 +130,11 @@ __device__ static inline float box_exit(float px, float py, float pz, float dx, 
                  axis_far(pz, dz, mnz, mnz + side));
 }
 
-/* box_exit(...) > SVO_EPSILON for one axis, without dividing. fl(a / d) >
- * 2^-23 holds exactly when a / d > 2^-23 (1 + 2^-24), the midpoint to the
- * next float (a tie rounds to the even 2^-23). For a normal t = d 2^-23 no
- * float lies in (|t|, |t| (1 + 2^-24)], so the test is a > t for d > 0 and
- * a < t for d < 0. Components with |d| < 2^-100 take the division. */
+/* box_exit(...) > SVO_EPSILON for one axis of the box [mn, mx]. For 2^-100
+ * <= |d| no division: fl(a / d) > 2^-23 holds exactly when a / d > 2^-23
+ * (1 + 2^-24), the midpoint to the next float (a tie rounds to the even
+ * 2^-23), and for a normal t = d 2^-23 no float lies in (|t|, |t| (1 +
+ * 2^-24)], so the test is a > t for d > 0 and a < t for d < 0. */
 __device__ static inline bool axis_exit_gt_eps(float p, float d, float mn, float mx)
 {
     if (d == 0.0f) return true; /* quotient F32_MAX */
@@ -147,28 +154,17 @@ __device__ static inline float dda_len(float pos, float neg, float d)
 /* -1, 0 or 1 */
 __device__ static inline int dir_step(float d) { return d > 0.0f ? 1 : (d < 0.0f ? -1 : 0); }
 
-/* Per-lane ray state (22 registers). `node` packs the current node's
- * coordinates (7 bits each: inner nodes sit at level <= depth - 6 <= 7), its
- * level, the child slot being visited and the DDA phase flag; `vox` packs
+/* Per-lane ray state. `node` packs the leaf-grid cell the ray is in (8 bits
+ * an axis), the current node's size S (it spans 2^S cells an axis; S <= 8)
+ * and the phase flags; the node is the one holding the cell. Outside a leaf
+ * the ray is in an empty child slot of it, 2^(S - 1) cells wide. `vox` packs
  * the leaf DDA voxel and iteration count. */
-/* axis_exit_gt_eps as a 0/1 integer for |d| >= 2^-100 or d == 0: the sign of
- * the exact-sign difference a - t (IEEE subtraction is 0 only for equal
- * operands, and rounding keeps the sign). Callers handle |d| < 2^-100. */
-__device__ static inline uint32_t axis_exit_fast(float p, float d, float mn, float mx)
-{
-    const float a = (d > 0.0f ? mx : mn) - p;
-    const float t = d * 0x1p-23f;
-    const float u = d > 0.0f ? a - t : t - a;
-    return u > 0.0f ? 1u : (d == 0.0f ? 1u : 0u);
-}
-
 struct trace_lane {
     float    px, py, pz;   /* position relative to the root centre */
     float    dx, dy, dz;
     float    dist;
     uint32_t steps;
-    uint32_t cur;          /* current node, SVO_NONE once popped empty */
-    uint32_t node;         /* cx | cy << 7 | cz << 14 | lvl << 21 | rc << 24 | dda << 27 */
+    uint32_t node;         /* x | y << 8 | z << 16 | S << 24 | flags */
     uint32_t leaf;         /* leaf index during the DDA */
     uint32_t vox;          /* x | y << 5 | z << 10 | it << 15 */
     float    tmx, tmy, tmz, tdx, tdy, tdz;
@@ -176,19 +172,35 @@ struct trace_lane {
     uint32_t wi, wv;       /* last bit word index and value */
 };
 
-#define ND_CX(n)  ((n) & 127u)
-#define ND_CY(n)  (((n) >> 7) & 127u)
-#define ND_CZ(n)  (((n) >> 14) & 127u)
-#define ND_LVL(n) (((n) >> 21) & 7u)
-#define ND_RC(n)  (((n) >> 24) & 7u)
-#define ND_DDA    (1u << 27)
-#define ND_ADV    (1u << 28)   /* an advance out of the child slot is pending */
-#define ND_SETUP  (1u << 29)   /* entered a leaf: its DDA is set up at the lane's next burst */
+#define ND_X(n)   ((n) & 255u)
+#define ND_Y(n)   (((n) >> 8) & 255u)
+#define ND_Z(n)   (((n) >> 16) & 255u)
+#define ND_S(n)   (((n) >> 24) & 15u)
+#define ND_DDA    (1u << 28)
+#define ND_ADV    (1u << 29)   /* an advance out of the child slot is pending */
+#define ND_SETUP  (1u << 30)   /* entered a leaf: its DDA is set up at the lane's next burst */
+#define ND_ODD    (1u << 31)   /* direction outside move_axis' range */
 
 __device__ static inline svo_res res_miss(uint32_t steps)
 {
     svo_res r = {SVO_F32_MAX, SVO_NONE, 0u, 0u, steps, 0u};
     return r;
+}
+
+/* ND_ODD for a ray whose direction components are not all 0 or in [2^-100,
+ * 2^26) with one of them not 0, or whose position is not finite. Such rays
+ * take the reference's pop test node by node and the counted leaf DDA: they
+ * may not move at all, so only its iteration cap is sure to end the walk. Any
+ * other ray stays as it is: a move changes each coordinate by at most its
+ * node's size. */
+__device__ static inline uint32_t ray_odd(const trace_lane& L)
+{
+    const float ax = fabsf(L.dx), ay = fabsf(L.dy), az = fabsf(L.dz);
+    const bool ok = (ax == 0.0f || (ax >= 0x1p-100f && ax < 0x1p26f)) &&
+                    (ay == 0.0f || (ay >= 0x1p-100f && ay < 0x1p26f)) &&
+                    (az == 0.0f || (az >= 0x1p-100f && az < 0x1p26f)) && fmaxf(fmaxf(ax, ay), az) > 0.0f &&
+                    fabsf(L.px) < SVO_INF && fabsf(L.py) < SVO_INF && fabsf(L.pz) < SVO_INF;
+    return ok ? 0u : ND_ODD;
 }
 
 /* Ray setup (tg_sparse_voxel_octree.c:570-594) for the ray whose world-space
@@ -198,8 +210,7 @@ __device__ static inline bool lane_init_self(const trace_params& P, float half, 
 {
     const float ox = L.px - P.cx, oy = L.py - P.cy, oz = L.pz - P.cz;
     L.steps = 0;
-    L.cur = 0;
-    L.node = 0;
+    L.node = P.leaf_level << 24;
     if (!have_td) {
         L.tdx = dda_len(1.0f, 1.0f, L.dx);
         L.tdy = dda_len(1.0f, 1.0f, L.dy);
@@ -211,6 +222,7 @@ __device__ static inline bool lane_init_self(const trace_params& P, float half, 
          * origin with distance 0 */
         L.px = ox; L.py = oy; L.pz = oz;
         L.dist = 0.0f;
+        L.node |= ray_odd(L);
         return true;
     }
     const float enter = fmax2(fmax2(axis_near(ox, L.dx, -half, half), axis_near(oy, L.dy, -half, half)),
@@ -221,23 +233,17 @@ __device__ static inline bool lane_init_self(const trace_params& P, float half, 
     L.px = ox; L.py = oy; L.pz = oz;
     if (enter > 0.0f) { L.px = ox + L.dx * enter; L.py = oy + L.dy * enter; L.pz = oz + L.dz * enter; }
     L.dist = enter > 0.0f ? enter : 0.0f;
+    L.node |= ray_odd(L);
     return true;
 }
 
-template <bool kLds>
-__device__ static inline uint2 inner_at(const uint2* __restrict__ g, const uint2* s, uint32_t i)
-{
-    if constexpr (kLds) return s[i];
-    else return g[i];
-}
-
-/* Brick masks follow the inner nodes in LDS. */
+/* Brick masks, in LDS when they fit. */
 template <bool kLds>
 __device__ static inline unsigned long long bricks_at(const unsigned long long* __restrict__ g, const uint2* s,
-                                                      uint32_t n_inner, uint32_t leaf)
+                                                      uint32_t leaf)
 {
     if constexpr (kLds) {
-        const uint2 v = s[n_inner + leaf];
+        const uint2 v = s[leaf];
         return ((unsigned long long)v.y << 32) | v.x;
     } else {
         return g[leaf];
@@ -249,43 +255,37 @@ __device__ static inline uint32_t lane_rank(unsigned long long mask)
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-/* Minimum corner of child slot rc of the node packed in n. */
-__device__ static inline void child_min(uint32_t n, uint32_t rc, float half, float cs, float& x, float& y, float& z)
+/* Minimum corner of a lane's leaf. */
+__device__ static inline void leaf_min(uint32_t n, float half, float& x, float& y, float& z)
 {
-    x = -half + (float)(2u * ND_CX(n) + (rc & 1u)) * cs;
-    y = -half + (float)(2u * ND_CY(n) + ((rc >> 1) & 1u)) * cs;
-    z = -half + (float)(2u * ND_CZ(n) + (rc >> 2)) * cs;
+    x = -half + 32.0f * (float)ND_X(n);
+    y = -half + 32.0f * (float)ND_Y(n);
+    z = -half + 32.0f * (float)ND_Z(n);
 }
 
-/* Pops every node the position has left: a wave-uniform loop over the
- * lanes in `adv`, walking parent links; cur / n are the current node and
- * its packed coordinates. kDivide uses the dividing exit test (needed for
- * direction components below 2^-100). */
-template <bool kLds, bool kDivide>
-__device__ static inline void pop_walk(const trace_params& P, const uint2* s_inner, float half, const trace_lane& L,
-                                       bool adv, uint32_t& cur, uint32_t& n)
+/* One axis of a move, in units of leaf-grid cells (32 voxels). For the
+ * position p and direction d along the axis:
+ *   k  the cell the descent picks inside the node: the boundaries below p,
+ *      and the one at p when d > 0 (the reference compares p with each
+ *      node's centre in turn; a node's cells are then a clamp of k);
+ *   e  the cell whose node the ray has not left yet: the pop test keeps a
+ *      node when its far plane B has fl(B - p) > d 2^-23 (see
+ *      axis_exit_gt_eps), a test that is monotone in B and, for |d| < 2^26,
+ *      can only fail for the boundaries nearest p. Seen from cell c the node
+ *      of size 2^s is kept when it holds e as well. */
+__device__ static inline void move_axis(float p, float d, uint32_t off, int c, int& k, int& e)
 {
-    uint32_t popping = adv ? 1u : 0u;
-    while (true) {
-        const uint32_t live = popping & (cur != SVO_NONE ? 1u : 0u);
-        if (!__any(live)) break;
-        const uint32_t lvl = ND_LVL(n);
-        const float ns = (float)(1u << (P.depth - lvl));
-        const float nmx = -half + (float)ND_CX(n) * ns, nmy = -half + (float)ND_CY(n) * ns,
-                    nmz = -half + (float)ND_CZ(n) * ns;
-        uint32_t inside;
-        if constexpr (kDivide)
-            inside = (axis_exit_gt_eps(L.px, L.dx, nmx, nmx + ns) && axis_exit_gt_eps(L.py, L.dy, nmy, nmy + ns) &&
-                      axis_exit_gt_eps(L.pz, L.dz, nmz, nmz + ns)) ? 1u : 0u;
-        else
-            inside = axis_exit_fast(L.px, L.dx, nmx, nmx + ns) & axis_exit_fast(L.py, L.dy, nmy, nmy + ns) &
-                     axis_exit_fast(L.pz, L.dz, nmz, nmz + ns);
-        const uint32_t up = live & (inside ^ 1u);
-        const uint32_t par = inner_at<kLds>(P.inner, s_inner, live ? cur : 0u).y & 0xFFFFFFu;
-        cur = up ? (par == 0xFFFFFFu ? SVO_NONE : par) : cur;
-        n = up ? ((ND_CX(n) >> 1) | ((ND_CY(n) >> 1) << 7) | ((ND_CZ(n) >> 1) << 14) | (((lvl - 1u) & 7u) << 21)) : n;
-        popping = up;
-    }
+    /* beyond 2^24 (and NaN: the lower bound) any value outside the grid does */
+    const int fi = (int)__builtin_amdgcn_fmed3f(floorf(p), -0x1p24f, 0x1p24f) & ~31;
+    const float bf = (float)fi;
+    const int f = (fi >> 5) + (int)off;
+    const bool pos = d > 0.0f;
+    k = f - (bf == p && !pos ? 1 : 0);
+    const float a = (pos ? bf + 32.0f : bf) - p;
+    const float t = d * 0x1p-23f;
+    const int up = f + (a > t ? 0 : 1), down = f - (a < t ? 0 : 1);
+    e = pos ? (up > c ? up : c) : (down < c ? down : c);
+    e = d == 0.0f ? c : e;
 }
 
 /* Exact skip of an 8^3 brick holding no solid voxel: the state of
@@ -412,84 +412,111 @@ __device__ static inline uint32_t brick_cross(int& x, int& y, int& z, float& tmx
     return 1u;
 }
 
-/* One step of a lane: up to node_iters iterations of the reference's node
- * loop while the lane descends, then up to DDA_BURST iterations of the leaf
- * DDA. Returns true when the ray is done; res is then its result. */
+/* One step of a lane: up to node_iters moves (the reference's node loop from
+ * one advance to the next) while the ray is outside the leaves, then up to
+ * `burst` iterations of the leaf DDA. Returns true when the ray is done; res
+ * is then its result.
+ *
+ * A move leaves the empty child slot (or the leaf) the ray is in, pops the
+ * nodes the position has left and descends to the next leaf or empty slot.
+ * The reference walks the tree for that, a node per iteration. Node boxes
+ * are aligned powers of two and both walks ask only where p lies among cell
+ * boundaries, so here the pops are the bits in which two cell coordinates
+ * differ, the descent is one clamp per axis, and the leaf or the size of the
+ * empty slot comes from the leaf grid: one load in place of a chain of node
+ * loads. The iterations the walk would have taken are added to steps. */
 template <bool kLds, bool kSkip = false, uint32_t kDda = 0u>
-__device__ static inline bool lane_step(const trace_params& P, const uint2* s_inner, float half, float maxd,
+__device__ static inline bool lane_step(const trace_params& P, const uint2* s_bricks, float half, float maxd,
                                         trace_lane& L, svo_res& res, bool active, bool allow_node, bool allow_dda,
-                                        bool defer_leave = false, uint32_t cross = 0u, uint32_t node_iters = 1u,
-                                        uint32_t burst = DDA_BURST)
+                                        uint32_t cross = 0u, uint32_t node_iters = 1u, uint32_t burst = DDA_BURST)
 {
-    bool adv = false, done = false;
-    /* a lane with a pending advance waits for the wave's next advance */
-    const bool pend = active && (L.node & ND_ADV);
-    allow_node = allow_node && active && !pend;
-    allow_dda = allow_dda && active && !pend;
-    /* a lane that descended to an inner node may take the next node
-     * iteration in the same step (wave-uniform loop) */
-    bool go = allow_node && !(L.node & ND_DDA);
+    bool done = false;
+    bool mv = allow_node && active && !(L.node & ND_DDA);
+    allow_dda = allow_dda && active;
 #pragma unroll 1
     for (uint32_t ni = 0; ni < node_iters; ni++) {
-        if (ni != 0u && !__any(go)) break;
-        if (go && (L.cur == SVO_NONE || L.steps >= TGX_SVO_MAX_STEPS || L.dist > maxd)) {
-            res = res_miss(L.steps);
-            done = true;
-            go = false;
-            allow_dda = false;
-        }
-        if (go) {
-            /* one iteration of the reference's node loop */
-            L.steps++;
-            const uint2 nd = inner_at<kLds>(P.inner, s_inner, L.cur);
+        if (!__any(mv)) break;
+        if (mv) {
             const uint32_t n = L.node;
-            const uint32_t lvl = ND_LVL(n);
-            const float ps = (float)(1u << (P.depth - lvl));
-            const float ce = ps * 0.5f;
-            const float pmx = -half + (float)ND_CX(n) * ps, pmy = -half + (float)ND_CY(n) * ps,
-                        pmz = -half + (float)ND_CZ(n) * ps;
-            const float hx = pmx + ce, hy = pmy + ce, hz = pmz + ce;
-            uint32_t rc = 0;
-            if (hx < L.px || (L.px == hx && L.dx > 0.0f)) rc |= 1u;
-            if (hy < L.py || (L.py == hy && L.dy > 0.0f)) rc |= 2u;
-            if (hz < L.pz || (L.pz == hz && L.dz > 0.0f)) rc |= 4u;
-            L.node = (n & ~(7u << 24)) | (rc << 24);
-            adv = true;
-            const uint32_t valid = nd.y >> 24;
-            if (valid & (1u << rc)) {
-                const uint32_t ci = nd.x + (uint32_t)__popc(valid & ((1u << rc) - 1u));
-                if (lvl + 1u < P.leaf_level) {
-                    L.cur = ci;
-                    L.node = (2u * ND_CX(n) + (rc & 1u)) | ((2u * ND_CY(n) + ((rc >> 1) & 1u)) << 7) |
-                             ((2u * ND_CZ(n) + (rc >> 2)) << 14) | ((lvl + 1u) << 21);
-                    adv = false;
-                } else {
-                    const uint32_t leaf = ci - P.n_inner;
-                    const unsigned long long bm = bricks_at<kLds>(P.bricks, s_inner, P.n_inner, leaf);
-                    if (bm != 0ull) {
-                        /* the DDA over the 32^3 block starts at the lane's
-                         * next burst (its set-up runs once per step for all
-                         * lanes that entered a leaf) */
-                        L.bm = bm;
-                        L.leaf = leaf;
-                        L.node |= ND_DDA | ND_SETUP;
-                        adv = false;
-                    }
+            uint32_t S = ND_S(n);
+            int cx = (int)ND_X(n), cy = (int)ND_Y(n), cz = (int)ND_Z(n);
+            const bool adv = (n & ND_ADV) != 0u;
+            if (adv) {
+                const uint32_t q = S - 1u;
+                const float cs = (float)(32u << q);
+                const float mx = -half + 32.0f * (float)((cx >> q) << q), my = -half + 32.0f * (float)((cy >> q) << q),
+                            mz = -half + 32.0f * (float)((cz >> q) << q);
+                const float t_adv = box_exit(L.px, L.py, L.pz, L.dx, L.dy, L.dz, mx, my, mz, cs) + SVO_EPSILON;
+                L.px = L.px + L.dx * t_adv;
+                L.py = L.py + L.dy * t_adv;
+                L.pz = L.pz + L.dz * t_adv;
+                L.dist += t_adv;
+            }
+            const uint32_t off = 1u << (P.leaf_level - 1u);
+            int kx, ky, kz, ex, ey, ez;
+            move_axis(L.px, L.dx, off, cx, kx, ex);
+            move_axis(L.py, L.dy, off, cy, ky, ey);
+            move_axis(L.pz, L.dz, off, cz, kz, ez);
+            uint32_t up;
+            if (n & ND_ODD) {
+                /* the reference's test node by node */
+                up = S;
+                while (adv && up <= P.leaf_level) {
+                    const float ns = (float)(32u << up);
+                    const float mx = -half + 32.0f * (float)((cx >> up) << up), my = -half + 32.0f * (float)((cy >> up) << up),
+                                mz = -half + 32.0f * (float)((cz >> up) << up);
+                    if (axis_exit_gt_eps(L.px, L.dx, mx, mx + ns) && axis_exit_gt_eps(L.py, L.dy, my, my + ns) &&
+                        axis_exit_gt_eps(L.pz, L.dz, mz, mz + ns))
+                        break;
+                    up++;
+                }
+            } else {
+                const uint32_t df = adv ? (uint32_t)((cx ^ ex) | (cy ^ ey) | (cz ^ ez)) : 0u;
+                up = 32u - (uint32_t)__clz((int)df);
+                up = up > S ? up : S;
+            }
+            S = up;
+            if (S > P.leaf_level || L.steps >= TGX_SVO_MAX_STEPS || L.dist > maxd) {
+                res = res_miss(L.steps);
+                done = true;
+                mv = false;
+                allow_dda = false;
+            } else {
+                const int m = (1 << S) - 1;
+                kx = max(cx & ~m, min(kx, cx | m));
+                ky = max(cy & ~m, min(ky, cy | m));
+                kz = max(cz & ~m, min(kz, cz | m));
+                const uint32_t cell = (uint32_t)kx | ((uint32_t)ky << P.leaf_level) | ((uint32_t)kz << (2u * P.leaf_level));
+                const uint32_t g = P.grid[cell];
+                const bool leaf = !(g & SVO_GRID_EMPTY);
+                const uint32_t q = leaf ? 0u : g & 15u;
+                /* node iterations of the reference's descent */
+                L.steps += S - q;
+                L.node = (uint32_t)kx | ((uint32_t)ky << 8) | ((uint32_t)kz << 16) | ((q + 1u) << 24) |
+                         (leaf ? ND_DDA | ND_SETUP : ND_ADV) | (n & ND_ODD);
+                L.leaf = g;
+                mv = !leaf;
+                if (L.steps > TGX_SVO_MAX_STEPS) {
+                    /* the cap ends the descent on the way */
+                    res = res_miss(TGX_SVO_MAX_STEPS);
+                    done = true;
+                    mv = false;
+                    allow_dda = false;
                 }
             }
-            go = !adv && !(L.node & ND_DDA);
         }
     }
     /* Up to DDA_BURST iterations of the leaf DDA. The loop is wave-uniform
      * (one __any exit) and lanes that stop are predicated off, which keeps
      * the scalar unit free of per-lane exit bookkeeping. */
-    const bool in_dda = (L.node & ND_DDA) && allow_dda;
+    bool in_dda = (L.node & ND_DDA) && allow_dda;
     if (__any(in_dda && (L.node & ND_SETUP))) {
         if (in_dda && (L.node & ND_SETUP)) {
             /* tg_amanatides_woo setup over the 32^3 block (the child slot's
              * box), entry voxel clamped */
             float cmx, cmy, cmz;
-            child_min(L.node, ND_RC(L.node), half, 32.0f, cmx, cmy, cmz);
+            leaf_min(L.node, half, cmx, cmy, cmz);
+            L.bm = bricks_at<kLds>(P.bricks, s_bricks, L.leaf);
             const float gx = L.px - cmx, gy = L.py - cmy, gz = L.pz - cmz;
             const int x0 = (int)fmin2(fmax2(floorf(gx), 0.0f), 31.0f);
             const int y0 = (int)fmin2(fmax2(floorf(gy), 0.0f), 31.0f);
@@ -523,15 +550,15 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_in
         /* brick skips need every moving axis' t_delta below 2^100 */
         const uint32_t skip_ok = (!kSkip || ((sx == 0 || tdx < 0x1p100f) && (sy == 0 || tdy < 0x1p100f) &&
                                              (sz == 0 || tdz < 0x1p100f))) ? 1u : 0u;
-        /* With every moving axis' t_delta below 2^100 no t_max overflows,
-         * so each step moves a coordinate and the walk leaves the 32^3
-         * block within 94 steps: the iteration cap cannot bind, and a wave
-         * whose DDA lanes all have such directions runs the walk without
-         * counting iterations, two per exit test. A lane's count is then
-         * left behind, which only lanes that never take this path read. */
-        const bool small_td = (sx == 0 || tdx < 0x1p100f) && (sy == 0 || tdy < 0x1p100f) &&
-                              (sz == 0 || tdz < 0x1p100f);
-        if (kDda != 0u && !kSkip && __all(small_td || !in_dda)) {
+        /* Without odd rays every moving axis' t_delta is at most 2^100 and
+         * one axis moves, so no t_max overflows, each step moves a
+         * coordinate and the walk leaves the 32^3 block within 94 steps: the
+         * iteration cap cannot bind, and a wave whose DDA lanes all have such
+         * rays runs the walk without counting iterations, two per exit test.
+         * A lane's count is then left behind, which only lanes that never
+         * take this path read. */
+        const bool regular = !(L.node & ND_ODD);
+        if (kDda != 0u && !kSkip && __all(regular || !in_dda)) {
             /* the count is not kept on this path (see above) */
             it = 0u;
 #pragma unroll 1
@@ -633,21 +660,12 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_in
         hit = hit_i != 0u;
         leave = leave_i != 0u;
         if (in_dda && !hit && !leave) L.vox = (uint32_t)x | ((uint32_t)y << 5) | ((uint32_t)z << 10) | (it << 15);
-        if (leave) {
-            L.node &= ~ND_DDA;
-            adv = true;
-        }
-        /* a lane that left its leaf may leave the advance to a later step
-         * (ND_ADV), taken with other lanes in the same phase */
-        if (defer_leave && leave) {
-            L.node |= ND_ADV;
-            adv = false;
-        }
+        if (leave) L.node ^= ND_DDA | ND_ADV;
     }
     if (hit) {
         /* distance to the voxel's entry plane and the entry face */
         float vmx, vmy, vmz;
-        child_min(L.node, ND_RC(L.node), half, 32.0f, vmx, vmy, vmz);
+        leaf_min(L.node, half, vmx, vmy, vmz);
         vmx = vmx + (float)x; vmy = vmy + (float)y; vmz = vmz + (float)z;
         const float nx = axis_near(L.px, L.dx, vmx, vmx + 1.0f);
         const float ny = axis_near(L.py, L.dy, vmy, vmy + 1.0f);
@@ -664,42 +682,6 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_in
         res.steps = L.steps;
         res.pad = 0u;
         done = true;
-    }
-    /* Advances run for many lanes at once: a lane's advance waits (ND_ADV)
-     * until enough of the wave's active lanes want one. */
-    const bool want = adv || pend;
-    const uint32_t n_want = (uint32_t)__popcll(__ballot(want));
-    const uint32_t n_act = (uint32_t)__popcll(__ballot(active));
-    const bool run_adv = n_want >= TRACE_ADV_MIN || 2u * n_want >= n_act;
-    if (!run_adv && adv) L.node |= ND_ADV;
-    adv = run_adv && want;
-    if (__any(adv)) {
-        /* leave the child box, then pop every node the position has left
-         * (wave-uniform loop, lanes predicated) */
-        uint32_t n = L.node & ~ND_ADV;
-        uint32_t cur = L.cur;
-        if (adv) {
-            const float cs = (float)(1u << (P.depth - ND_LVL(n) - 1u));
-            float cmx, cmy, cmz;
-            child_min(n, ND_RC(n), half, cs, cmx, cmy, cmz);
-            const float t_adv = box_exit(L.px, L.py, L.pz, L.dx, L.dy, L.dz, cmx, cmy, cmz, cs) + SVO_EPSILON;
-            L.px = L.px + L.dx * t_adv;
-            L.py = L.py + L.dy * t_adv;
-            L.pz = L.pz + L.dz * t_adv;
-            L.dist += t_adv;
-        }
-        /* a wave with a direction component below 2^-100 in an advancing
-         * lane takes the dividing pop test; all others the exact
-         * division-free one */
-        const bool tiny = adv && (fabsf(L.dx) < 0x1p-100f || fabsf(L.dy) < 0x1p-100f || fabsf(L.dz) < 0x1p-100f);
-        if (__any(tiny))
-            pop_walk<kLds, true>(P, s_inner, half, L, adv, cur, n);
-        else
-            pop_walk<kLds, false>(P, s_inner, half, L, adv, cur, n);
-        if (adv) {
-            L.cur = cur;
-            L.node = n;
-        }
     }
     return done;
 }
@@ -763,24 +745,23 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
                                                           uint32_t burst, uint32_t chunk, uint32_t small_rays,
                                                           uint32_t small_blocks, const trace_fuse F)
 {
-    extern __shared__ uint2 s_inner[];
+    extern __shared__ uint2 s_bricks[];
     /* a queue of fewer than small_rays rays is traced by the first
      * small_blocks workgroups (one per CU) alone: with few rays per lane the
      * launch is as long as its slowest rays, which run faster with fewer
      * waves per SIMD */
-    const uint32_t n_rays = *n_rays_ptr;
+    const uint32_t n_rays = __builtin_amdgcn_readfirstlane(*n_rays_ptr);
     const bool small = n_rays < small_rays;
     if (small && blockIdx.x >= small_blocks) return;
     if constexpr (kLds) {
-        for (uint32_t i = threadIdx.x; i < P.n_inner; i += blockDim.x) s_inner[i] = P.inner[i];
         const uint2* gb = (const uint2*)P.bricks;
-        for (uint32_t i = threadIdx.x; i < P.n_leaves; i += blockDim.x) s_inner[P.n_inner + i] = gb[i];
+        for (uint32_t i = threadIdx.x; i < P.n_leaves; i += blockDim.x) s_bricks[i] = gb[i];
         __syncthreads();
     }
     const uint32_t lane = threadIdx.x & 63u;
     /* fused GI: each lane's bounce ray origin and id, behind the nodes; the
      * wave's part of the stash is a uniform base indexed by lane */
-    float4* s_ray = (float4*)(s_inner + (kLds ? ((P.n_inner + P.n_leaves + 1u) & ~1u) : 0u)) +
+    float4* s_ray = (float4*)(s_bricks + (kLds ? ((P.n_leaves + 1u) & ~1u) : 0u)) +
                     __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
     const float half = P.half;
     trace_lane L = {};
@@ -789,7 +770,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
     uint32_t n_hit0 = 0;
     /* pending: the lane holds a ray (world origin in px..pz, direction in
      * dx..dz) that is set up at the next iteration's start */
-    bool active = false, exhausted = false, pending = false;
+    bool active = false, pending = false;
     /* The wave's slice of the queue, rays [q_next, q_end) taken from the
      * cursor and not handed out yet: one atomic takes `chunk` rays for
      * several refills (same-address atomics of all waves serialise). Near
@@ -797,7 +778,6 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
      * atomic) a wave takes only what it hands out, so no wave holds back
      * rays that idle waves could trace. */
     uint32_t q_next = 0, q_end = 0, seen = 0;
-    bool drained = false;
     const uint32_t n_waves = (small && small_blocks < gridDim.x ? small_blocks : gridDim.x) * (TRACE_BLOCK / 64u);
     /* The queue is split into TRACE_SEGS segments with a cursor each (16
      * words apart). A wave starts in segment blockIdx.x mod TRACE_SEGS
@@ -809,7 +789,15 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
     auto seg_start = [n_rays](uint32_t k) { return (uint32_t)((uint64_t)n_rays * k / TRACE_SEGS); };
     seen = seg_start(seg);
     const uint32_t seg_waves = (n_waves + TRACE_SEGS - 1u) / TRACE_SEGS;
-    while (true) {
+    do {
+        /* the queue state is the wave's: kept in scalar registers */
+        q_next = __builtin_amdgcn_readfirstlane(q_next);
+        q_end = __builtin_amdgcn_readfirstlane(q_end);
+        seen = __builtin_amdgcn_readfirstlane(seen);
+        seg = __builtin_amdgcn_readfirstlane(seg);
+        seg_left = __builtin_amdgcn_readfirstlane(seg_left);
+        const bool drained = seg_left == 0u;
+        const bool exhausted = drained && q_next == q_end;
         /* wave-uniform refill once `refill` lanes are idle */
         const unsigned long long idle = __ballot(!active && !pending);
         const uint32_t want = (uint32_t)__popcll(idle);
@@ -833,9 +821,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
                 }
                 if ((uint64_t)base + take >= seg_hi) {
                     /* this segment has run dry: on to the next one */
-                    if (--seg_left == 0u) {
-                        drained = true;
-                    } else {
+                    if (--seg_left != 0u) {
                         seg = seg + 1u == TRACE_SEGS ? 0u : seg + 1u;
                         seen = seg_start(seg);
                     }
@@ -860,17 +846,12 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
                 q_next = nend - nb > used ? nb + used : nend;
                 q_end = nend;
             }
-            exhausted = drained && q_next == q_end;
         }
         if (pending) {
             pending = false;
             /* a shadow ray's step lengths are the sun's, set with its ray */
             active = lane_init_self(P, half, L, kFused && (slot & TRACE_SHADOW));
             if (!kFused && !active) out[slot] = res_miss(0u);
-        }
-        if (!__any(active || pending)) {
-            if (exhausted) break;
-            continue;
         }
         /* phase vote (tuning): a wave runs only DDA bursts in an iteration
          * once at least vote/64 of its active lanes are in a leaf DDA, and
@@ -887,8 +868,8 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
          * 1 bounce hit, 2 shadow ray started, 4 shadow hit; << 3 for the
          * second list */
         uint32_t ev = 0u;
-        if (lane_step<kLds, false, kDda>(P, s_inner, half, maxd, L, res, active, allow_node, allow_dda, false,
-                                         cross, node_iters, burst) &&
+        if (lane_step<kLds, false, kDda>(P, s_bricks, half, maxd, L, res, active, allow_node, allow_dda, cross,
+                                         node_iters, burst) &&
             active) {
             active = false;
             if constexpr (!kFused) {
@@ -936,7 +917,9 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
         if constexpr (!kFused) {
             if (__any(ev != 0u)) n_hit0 += (uint32_t)__popcll(__ballot(ev & 1u));
         }
-    }
+        /* the only exit, at the end: the compiler takes any other one for
+         * divergent and keeps the queue state in vector registers */
+    } while ((__ballot(active || pending) | (seg_left == 0u && q_next == q_end ? 0ull : 1ull)) != 0ull);
     if constexpr (!kFused) {
         if (lane == 0 && hit_counter && n_hit0) atomicAdd(hit_counter, n_hit0);
     }
@@ -1009,14 +992,13 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
                                                              uint32_t* __restrict__ cursor, uint32_t refill,
                                                              uint32_t node_iters, const trace_fuse F)
 {
-    extern __shared__ uint2 s_inner[];
-    const uint32_t lds_nodes = kLds ? ((P.n_inner + P.n_leaves + 1u) & ~1u) : 0u;
-    float4* planes = (float4*)(s_inner + lds_nodes);
+    extern __shared__ uint2 s_bricks[];
+    const uint32_t lds_nodes = kLds ? ((P.n_leaves + 1u) & ~1u) : 0u;
+    float4* planes = (float4*)(s_bricks + lds_nodes);
     rg_ctl* ctl = (rg_ctl*)(planes + RG_PLANES * RG_BLOCK);
     if constexpr (kLds) {
-        for (uint32_t i = threadIdx.x; i < P.n_inner; i += blockDim.x) s_inner[i] = P.inner[i];
         const uint2* gb = (const uint2*)P.bricks;
-        for (uint32_t i = threadIdx.x; i < P.n_leaves; i += blockDim.x) s_inner[P.n_inner + i] = gb[i];
+        for (uint32_t i = threadIdx.x; i < P.n_leaves; i += blockDim.x) s_bricks[i] = gb[i];
     }
     if (threadIdx.x == 0) ctl->exhausted = 0u;
     __syncthreads();
@@ -1060,8 +1042,8 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
             const bool step_node = active && !was_dda && !(L.node & ND_DDA);
             if (!__any(step_dda || step_node)) break;
             svo_res res;
-            if (lane_step<kLds, kSkip>(P, s_inner, half, maxd, L, res, active && (step_dda || step_node), step_node,
-                                       step_dda, true) &&
+            if (lane_step<kLds, kSkip>(P, s_bricks, half, maxd, L, res, active && (step_dda || step_node), step_node,
+                                       step_dda) &&
                 active && (step_dda || step_node)) {
                 active = false;
                 fused_result(P, F, L, res, slot, ox, oy, oz, sid, pending);
@@ -1092,8 +1074,8 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
             const uint32_t flags = (active ? 1u : 0u) | (pending ? 2u : 0u);
             planes[0 * RG_BLOCK + dst] = make_float4(L.px, L.py, L.pz, L.dist);
             planes[1 * RG_BLOCK + dst] = make_float4(L.dx, L.dy, L.dz, __uint_as_float(L.steps));
-            planes[2 * RG_BLOCK + dst] = make_float4(__uint_as_float(L.cur), __uint_as_float(L.node),
-                                                     __uint_as_float(L.leaf), __uint_as_float(L.vox));
+            planes[2 * RG_BLOCK + dst] = make_float4(__uint_as_float(L.node), __uint_as_float(L.leaf),
+                                                     __uint_as_float(L.vox), 0.0f);
             planes[3 * RG_BLOCK + dst] = make_float4(L.tmx, L.tmy, L.tmz, __uint_as_float(slot));
             planes[4 * RG_BLOCK + dst] = make_float4(L.tdx, L.tdy, L.tdz, __uint_as_float(flags));
             planes[5 * RG_BLOCK + dst] = make_float4(ox, oy, oz, __uint_as_float(sid));
@@ -1106,8 +1088,7 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
             const float4 e = planes[4 * RG_BLOCK + me], f = planes[5 * RG_BLOCK + me];
             L.px = a.x; L.py = a.y; L.pz = a.z; L.dist = a.w;
             L.dx = b.x; L.dy = b.y; L.dz = b.z; L.steps = __float_as_uint(b.w);
-            L.cur = __float_as_uint(c.x); L.node = __float_as_uint(c.y);
-            L.leaf = __float_as_uint(c.z); L.vox = __float_as_uint(c.w);
+            L.node = __float_as_uint(c.x); L.leaf = __float_as_uint(c.y); L.vox = __float_as_uint(c.z);
             L.tmx = d.x; L.tmy = d.y; L.tmz = d.z; slot = __float_as_uint(d.w);
             L.tdx = e.x; L.tdy = e.y; L.tdz = e.z;
             const uint32_t flags = __float_as_uint(e.w);
@@ -1115,7 +1096,7 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
             pending = (flags & 2u) != 0u;
             ox = f.x; oy = f.y; oz = f.z; sid = __float_as_uint(f.w);
             /* the leaf's brick mask and an empty bit-word cache */
-            if (active && (L.node & ND_DDA)) L.bm = bricks_at<kLds>(P.bricks, s_inner, P.n_inner, L.leaf);
+            if (active && (L.node & ND_DDA)) L.bm = bricks_at<kLds>(P.bricks, s_bricks, L.leaf);
             L.wi = 0xFFFFFFFFu;
         } else {
             active = false;
@@ -1670,16 +1651,15 @@ __global__ void svo_vis_pack_k(const svo_res* __restrict__ res, uint32_t n, floa
 static trace_params params_of(tgx_context* ctx)
 {
     trace_params P;
-    P.inner = (const uint2*)ctx->svo_inner.ptr;
+    P.grid = (const uint32_t*)ctx->svo_grid.ptr;
     P.bricks = (const unsigned long long*)ctx->svo_bricks.ptr;
     P.leaf_bits = (const uint32_t*)ctx->svo_leaf_bits.ptr;
     P.n_inner = ctx->svo_n_inner;
     P.n_leaves = ctx->svo_info.n_leaves;
-    P.depth = ctx->svo_info.depth;
     P.leaf_level = ctx->svo_info.depth - 5u;
     P.mnx = ctx->svo_info.min[0]; P.mny = ctx->svo_info.min[1]; P.mnz = ctx->svo_info.min[2];
     /* the kernels' former in-kernel expressions, in the same fp32 order */
-    P.half = (float)(1u << P.depth) * 0.5f;
+    P.half = (float)(1u << ctx->svo_info.depth) * 0.5f;
     P.cx = P.mnx + P.half; P.cy = P.mny + P.half; P.cz = P.mnz + P.half;
     return P;
 }
@@ -1710,8 +1690,8 @@ static int launch_trace(tgx_context* ctx, const svo_ray* rays, const uint32_t* n
          * fused GI trace one 16-B ray stash per lane */
         const bool fused = F.contrib != nullptr;
         const uint32_t stash = fused ? 16u * TRACE_BLOCK : 0u;
-        const bool lds = (uint64_t)P.n_inner + P.n_leaves <= TRACE_LDS_NODES_MAX;
-        const uint32_t shmem = (lds ? 8u * ((P.n_inner + P.n_leaves + 1u) & ~1u) : 0u) + stash;
+        const bool lds = P.n_leaves <= TRACE_LDS_LEAVES_MAX;
+        const uint32_t shmem = (lds ? 8u * ((P.n_leaves + 1u) & ~1u) : 0u) + stash;
         /* DDA form: 0 counted, 1 uncounted, 2 uncounted with brick crossing */
         const uint32_t dda = ctx->tuning.trace_dda == 0u ? 0u : (ctx->tuning.trace_cross ? 2u : 1u);
         decltype(&gi_trace_k<true, true, 0u>) kernel;
@@ -1752,8 +1732,8 @@ static int launch_trace_rg(tgx_context* ctx, const svo_ray* rays, const uint32_t
     const dim3 grid(want < (uint32_t)cus ? want : (uint32_t)cus);
     const trace_params P = params_of(ctx);
     const size_t state = sizeof(float4) * RG_PLANES * RG_BLOCK + sizeof(rg_ctl);
-    const size_t nodes = 8u * (size_t)((P.n_inner + P.n_leaves + 1u) & ~1u);
-    const bool lds = (uint64_t)P.n_inner + P.n_leaves <= TRACE_LDS_NODES_MAX && nodes + state <= (size_t)max_lds;
+    const size_t nodes = 8u * (size_t)((P.n_leaves + 1u) & ~1u);
+    const bool lds = P.n_leaves <= TRACE_LDS_LEAVES_MAX && nodes + state <= (size_t)max_lds;
     if (state > (size_t)max_lds)
         return tgx_fail(ctx, TGX_ERR_CAPACITY, "regrouped trace needs %zu B of LDS per workgroup, the device has %d",
                         state, max_lds);

@@ -80,7 +80,7 @@ struct tgx_context {
     tgx_buffer   svo_list_off;   /* n_leaves + 1                            */
     tgx_buffer   svo_list;       /* cluster idx lists                       */
     tgx_buffer   svo_frames;     /* per-cptr cluster transforms (build)     */
-    tgx_buffer   svo_inner;      /* uint2 per inner node (traversal layout) */
+    tgx_buffer   svo_grid;       /* u32 per 32^3 cell of the root (traversal layout) */
     tgx_buffer   svo_bricks;     /* u64 per leaf: 8^3 bricks holding solids */
     uint32_t     svo_n_inner = 0;/* inner nodes = index of the first leaf   */
     tgx_buffer   svo_rays;       /* staging for tgx_svo_trace               */
@@ -102,7 +102,7 @@ struct tgx_context {
     tgx_buffer   gi_sort;        /* sort keys and indices                   */
     uint32_t     gi_spp = 0;     /* spp of the last GI call                 */
     uint32_t     rg_lds_set = 0; /* regrouped trace variants whose LDS limit is raised */
-    tgx_tuning   tuning = {0u, 5u, 2u, 0u, 0u, 0u, 2048u, 1u, 16u, 40u, 3u, 8u, 32u, 8u};
+    tgx_tuning   tuning = {0u, 5u, 2u, 0u, 0u, 0u, 2048u, 1u, 16u, 32u, 2u, 12u, 32u, 8u};
 
     /* Neural irradiance cache (tgx_nrc.hip). */
     bool           nrc_ready = false;

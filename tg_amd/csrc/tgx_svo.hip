@@ -557,14 +557,31 @@ __global__ void svo_list_compact_k(const uint32_t* __restrict__ leaf_first_pair,
     for (uint32_t i = 0; i < leaf_n[l]; i++) list[o + i] = list_tmp[b + i];
 }
 
-/* Compact inner nodes for traversal (8 B): x = first child, y = parent
- * (24 bits, 0xFFFFFF for the root) | child-valid mask << 24. */
-__global__ void svo_inner_k(const svo_gnode* __restrict__ nodes, uint32_t n_inner, uint2* __restrict__ inner)
+/* Leaf grid for traversal, one entry per 32^3 cell of the root (cell x | y
+ * << leaf_level | z << 2 leaf_level): the leaf's index, or for a cell without
+ * a leaf that holds solid voxels SVO_GRID_EMPTY | q, the child slot that the
+ * descent to the cell ends in being 2^q cells wide. 1 MB at depth 11, 8 MB at
+ * 12, 64 MB at 13. */
+__global__ __launch_bounds__(256) void svo_grid_k(const svo_gnode* __restrict__ nodes, uint32_t leaf_level,
+                                                  const unsigned long long* __restrict__ bricks,
+                                                  uint32_t* __restrict__ grid)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_inner) return;
-    const svo_gnode n = nodes[i];
-    inner[i] = make_uint2(n.first_child, (n.parent & 0xFFFFFFu) | ((n.masks & 0xFFu) << 24));
+    if (i >> (3u * leaf_level)) return;
+    const uint32_t m = (1u << leaf_level) - 1u;
+    const uint32_t x = i & m, y = (i >> leaf_level) & m, z = i >> (2u * leaf_level);
+    uint32_t node = 0u;
+    for (uint32_t q = leaf_level; q-- > 0u;) {
+        const uint32_t rc = ((x >> q) & 1u) | (((y >> q) & 1u) << 1) | (((z >> q) & 1u) << 2);
+        const uint32_t valid = nodes[node].masks & 0xFFu;
+        if (!(valid & (1u << rc))) {
+            grid[i] = SVO_GRID_EMPTY | q;
+            return;
+        }
+        node = nodes[node].first_child + (uint32_t)__popc(valid & ((1u << rc) - 1u));
+    }
+    const uint32_t leaf = nodes[node].leaf_idx;
+    grid[i] = bricks[leaf] ? leaf : SVO_GRID_EMPTY;
 }
 
 /* Per leaf, one bit per 8^3 brick (bx + 4 by + 16 bz) that holds a solid
@@ -593,7 +610,7 @@ void tgx_svo_release(tgx_context* ctx)
                           &ctx->svo_list_off, &ctx->svo_list, &ctx->svo_frames, &ctx->svo_rays,
                           &ctx->svo_hits, &ctx->prim_tmp, &ctx->gi_counts, &ctx->gi_surf,
                           &ctx->gi_rays, &ctx->gi_res, &ctx->gi_shadow, &ctx->gi_shadow_res,
-                          &ctx->gi_weight, &ctx->gi_contrib, &ctx->gi_list, &ctx->gi_rays2, &ctx->gi_sort, &ctx->gi_bsurf, &ctx->gi_blist, &ctx->gi_bcount, &ctx->svo_inner,
+                          &ctx->gi_weight, &ctx->gi_contrib, &ctx->gi_list, &ctx->gi_rays2, &ctx->gi_sort, &ctx->gi_bsurf, &ctx->gi_blist, &ctx->gi_bcount, &ctx->svo_grid,
                           &ctx->svo_bricks};
     for (tgx_buffer* b : bufs) tgx_buffer_release(b);
     tgx_buffer* prev[] = {&ctx->svo_prev_keys, &ctx->svo_prev_off, &ctx->svo_prev_cand, &ctx->svo_old_bits,
@@ -933,18 +950,19 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
                            (uint32_t*)ctx->svo_list.ptr);
     TGX_LAUNCH_CHECK(ctx, "svo_list_compact_k");
 
-    /* Traversal layout: compact inner nodes and leaf brick masks. */
+    /* Traversal layout: leaf brick masks and the leaf grid. */
     const uint32_t n_inner = lvl_base[leaf_level];
-    if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_inner, 8ull * n_inner, "svo inner nodes")) ||
+    if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_grid, 4ull << (3u * leaf_level), "svo leaf grid")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_bricks, 8ull * nl, "svo leaf bricks")))
         return rc;
-    hipLaunchKernelGGL(svo_inner_k, dim3(blocks_for(n_inner)), dim3(256), 0, ctx->stream, (const svo_gnode*)nodes,
-                       n_inner, (uint2*)ctx->svo_inner.ptr);
-    TGX_LAUNCH_CHECK(ctx, "svo_inner_k");
     if (n_leaves)
         hipLaunchKernelGGL(svo_bricks_k, dim3(n_leaves), dim3(64), 0, ctx->stream, (const uint32_t*)ctx->svo_leaf_bits.ptr,
                            (unsigned long long*)ctx->svo_bricks.ptr);
     TGX_LAUNCH_CHECK(ctx, "svo_bricks_k");
+    hipLaunchKernelGGL(svo_grid_k, dim3(blocks_for(1ull << (3u * leaf_level))), dim3(256), 0, ctx->stream,
+                       (const svo_gnode*)nodes, leaf_level, (const unsigned long long*)ctx->svo_bricks.ptr,
+                       (uint32_t*)ctx->svo_grid.ptr);
+    TGX_LAUNCH_CHECK(ctx, "svo_grid_k");
     if (ctx->dynamic) {
         /* what the next tgx_svo_update compares against */
         if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_prev_keys, 4ull * nl, "svo previous keys")) ||
@@ -995,7 +1013,7 @@ int tgx_svo_device_bytes(tgx_context* ctx, uint64_t* bytes, uint64_t* solid_voxe
              + (4ull * TGX_SVO_BLOCK_WORDS + 2ull * TGX_SVO_BLOCK_WORDS) * nl /* bits, word prefixes */
              + 4ull * (nl + 1) + 2ull * ctx->svo_n_solid               /* material offsets, pool */
              + 4ull * nl + 4ull * (nl + 1) + 4ull * in.n_list_entries  /* cluster lists          */
-             + 8ull * ctx->svo_n_inner + 8ull * nl;                    /* traversal layout       */
+             + (4ull << (3u * (in.depth - 5u))) + 8ull * nl;           /* traversal layout       */
     if (solid_voxels) *solid_voxels = ctx->svo_n_solid;
     return TGX_OK;
 }
@@ -1272,7 +1290,7 @@ int tgx_svo_load(tgx_context* ctx, const char* path)
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_n, 4ull * nlr, "svo leaf n")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_list_off, 4ull * (nlr + 1), "svo list offsets")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_list, 4ull * (list.empty() ? 1 : list.size()), "svo list")) ||
-        (rc = tgx_buffer_reserve(ctx, &ctx->svo_inner, 8ull * hd.n_inner, "svo inner nodes")) ||
+        (rc = tgx_buffer_reserve(ctx, &ctx->svo_grid, 4ull << (3u * (in.depth - 5u)), "svo leaf grid")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_bricks, 8ull * nlr, "svo leaf bricks")))
         return rc;
     if (fseek(s.f, leaf_data_at, SEEK_SET) != 0) return tgx_fail(ctx, TGX_ERR_IO, "cannot seek in %s", path);
@@ -1286,13 +1304,14 @@ int tgx_svo_load(tgx_context* ctx, const char* path)
     TGX_HIP_CHECK(ctx, hipMemcpy(ctx->svo_list_off.ptr, off.data(), 4ull * (nl + 1u), hipMemcpyHostToDevice));
     if (!list.empty())
         TGX_HIP_CHECK(ctx, hipMemcpy(ctx->svo_list.ptr, list.data(), 4ull * list.size(), hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(svo_inner_k, dim3(blocks_for(hd.n_inner)), dim3(256), 0, ctx->stream,
-                       (const svo_gnode*)ctx->svo_nodes.ptr, hd.n_inner, (uint2*)ctx->svo_inner.ptr);
-    TGX_LAUNCH_CHECK(ctx, "svo_inner_k");
     if (nl)
         hipLaunchKernelGGL(svo_bricks_k, dim3(nl), dim3(64), 0, ctx->stream, (const uint32_t*)ctx->svo_leaf_bits.ptr,
                            (unsigned long long*)ctx->svo_bricks.ptr);
     TGX_LAUNCH_CHECK(ctx, "svo_bricks_k");
+    hipLaunchKernelGGL(svo_grid_k, dim3(blocks_for(1ull << (3u * (in.depth - 5u)))), dim3(256), 0, ctx->stream,
+                       (const svo_gnode*)ctx->svo_nodes.ptr, in.depth - 5u,
+                       (const unsigned long long*)ctx->svo_bricks.ptr, (uint32_t*)ctx->svo_grid.ptr);
+    TGX_LAUNCH_CHECK(ctx, "svo_grid_k");
     TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     ctx->svo_info = in;
     ctx->svo_n_inner = hd.n_inner;

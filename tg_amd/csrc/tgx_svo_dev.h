@@ -11,6 +11,10 @@
 #define SVO_EPSILON 1.192092896e-07f
 #define SVO_NONE    0xFFFFFFFFu
 
+/* Leaf-grid entry of a cell without a leaf holding solid voxels: this flag |
+ * q, where the empty child slot the cell lies in is 2^q cells wide. */
+#define SVO_GRID_EMPTY 0x80000000u
+
 /* Node layout on the device (32 B): canonical order, parent links. */
 struct svo_gnode {
     uint32_t first_child;
