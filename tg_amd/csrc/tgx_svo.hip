@@ -18,11 +18,11 @@
  *                        (level, Morton code), children of a node are then
  *                        contiguous in child-index order; svo_nodes_k links
  *                        each node to its parent (binary search one level up).
- *   4. svo_leaf_k        one workgroup per 32^3 leaf: for each listed
- *                        cluster in order, the trimmed block box is point
- *                        sampled in the reference's exact fp32 order
- *                        (:242-315); solid bits collect in LDS, the first
- *                        cluster to set a voxel writes its material.
+ *   4. svo_leaf_k        one workgroup per 32^3 leaf: the trimmed block box of
+ *      svo_leaf_mats_k   each candidate cluster is point sampled in the
+ *                        reference's exact fp32 order (:242-315); solid bits
+ *                        collect in LDS, then the material of the first
+ *                        candidate that sampled a voxel solid.
  * Traversal and GI live in tgx_gi.hip.
  */
 #include "tgx_svo_dev.h"
@@ -299,201 +299,316 @@ __global__ void svo_node_keys_k(const uint32_t* __restrict__ key, const uint32_t
     if (i < n && flag[i]) node_keys[rank[i]] = key[i];
 }
 
-/* Trilinear interpolation of the block corners (tg_sparse_voxel_octree.c:242-291). */
-__device__ static inline void sample_center(const f3* bc, uint32_t x, uint32_t y, uint32_t z, float& cx, float& cy,
-                                            float& cz)
+/* Leaf sampling. A leaf's candidate clusters are staged LEAF_STAGE at a time:
+ * eight lanes per cluster transform its corners (the cluster's in world space
+ * for the trimmed voxel range, the block's in cluster space for the
+ * interpolation), and its solid bits go to LDS. The waves of the workgroup then
+ * take clusters in turn, a lane per (y, z) row of the range: the interpolation
+ * over z and y is done once per row and only the one over x per voxel, in the
+ * reference's operation order (tg_sparse_voxel_octree.c:242-291), and a row's
+ * samples are the bits of one word of the leaf.
+ *
+ * Bound by the samples' arithmetic: a cluster covers about 14^3 voxels of its
+ * leaf. One voxel per lane with the full interpolation took 80 instructions a
+ * sample and two barriers a cluster; now about 30 and none, so that waves run
+ * different clusters at once and the leaf with the most clusters (164 of 16 on
+ * average) no longer makes the launch. 512 objects, depth 11: bits 0.69 -> 0.16
+ * ms, materials 0.73 -> 0.29 ms. 512 lanes against 256: 0.16 and 0.20 ms. */
+#define LEAF_BLOCK 512u
+#define LEAF_STAGE (LEAF_BLOCK / 8u)
+
+struct leaf_stage {
+    float    c[LEAF_STAGE][24];      /* block corners in cluster space, x y z each */
+    uint32_t lo[LEAF_STAGE];         /* trimmed range: x | y << 8 | z << 16 ... */
+    uint32_t hi[LEAF_STAGE];         /* ... one past it; equal where empty */
+    uint32_t cidx[LEAF_STAGE];
+    uint32_t bits[LEAF_STAGE][16];
+};
+
+/* Stages n clusters from pair_cptr; slices z0 .. z1 of the leaf only. */
+__device__ static inline void leaf_stage_load(leaf_stage& st, const uint32_t* __restrict__ pair_cptr, uint32_t n,
+                                              const svo_frame* __restrict__ frames, const uint32_t* __restrict__ bits,
+                                              float pminx, float pminy, float pminz, uint32_t quirk, uint32_t z0,
+                                              uint32_t z1)
 {
-    const float tz = ((float)z + 0.5f) / 32.0f;
-    const float omtz = 1.0f - tz;
-    const float pz0x = omtz * bc[0].x + tz * bc[4].x, pz0y = omtz * bc[0].y + tz * bc[4].y, pz0z = omtz * bc[0].z + tz * bc[4].z;
-    const float pz1x = omtz * bc[1].x + tz * bc[5].x, pz1y = omtz * bc[1].y + tz * bc[5].y, pz1z = omtz * bc[1].z + tz * bc[5].z;
-    const float pz2x = omtz * bc[2].x + tz * bc[6].x, pz2y = omtz * bc[2].y + tz * bc[6].y, pz2z = omtz * bc[2].z + tz * bc[6].z;
-    const float pz3x = omtz * bc[3].x + tz * bc[7].x, pz3y = omtz * bc[3].y + tz * bc[7].y, pz3z = omtz * bc[3].z + tz * bc[7].z;
-    const float ty = ((float)y + 0.5f) / 32.0f;
-    const float omty = 1.0f - ty;
-    const float py0x = omty * pz0x + ty * pz2x, py0y = omty * pz0y + ty * pz2y, py0z = omty * pz0z + ty * pz2z;
-    const float py1x = omty * pz1x + ty * pz3x, py1y = omty * pz1y + ty * pz3y, py1z = omty * pz1z + ty * pz3z;
-    const float tx = ((float)x + 0.5f) / 32.0f;
-    const float omtx = 1.0f - tx;
-    cx = omtx * py0x + tx * py1x;
-    cy = omtx * py0y + tx * py1y;
-    cz = omtx * py0z + tx * py1z;
+    const uint32_t k = threadIdx.x >> 3, i = threadIdx.x & 7u;
+    const float pmaxx = pminx + 32.0f, pmaxy = pminy + 32.0f, pmaxz = pminz + 32.0f;
+    if (k < n) {
+        const svo_frame& f = frames[pair_cptr[k]];
+        const f3 bc = mulv(f.ws2cs, (i & 1u) ? pmaxx : pminx, (i & 2u) ? pmaxy : pminy, (i & 4u) ? pmaxz : pminz, 1.0f);
+        st.c[k][3u * i] = bc.x; st.c[k][3u * i + 1u] = bc.y; st.c[k][3u * i + 2u] = bc.z;
+        /* the cluster's AABB over its corners (:134-197); the reductions pair
+         * corners as the reference's min / max expressions nest, (0 1) (2 3)
+         * (4 6) (5 7), with corner 2 again in place of 3 under the quirk */
+        const f3 cw = mulv(f.cs2ws, (i & 1u) ? 8.0f : 0.0f, (i & 2u) ? 8.0f : 0.0f, (i & 4u) ? 8.0f : 0.0f, 1.0f);
+        f3 mn = cw, mx = cw;
+        const uint32_t lane = threadIdx.x & 63u, g = lane & ~7u;
+        const uint32_t p1 = i == 4u ? 6u : i == 5u ? 7u : i == 2u ? (quirk ? 2u : 3u) : i == 0u ? 1u : i;
+        const uint32_t p2 = i == 0u ? 2u : i == 4u ? 5u : i, p3 = i == 0u ? 4u : i;
+        const uint32_t part[3] = {g | p1, g | p2, g | p3};
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const f3 on = {__shfl(mn.x, (int)part[r]), __shfl(mn.y, (int)part[r]), __shfl(mn.z, (int)part[r])};
+            const f3 ox = {__shfl(mx.x, (int)part[r]), __shfl(mx.y, (int)part[r]), __shfl(mx.z, (int)part[r])};
+            mn = {fmin2(mn.x, on.x), fmin2(mn.y, on.y), fmin2(mn.z, on.z)};
+            mx = {fmax2(mx.x, ox.x), fmax2(mx.y, ox.y), fmax2(mx.z, ox.z)};
+        }
+        if (i == 0u) {
+            /* trimmed box (:218-233), clamped into [0, 32] */
+            const float tlo[3] = {fmax2(pminx, floorf(mn.x)) - pminx, fmax2(pminy, floorf(mn.y)) - pminy, fmax2(pminz, floorf(mn.z)) - pminz};
+            const float thi[3] = {fmin2(pmaxx, ceilf(mx.x)) - pminx, fmin2(pmaxy, ceilf(mx.y)) - pminy, fmin2(pmaxz, ceilf(mx.z)) - pminz};
+            uint32_t lo[3], hi[3];
+            for (int a = 0; a < 3; a++) {
+                lo[a] = (uint32_t)fmin2(32.0f, fmax2(0.0f, tlo[a]));
+                hi[a] = (uint32_t)fmin2(32.0f, fmax2(0.0f, thi[a]));
+            }
+            lo[2] = lo[2] > z0 ? lo[2] : z0;
+            hi[2] = hi[2] < z1 ? hi[2] : z1;
+            const bool empty = hi[0] <= lo[0] || hi[1] <= lo[1] || hi[2] <= lo[2];
+            st.lo[k] = lo[0] | (lo[1] << 8) | (lo[2] << 16);
+            st.hi[k] = empty ? st.lo[k] : hi[0] | (hi[1] << 8) | (hi[2] << 16);
+            st.cidx[k] = f.cidx;
+        }
+    }
+    for (uint32_t j = threadIdx.x; j < 16u * n; j += LEAF_BLOCK)
+        st.bits[j >> 4][j & 15u] = bits[(size_t)frames[pair_cptr[j >> 4]].cidx * 16u + (j & 15u)];
 }
 
-/* Leaf sampling, in two passes over the same leaves with the same
- * arithmetic. kMats false: the leaf's bits, its cluster list and its solid
- * voxel count. kMats true (after the counts are scanned into mat_off): the
- * materials of its solid voxels only, in bit order, at mat_off[leaf] in the
- * pool, and the per-word prefix counts that index them (wpre[w] = solid
- * voxels in the leaf's words before w). A voxel's material is that of the
- * first cluster in list order that samples it solid. */
-template <bool kMats>
-__global__ __launch_bounds__(256) void svo_leaf_k(const svo_gnode* __restrict__ nodes, uint32_t leaf_base,
-                                                  const uint32_t* __restrict__ pair_cptr,
-                                                  const uint32_t* __restrict__ leaf_first_pair, uint32_t n_pairs,
-                                                  uint32_t n_leaves, const svo_frame* __restrict__ frames,
-                                                  const uint32_t* __restrict__ bits,
-                                                  const uint8_t* __restrict__ materials, float mnx, float mny,
-                                                  float mnz, uint32_t quirk, uint32_t* __restrict__ leaf_bits,
-                                                  uint32_t* __restrict__ leaf_solid, const uint32_t* __restrict__ mat_off,
-                                                  uint16_t* __restrict__ wpre, uint16_t* __restrict__ pool,
-                                                  uint32_t* __restrict__ leaf_n,
-                                                  uint32_t* __restrict__ list_tmp, svo_gnode* __restrict__ nodes_rw,
-                                                  const uint32_t* __restrict__ reuse, const uint32_t* __restrict__ old_bits,
-                                                  const uint32_t* __restrict__ old_off, const uint16_t* __restrict__ old_wpre,
-                                                  const uint16_t* __restrict__ old_pool, const uint32_t* __restrict__ old_n,
-                                                  const uint32_t* __restrict__ old_list_off,
-                                                  const uint32_t* __restrict__ old_list)
+/* Calls f(row word 32 z + y of the leaf, voxel x, cluster voxel v) for every
+ * sample of staged cluster k that falls on a solid voxel, a lane per row;
+ * row_done(row word) after each row. Called by whole waves. */
+template <typename F, typename R>
+__device__ static inline void leaf_rows(const leaf_stage& st, uint32_t k, F&& f, R&& row_done)
 {
-    __shared__ uint32_t lbits[TGX_SVO_BLOCK_WORDS];
-    __shared__ uint32_t fbits[kMats ? TGX_SVO_BLOCK_WORDS : 1];
-    __shared__ uint16_t lpre[kMats ? TGX_SVO_BLOCK_WORDS : 1];
-    __shared__ uint32_t wsum[4];
-    __shared__ int any_flag;
-    __shared__ uint32_t n_contrib, last_cidx;
-    const uint32_t leaf = blockIdx.x;
-    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(st.lo[k]), hi = __builtin_amdgcn_readfirstlane(st.hi[k]);
+    if (lo == hi) return;
+    const uint32_t x0 = lo & 255u, y0 = (lo >> 8) & 255u, z0 = lo >> 16;
+    const uint32_t x1 = hi & 255u, ny = ((hi >> 8) & 255u) - y0, n_rows = ny * ((hi >> 16) - z0);
+    const uint32_t inv = 65536u / ny + 1u;   /* r / ny for r < 1024, ny <= 32 */
+    const float* c = st.c[k];
+    for (uint32_t r = lane; r < n_rows; r += 64u) {
+        const uint32_t q = (r * inv) >> 16;
+        const uint32_t y = y0 + r - q * ny, z = z0 + q;
+        const float tz = ((float)z + 0.5f) / 32.0f, omtz = 1.0f - tz;
+        const float ty = ((float)y + 0.5f) / 32.0f, omty = 1.0f - ty;
+        float p0[3], p1[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const float pz0 = omtz * c[a] + tz * c[12 + a], pz1 = omtz * c[3 + a] + tz * c[15 + a];
+            const float pz2 = omtz * c[6 + a] + tz * c[18 + a], pz3 = omtz * c[9 + a] + tz * c[21 + a];
+            p0[a] = omty * pz0 + ty * pz2;
+            p1[a] = omty * pz1 + ty * pz3;
+        }
+        for (uint32_t x = x0; x < x1; x++) {
+            const float tx = ((float)x + 0.5f) / 32.0f, omtx = 1.0f - tx;
+            /* 0 <= centre < 8 on each axis as its floor in 0 .. 7 */
+            const uint32_t ix = (uint32_t)(int)floorf(omtx * p0[0] + tx * p1[0]);
+            const uint32_t iy = (uint32_t)(int)floorf(omtx * p0[1] + tx * p1[1]);
+            const uint32_t iz = (uint32_t)(int)floorf(omtx * p0[2] + tx * p1[2]);
+            if ((ix | iy | iz) < 8u) {
+                const uint32_t v = 64u * iz + 8u * iy + ix;
+                if ((st.bits[k][v >> 5] >> (v & 31u)) & 1u) f(x, v, 32u * z + y);
+            }
+        }
+        row_done(32u * z + y);
+    }
+}
+
+/* First pass, a workgroup per leaf: its bits, the per-word prefix counts that
+ * index its materials (wpre[w] = solid voxels in the leaf's words before w),
+ * its solid voxel count and its list: the clusters with a sample on a solid
+ * voxel, in candidate order. */
+__global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __restrict__ nodes, uint32_t leaf_base,
+                                                         const uint32_t* __restrict__ pair_cptr,
+                                                         const uint32_t* __restrict__ leaf_first_pair, uint32_t n_pairs,
+                                                         uint32_t n_leaves, const svo_frame* __restrict__ frames,
+                                                         const uint32_t* __restrict__ bits, float mnx, float mny,
+                                                         float mnz, uint32_t quirk, uint32_t* __restrict__ leaf_bits,
+                                                         uint32_t* __restrict__ leaf_solid, uint16_t* __restrict__ wpre,
+                                                         uint32_t* __restrict__ leaf_n, uint32_t* __restrict__ list_tmp,
+                                                         svo_gnode* __restrict__ nodes_rw,
+                                                         const uint32_t* __restrict__ reuse,
+                                                         const uint32_t* __restrict__ old_bits,
+                                                         const uint32_t* __restrict__ old_off,
+                                                         const uint16_t* __restrict__ old_wpre,
+                                                         const uint32_t* __restrict__ old_n,
+                                                         const uint32_t* __restrict__ old_list_off,
+                                                         const uint32_t* __restrict__ old_list)
+{
+    const uint32_t leaf = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     if (reuse && reuse[leaf] != SVO_NONE) {
         /* an update: same candidate clusters in the same order, none of
          * them new, so the previous build's leaf is this leaf */
         const uint32_t j = reuse[leaf];
-        if constexpr (!kMats) {
-            const uint4* sb = (const uint4*)(old_bits + (size_t)j * TGX_SVO_BLOCK_WORDS);
-            uint4* db = (uint4*)(leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS);
-            for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS / 4u; w += blockDim.x) db[w] = sb[w];
-            const uint32_t n = old_n[j], b = leaf_first_pair[leaf], o = old_list_off[j];
-            for (uint32_t i = tid; i < n; i += blockDim.x) list_tmp[b + i] = old_list[o + i];
-            if (tid == 0) {
-                leaf_n[leaf] = n;
-                nodes_rw[leaf_base + leaf].leaf_n = n;
-                leaf_solid[leaf] = old_off[j + 1] - old_off[j];
-            }
-        } else {
-            const uint2* sw = (const uint2*)(old_wpre + (size_t)j * TGX_SVO_BLOCK_WORDS);
-            uint2* dw = (uint2*)(wpre + (size_t)leaf * TGX_SVO_BLOCK_WORDS);
-            for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS / 4u; w += blockDim.x) dw[w] = sw[w];
-            const uint32_t o = old_off[j], n = old_off[j + 1] - o, d = mat_off[leaf];
-            for (uint32_t i = tid; i < n; i += blockDim.x) pool[d + i] = old_pool[o + i];
+        const uint4* sb = (const uint4*)(old_bits + (size_t)j * TGX_SVO_BLOCK_WORDS);
+        uint4* db = (uint4*)(leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS);
+        const uint2* sw = (const uint2*)(old_wpre + (size_t)j * TGX_SVO_BLOCK_WORDS);
+        uint2* dw = (uint2*)(wpre + (size_t)leaf * TGX_SVO_BLOCK_WORDS);
+        for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS / 4u; w += LEAF_BLOCK) {
+            db[w] = sb[w];
+            dw[w] = sw[w];
+        }
+        const uint32_t n = old_n[j], b = leaf_first_pair[leaf], o = old_list_off[j];
+        for (uint32_t i = tid; i < n; i += LEAF_BLOCK) list_tmp[b + i] = old_list[o + i];
+        if (tid == 0) {
+            leaf_n[leaf] = n;
+            nodes_rw[leaf_base + leaf].leaf_n = n;
+            leaf_solid[leaf] = old_off[j + 1] - old_off[j];
         }
         return;
     }
+    __shared__ leaf_stage st;
+    __shared__ uint32_t lbits[TGX_SVO_BLOCK_WORDS];
+    __shared__ uint32_t s_any[LEAF_STAGE];
+    __shared__ uint32_t wsum[LEAF_BLOCK / 64u];
     const svo_gnode nd = nodes[leaf_base + leaf];
     const float pminx = mnx + (float)nd.cx * 32.0f, pminy = mny + (float)nd.cy * 32.0f, pminz = mnz + (float)nd.cz * 32.0f;
-    const float pmaxx = pminx + 32.0f, pmaxy = pminy + 32.0f, pmaxz = pminz + 32.0f;
-    for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS; w += blockDim.x) lbits[w] = 0u;
-    if (tid == 0) { n_contrib = 0u; last_cidx = SVO_NONE; }
-    uint16_t* mats = nullptr;
-    if constexpr (kMats) {
-        /* the leaf's final bits (first pass) and their per-word prefix */
-        const uint32_t* fb = leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS;
-        uint32_t c[4], tot = 0;
-        for (uint32_t i = 0; i < 4u; i++) {
-            const uint32_t w = 4u * tid + i;
-            fbits[w] = fb[w];
-            c[i] = (uint32_t)__popc(fbits[w]);
-            tot += c[i];
-        }
-        /* exclusive scan of the 256 threads' totals: wave scan, then waves */
-        const uint32_t lane = tid & 63u, wv = tid >> 6;
-        uint32_t incl = tot;
-        for (uint32_t d = 1; d < 64u; d <<= 1) {
-            const uint32_t u = __shfl_up(incl, d);
-            if (lane >= d) incl += u;
-        }
-        if (lane == 63u) wsum[wv] = incl;
+    for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS; w += LEAF_BLOCK) lbits[w] = 0u;
+    const uint32_t b = leaf_first_pair[leaf];
+    const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
+    /* wave 0: list entries so far, and the last flagged cluster */
+    uint32_t n_contrib = 0u, last_cidx = SVO_NONE;
+    for (uint32_t s0 = b; s0 < e; s0 += LEAF_STAGE) {
+        const uint32_t n = e - s0 < LEAF_STAGE ? e - s0 : LEAF_STAGE;
+        leaf_stage_load(st, pair_cptr + s0, n, frames, bits, pminx, pminy, pminz, quirk, 0u, 32u);
         __syncthreads();
-        uint32_t run = incl - tot;
-        for (uint32_t k = 0; k < wv; k++) run += wsum[k];
-        for (uint32_t i = 0; i < 4u; i++) {
-            lpre[4u * tid + i] = (uint16_t)run;
-            wpre[(size_t)leaf * TGX_SVO_BLOCK_WORDS + 4u * tid + i] = (uint16_t)run;
-            run += c[i];
+        for (uint32_t k = wave; k < n; k += LEAF_BLOCK / 64u) {
+            uint32_t mask = 0u, any = 0u;
+            leaf_rows(st, k, [&](uint32_t x, uint32_t, uint32_t) { mask |= 1u << x; },
+                      [&](uint32_t w) {
+                          if (mask) atomicOr(&lbits[w], mask);
+                          any |= mask;
+                          mask = 0u;
+                      });
+            const bool some = __any(any != 0u);
+            if (lane == 0u) s_any[k] = some ? 1u : 0u;
         }
-        mats = pool + mat_off[leaf];
+        __syncthreads();
+        if (wave == 0u) {
+            /* the flagged clusters in order; one equal to the flagged
+             * cluster before it is listed once */
+            const bool flag = lane < n && s_any[lane] != 0u;
+            const uint32_t c = lane < n ? st.cidx[lane] : SVO_NONE;
+            const unsigned long long fm = __ballot(flag);
+            const unsigned long long below = fm & ((1ull << lane) - 1ull);
+            const uint32_t prev = __shfl(c, below ? 63 - __clzll((long long)below) : 0);
+            const bool keep = flag && c != (below ? prev : last_cidx);
+            const unsigned long long km = __ballot(keep);
+            if (keep) list_tmp[b + n_contrib + (uint32_t)__popcll(km & ((1ull << lane) - 1ull))] = c;
+            n_contrib += (uint32_t)__popcll(km);
+            if (fm) last_cidx = __shfl(c, 63 - __clzll((long long)fm));
+        }
+        /* st is rewritten by the next stage */
+        __syncthreads();
+    }
+    __syncthreads();
+    /* bits, prefix counts and total: two words per thread */
+    const uint32_t w0 = lbits[2u * tid], w1 = lbits[2u * tid + 1u];
+    const uint32_t c0 = (uint32_t)__popc(w0), c1 = (uint32_t)__popc(w1);
+    uint32_t incl = c0 + c1;
+#pragma unroll
+    for (uint32_t d = 1; d < 64u; d <<= 1) {
+        const uint32_t u = __shfl_up(incl, d);
+        if (lane >= d) incl += u;
+    }
+    if (lane == 63u) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t run = incl - c0 - c1, total = 0u;
+    for (uint32_t k = 0; k < LEAF_BLOCK / 64u; k++) {
+        run += k < wave ? wsum[k] : 0u;
+        total += wsum[k];
+    }
+    ((uint2*)(leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS))[tid] = make_uint2(w0, w1);
+    ((uint32_t*)(wpre + (size_t)leaf * TGX_SVO_BLOCK_WORDS))[tid] = run | ((run + c0) << 16);
+    if (tid == 0) {
+        leaf_n[leaf] = n_contrib;
+        nodes_rw[leaf_base + leaf].leaf_n = n_contrib;
+        leaf_solid[leaf] = total;
+    }
+}
+
+/* Second pass (after the counts are scanned into mat_off), LEAF_PARTS
+ * workgroups per leaf, eight z slices each: the materials of the leaf's solid
+ * voxels, in bit order, at mat_off[leaf] in the pool. A voxel's material is
+ * that of the first candidate that samples it solid: the samples of a
+ * candidate k on cluster voxel v lower the voxel's key to k << 9 | v, so waves
+ * run different candidates in any order (a wave's lanes are on rows of the
+ * same x: each row's keys are rotated by exclusive or so that they fall on
+ * different LDS banks: 0.38 -> 0.29 ms). One workgroup a leaf holds 128 KB of
+ * keys and takes 0.54 ms, 2, 4 and 8 take 0.35, 0.29 and 0.45. Keys hold 2^LEAF_SPAN candidates;
+ * more are taken in turns, each turn filling voxels that no earlier one has. */
+#define LEAF_PARTS 4u
+#define LEAF_SLICES (32u / LEAF_PARTS)
+#define LEAF_SPAN 22u
+__global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_mats_k(const svo_gnode* __restrict__ nodes, uint32_t leaf_base,
+                                                              const uint32_t* __restrict__ pair_cptr,
+                                                              const uint32_t* __restrict__ leaf_first_pair,
+                                                              uint32_t n_pairs, uint32_t n_leaves,
+                                                              const svo_frame* __restrict__ frames,
+                                                              const uint32_t* __restrict__ bits,
+                                                              const uint8_t* __restrict__ materials, float mnx,
+                                                              float mny, float mnz, uint32_t quirk,
+                                                              const uint32_t* __restrict__ leaf_bits,
+                                                              const uint16_t* __restrict__ wpre,
+                                                              const uint32_t* __restrict__ mat_off,
+                                                              uint16_t* __restrict__ pool,
+                                                              const uint32_t* __restrict__ reuse,
+                                                              const uint32_t* __restrict__ old_off,
+                                                              const uint16_t* __restrict__ old_pool)
+{
+    const uint32_t leaf = blockIdx.x / LEAF_PARTS, part = blockIdx.x % LEAF_PARTS;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    if (reuse && reuse[leaf] != SVO_NONE) {
+        const uint32_t j = reuse[leaf];
+        const uint32_t o = old_off[j], n = old_off[j + 1] - o, d = mat_off[leaf];
+        for (uint32_t i = part * LEAF_BLOCK + tid; i < n; i += LEAF_PARTS * LEAF_BLOCK) pool[d + i] = old_pool[o + i];
+        return;
+    }
+    __shared__ leaf_stage st;
+    __shared__ uint32_t key[LEAF_SLICES * 1024u];
+    __shared__ uint32_t s_bits[LEAF_SLICES * 32u], s_done[LEAF_SLICES * 32u];
+    const svo_gnode nd = nodes[leaf_base + leaf];
+    const float pminx = mnx + (float)nd.cx * 32.0f, pminy = mny + (float)nd.cy * 32.0f, pminz = mnz + (float)nd.cz * 32.0f;
+    const uint32_t z0 = part * LEAF_SLICES, row0 = 32u * z0;
+    const size_t word0 = (size_t)leaf * TGX_SVO_BLOCK_WORDS + row0;
+    for (uint32_t w = tid; w < LEAF_SLICES * 32u; w += LEAF_BLOCK) {
+        s_bits[w] = leaf_bits[word0 + w];
+        s_done[w] = 0u;
     }
     const uint32_t b = leaf_first_pair[leaf];
     const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
-    __syncthreads();
-    for (uint32_t k = b; k < e; k++) {
-        const svo_frame& f = frames[pair_cptr[k]];
-        /* cluster corners in world space and their AABB (:134-197) */
-        f3 cw[8];
-        for (int i = 0; i < 8; i++)
-            cw[i] = mulv(f.cs2ws, (i & 1) ? 8.0f : 0.0f, (i & 2) ? 8.0f : 0.0f, (i & 4) ? 8.0f : 0.0f, 1.0f);
-        const int c3 = quirk ? 2 : 3;
-        const float minx = fmin2(fmin2(fmin2(cw[0].x, cw[1].x), fmin2(cw[2].x, cw[c3].x)), fmin2(fmin2(cw[4].x, cw[6].x), fmin2(cw[5].x, cw[7].x)));
-        const float miny = fmin2(fmin2(fmin2(cw[0].y, cw[1].y), fmin2(cw[2].y, cw[c3].y)), fmin2(fmin2(cw[4].y, cw[6].y), fmin2(cw[5].y, cw[7].y)));
-        const float minz = fmin2(fmin2(fmin2(cw[0].z, cw[1].z), fmin2(cw[2].z, cw[c3].z)), fmin2(fmin2(cw[4].z, cw[6].z), fmin2(cw[5].z, cw[7].z)));
-        const float maxx = fmax2(fmax2(fmax2(cw[0].x, cw[1].x), fmax2(cw[2].x, cw[c3].x)), fmax2(fmax2(cw[4].x, cw[6].x), fmax2(cw[5].x, cw[7].x)));
-        const float maxy = fmax2(fmax2(fmax2(cw[0].y, cw[1].y), fmax2(cw[2].y, cw[c3].y)), fmax2(fmax2(cw[4].y, cw[6].y), fmax2(cw[5].y, cw[7].y)));
-        const float maxz = fmax2(fmax2(fmax2(cw[0].z, cw[1].z), fmax2(cw[2].z, cw[c3].z)), fmax2(fmax2(cw[4].z, cw[6].z), fmax2(cw[5].z, cw[7].z)));
-        /* block corners in cluster space (:199-211) */
-        f3 bc[8];
-        for (int i = 0; i < 8; i++)
-            bc[i] = mulv(f.ws2cs, (i & 1) ? pmaxx : pminx, (i & 2) ? pmaxy : pminy, (i & 4) ? pmaxz : pminz, 1.0f);
-        /* trimmed box (:218-233), clamped into [0, 32] */
-        const float tlo[3] = {fmax2(pminx, floorf(minx)) - pminx, fmax2(pminy, floorf(miny)) - pminy, fmax2(pminz, floorf(minz)) - pminz};
-        const float thi[3] = {fmin2(pmaxx, ceilf(maxx)) - pminx, fmin2(pmaxy, ceilf(maxy)) - pminy, fmin2(pmaxz, ceilf(maxz)) - pminz};
-        uint32_t lo[3], hi[3];
-        for (int a = 0; a < 3; a++) {
-            lo[a] = (uint32_t)fmin2(32.0f, fmax2(0.0f, tlo[a]));
-            hi[a] = (uint32_t)fmin2(32.0f, fmax2(0.0f, thi[a]));
-        }
-        const uint32_t nx = hi[0] > lo[0] ? hi[0] - lo[0] : 0u;
-        const uint32_t ny = hi[1] > lo[1] ? hi[1] - lo[1] : 0u;
-        const uint32_t nz = hi[2] > lo[2] ? hi[2] - lo[2] : 0u;
-        const uint32_t nv = nx * ny * nz;
-        const uint64_t coff = (uint64_t)f.cidx * 512u;
-        if (tid == 0) any_flag = 0;
-        __syncthreads();
-        bool any = false;
-        for (uint32_t j = tid; j < nv; j += blockDim.x) {
-            const uint32_t x = lo[0] + j % nx, y = lo[1] + (j / nx) % ny, z = lo[2] + j / (nx * ny);
-            float cx, cy, cz;
-            sample_center(bc, x, y, z, cx, cy, cz);
-            if (cx < 0.0f || cx >= 8.0f || cy < 0.0f || cy >= 8.0f || cz < 0.0f || cz >= 8.0f) continue;
-            const uint32_t v = 64u * (uint32_t)cz + 8u * (uint32_t)cy + (uint32_t)cx;
-            const uint64_t cv = coff + v;
-            if (!(bits[cv >> 5] & (1u << (uint32_t)(cv & 31u)))) continue;
-            any = true;
-            const uint32_t bv = 1024u * z + 32u * y + x;
-            const uint32_t m = 1u << (bv & 31u);
-            /* Within one cluster each block voxel is visited once; earlier
-             * clusters' bits are complete (barrier), so the first cluster in
-             * list order writes the material. */
-            if (!(lbits[bv >> 5] & m)) {
-                atomicOr(&lbits[bv >> 5], m);
-                if constexpr (kMats)
-                    mats[lpre[bv >> 5] + (uint32_t)__popc(fbits[bv >> 5] & (m - 1u))] =
-                        (uint16_t)(f.lut | (materials ? (uint32_t)materials[cv] : 0u));
-            }
-        }
-        if constexpr (!kMats) {
-            if (any) any_flag = 1;
+    uint16_t* mats = pool + mat_off[leaf];
+    for (uint32_t t0 = b; t0 < e; t0 += 1u << LEAF_SPAN) {
+        const uint32_t t1 = e - t0 < (1u << LEAF_SPAN) ? e : t0 + (1u << LEAF_SPAN);
+        for (uint32_t v = tid; v < LEAF_SLICES * 1024u; v += LEAF_BLOCK) key[v] = SVO_NONE;
+        for (uint32_t s0 = t0; s0 < t1; s0 += LEAF_STAGE) {
+            const uint32_t n = t1 - s0 < LEAF_STAGE ? t1 - s0 : LEAF_STAGE;
+            leaf_stage_load(st, pair_cptr + s0, n, frames, bits, pminx, pminy, pminz, quirk, z0, z0 + LEAF_SLICES);
             __syncthreads();
-            if (tid == 0 && any_flag && last_cidx != f.cidx) {
-                list_tmp[b + n_contrib] = f.cidx;
-                n_contrib++;
-                last_cidx = f.cidx;
+            for (uint32_t k = wave; k < n; k += LEAF_BLOCK / 64u)
+                leaf_rows(st, k,
+                          [&](uint32_t x, uint32_t v, uint32_t w) {
+                              atomicMin(&key[32u * (w - row0) + (x ^ (w & 31u))], ((s0 - t0 + k) << 9) | v);
+                          },
+                          [](uint32_t) {});
+            /* st is rewritten by the next stage */
+            __syncthreads();
+        }
+        /* a half wave per row */
+        for (uint32_t i = tid; i < LEAF_SLICES * 1024u; i += LEAF_BLOCK) {
+            const uint32_t w = i >> 5, m = 1u << (i & 31u), q = key[i ^ (w & 31u)];
+            const bool mine = q != SVO_NONE && !(s_done[w] & m);
+            if (mine) {
+                const svo_frame& f = frames[pair_cptr[t0 + (q >> 9)]];
+                mats[(uint32_t)wpre[word0 + w] + (uint32_t)__popc(s_bits[w] & (m - 1u))] =
+                    (uint16_t)(f.lut | (materials ? (uint32_t)materials[(size_t)f.cidx * TGX_VOXELS_PER_CLUSTER + (q & 511u)] : 0u));
             }
+            /* rows are 32 consecutive lanes: the half wave's ballot */
+            const unsigned long long got = __ballot(mine);
+            if ((i & 31u) == 0u) s_done[w] |= (uint32_t)(got >> (tid & 32u));
         }
         __syncthreads();
-    }
-    if constexpr (!kMats) {
-        uint32_t* out = leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS;
-        uint32_t cnt = 0;
-        for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS; w += blockDim.x) {
-            out[w] = lbits[w];
-            cnt += (uint32_t)__popc(lbits[w]);
-        }
-        for (uint32_t d = 32; d > 0; d >>= 1) cnt += __shfl_xor(cnt, d);
-        if ((tid & 63u) == 0u) wsum[tid >> 6] = cnt;
-        __syncthreads();
-        if (tid == 0) {
-            leaf_n[leaf] = n_contrib;
-            nodes_rw[leaf_base + leaf].leaf_n = n_contrib;
-            leaf_solid[leaf] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-        }
     }
 }
 
@@ -902,16 +1017,14 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
     const uint32_t* rz = update ? reuse.as<uint32_t>() : nullptr;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_k");
-        hipLaunchKernelGGL(svo_leaf_k<false>, dim3(n_leaves), dim3(256), 0, ctx->stream, nodes, lvl_base[leaf_level],
+        hipLaunchKernelGGL(svo_leaf_k, dim3(n_leaves), dim3(LEAF_BLOCK), 0, ctx->stream, nodes, lvl_base[leaf_level],
                            lvl_scptr[leaf_level].as<uint32_t>(), lvl_first[leaf_level].as<uint32_t>(), n_leaf_pairs,
-                           n_leaves, frames, (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx),
-                           mn[0], mn[1], mn[2], quirk, (uint32_t*)ctx->svo_leaf_bits.ptr, solid.as<uint32_t>(),
-                           (const uint32_t*)nullptr, (uint16_t*)nullptr, (uint16_t*)nullptr,
+                           n_leaves, frames, (const uint32_t*)ctx->bits.ptr, mn[0], mn[1], mn[2], quirk,
+                           (uint32_t*)ctx->svo_leaf_bits.ptr, solid.as<uint32_t>(), (uint16_t*)ctx->svo_leaf_wpre.ptr,
                            (uint32_t*)ctx->svo_leaf_n.ptr, list_tmp.as<uint32_t>(), nodes, rz,
                            (const uint32_t*)ctx->svo_old_bits.ptr, (const uint32_t*)ctx->svo_old_moff.ptr,
-                           (const uint16_t*)ctx->svo_old_wpre.ptr, (const uint16_t*)ctx->svo_old_mats.ptr,
-                           (const uint32_t*)ctx->svo_old_n.ptr, (const uint32_t*)ctx->svo_old_list_off.ptr,
-                           (const uint32_t*)ctx->svo_old_list.ptr);
+                           (const uint16_t*)ctx->svo_old_wpre.ptr, (const uint32_t*)ctx->svo_old_n.ptr,
+                           (const uint32_t*)ctx->svo_old_list_off.ptr, (const uint32_t*)ctx->svo_old_list.ptr);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_k");
     if ((rc = tgx_prim_exclusive_scan_u32(ctx, solid.as<uint32_t>(), (uint32_t*)ctx->svo_leaf_moff.ptr, n_leaves))) return rc;
@@ -924,18 +1037,15 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
     ctx->svo_n_solid = n_solid;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_mats_k");
-        hipLaunchKernelGGL(svo_leaf_k<true>, dim3(n_leaves), dim3(256), 0, ctx->stream, nodes, lvl_base[leaf_level],
-                           lvl_scptr[leaf_level].as<uint32_t>(), lvl_first[leaf_level].as<uint32_t>(), n_leaf_pairs,
-                           n_leaves, frames, (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx),
-                           mn[0], mn[1], mn[2], quirk, (uint32_t*)ctx->svo_leaf_bits.ptr, (uint32_t*)nullptr,
-                           (const uint32_t*)ctx->svo_leaf_moff.ptr, (uint16_t*)ctx->svo_leaf_wpre.ptr,
-                           (uint16_t*)ctx->svo_leaf_mats.ptr, (uint32_t*)nullptr, (uint32_t*)nullptr, nodes, rz,
-                           (const uint32_t*)ctx->svo_old_bits.ptr, (const uint32_t*)ctx->svo_old_moff.ptr,
-                           (const uint16_t*)ctx->svo_old_wpre.ptr, (const uint16_t*)ctx->svo_old_mats.ptr,
-                           (const uint32_t*)ctx->svo_old_n.ptr, (const uint32_t*)ctx->svo_old_list_off.ptr,
-                           (const uint32_t*)ctx->svo_old_list.ptr);
+        hipLaunchKernelGGL(svo_leaf_mats_k, dim3(n_leaves * LEAF_PARTS), dim3(LEAF_BLOCK), 0, ctx->stream, nodes,
+                           lvl_base[leaf_level], lvl_scptr[leaf_level].as<uint32_t>(),
+                           lvl_first[leaf_level].as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
+                           (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx), mn[0], mn[1], mn[2], quirk,
+                           (const uint32_t*)ctx->svo_leaf_bits.ptr, (const uint16_t*)ctx->svo_leaf_wpre.ptr,
+                           (const uint32_t*)ctx->svo_leaf_moff.ptr, (uint16_t*)ctx->svo_leaf_mats.ptr, rz,
+                           (const uint32_t*)ctx->svo_old_moff.ptr, (const uint16_t*)ctx->svo_old_mats.ptr);
     }
-    TGX_LAUNCH_CHECK(ctx, "svo_leaf_k");
+    TGX_LAUNCH_CHECK(ctx, "svo_leaf_mats_k");
     if ((rc = tgx_prim_exclusive_scan_u32(ctx, (const uint32_t*)ctx->svo_leaf_n.ptr, (uint32_t*)ctx->svo_list_off.ptr, n_leaves))) return rc;
     uint32_t n_list = 0;
     if ((rc = scan_total(ctx, (const uint32_t*)ctx->svo_leaf_n.ptr, (const uint32_t*)ctx->svo_list_off.ptr, n_leaves, &n_list))) return rc;
