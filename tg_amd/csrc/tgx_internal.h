@@ -150,6 +150,7 @@ struct tgx_context {
     tgx_buffer          svo_arena;
     size_t              svo_arena_used = 0, svo_arena_want = 0, svo_arena_spill_bytes = 0;
     std::vector<void*>  svo_arena_spill;
+    uint64_t            svo_pairs_need = 0; /* most (node, cluster) pairs on a level of the last build */
 
     /* Profiling. */
     bool                           profiling = false;
@@ -161,6 +162,7 @@ int  tgx_fail(tgx_context* ctx, int code, const char* fmt, ...);
 int  tgx_prim_exclusive_scan_u32(tgx_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n);
 int  tgx_prim_sort_pairs_u32(tgx_context* ctx, const uint32_t* keys_in, uint32_t* keys_out,
                              const uint32_t* vals_in, uint32_t* vals_out, uint32_t n, unsigned end_bit);
+int  tgx_prim_sort_keys_u64(tgx_context* ctx, const uint64_t* keys_in, uint64_t* keys_out, uint32_t n, unsigned end_bit);
 void tgx_svo_release(tgx_context* ctx);
 void tgx_nrc_release(tgx_context* ctx);
 /* Visibility camera records for captured frames: tgx_vis_cams_upload

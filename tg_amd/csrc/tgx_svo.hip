@@ -6,18 +6,17 @@
  *   1. svo_frames_k      per cluster pointer: emptiness flag and the three
  *                        cluster transforms of the reference (world->cluster
  *                        :23-60, cluster->world :62-100 and its inverse).
- *   2. per level         (node, cluster pointer) pairs; svo_children_k runs
+ *   2. per level         (node, cluster pointer) pairs; svo_expand_k runs
  *                        tg_intersect_aabb_obb_ignore_contact for the 8
- *                        children of each pair, a scan sizes the next level
- *                        and svo_emit_k writes it. Pairs stay ordered by the
- *                        parent pair, so every node's clusters stay in
- *                        ascending pointer order (the reference's list order)
- *                        without sorting between levels.
- *   3. per level         stable radix sort of the pairs by Morton code; each
- *                        distinct code is a node. Nodes are numbered by
- *                        (level, Morton code), children of a node are then
- *                        contiguous in child-index order; svo_nodes_k links
- *                        each node to its parent (binary search one level up).
+ *                        children of each pair, appends the survivors to the
+ *                        next level's pairs and sets their cells in its bitmap.
+ *   3. svo_nodes_k       the bitmaps of all levels, one after the other, are the
+ *                        nodes in (level, Morton code) order: a scan of their
+ *                        popcounts numbers them, a node's children are one byte
+ *                        of the next level, contiguous in child-index order.
+ *      svo_pair_*_k      the leaf level's pairs sorted by (leaf, cluster
+ *                        pointer): each leaf's clusters in ascending pointer
+ *                        order (the reference's list order).
  *   4. svo_leaf_k        one workgroup per 32^3 leaf: the trimmed block box of
  *      svo_leaf_mats_k   each candidate cluster is point sampled in the
  *                        reference's exact fp32 order (:242-315); solid bits
@@ -25,7 +24,7 @@
  *                        candidate that sampled a voxel solid.
  * Traversal and GI live in tgx_gi.hip.
  */
-#include "tgx_svo_dev.h"
+#include "tgx_gi_dev.h"
 #include "tgx_m4.h"
 
 #include <algorithm>
@@ -137,12 +136,6 @@ __device__ static bool obb_overlaps_cluster(const f3* c)
 /* Build kernels                                                            */
 /* ------------------------------------------------------------------------ */
 
-__global__ void svo_fill_k(uint32_t* p, uint64_t n, uint32_t v)
-{
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 __global__ __launch_bounds__(256) void svo_frames_k(const tgx_object* __restrict__ objects,
                                                     const uint32_t* __restrict__ cptrs,
                                                     const uint32_t* __restrict__ c2o,
@@ -175,128 +168,284 @@ __global__ __launch_bounds__(256) void svo_frames_k(const tgx_object* __restrict
     frames[cp] = f;
 }
 
-/* Level 0: the root's pairs are the non-empty cluster pointers in order. */
-__global__ void svo_compact_k(const uint32_t* __restrict__ nonempty, const uint32_t* __restrict__ pos, uint32_t n,
-                              uint32_t* __restrict__ out_coord, uint32_t* __restrict__ out_cptr)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !nonempty[i]) return;
-    out_coord[pos[i]] = 0u;
-    out_cptr[pos[i]] = i;
-}
-
 /* Packed node coordinates: x | y << 10 | z << 20. */
 __device__ static inline void unpack(uint32_t p, uint32_t& x, uint32_t& y, uint32_t& z)
 {
     x = p & 0x3FFu; y = (p >> 10) & 0x3FFu; z = p >> 20;
 }
 
-__global__ __launch_bounds__(256) void svo_children_k(const uint32_t* __restrict__ coord, const uint32_t* __restrict__ cptr,
-                                                      uint32_t n, const svo_frame* __restrict__ frames, float mnx,
-                                                      float mny, float mnz, float side,
-                                                      uint32_t* __restrict__ masks, uint32_t* __restrict__ counts)
+/* The nodes of all levels as one bitmap: level l's 8^l cells in Morton order
+ * from word node_word(l), so bits in word order are the nodes in canonical
+ * order and a node's children are one byte of the next level. */
+__host__ __device__ static inline uint32_t level_words(uint32_t l) { return l < 2u ? 1u : 1u << (3u * l - 5u); }
+__host__ __device__ static inline uint32_t node_word(uint32_t l)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t x, y, z;
-    unpack(coord[i], x, y, z);
-    /* Parent box in world space: exact integers (tg_sparse_voxel_octree.c:344,359-365). */
-    const float pminx = mnx + (float)x * side, pminy = mny + (float)y * side, pminz = mnz + (float)z * side;
-    const float pmaxx = pminx + side, pmaxy = pminy + side, pmaxz = pminz + side;
-    const float cex = (pmaxx - pminx) * 0.5f, cey = (pmaxy - pminy) * 0.5f, cez = (pmaxz - pminz) * 0.5f;
-    const float* m = frames[cptr[i]].ws2ms;
-    uint32_t mask = 0;
-    for (uint32_t c = 0; c < 8; c++) {
-        const float cminx = pminx + (float)(c % 2) * cex;
-        const float cminy = pminy + (float)((c / 2) % 2) * cey;
-        const float cminz = pminz + (float)((c / 4) % 2) * cez;
-        const float cmaxx = cminx + cex, cmaxy = cminy + cey, cmaxz = cminz + cez;
-        f3 k[8];
-        for (int j = 0; j < 8; j++)
-            k[j] = mulv(m, (j & 1) ? cmaxx : cminx, (j & 2) ? cmaxy : cminy, (j & 4) ? cmaxz : cminz, 1.0f);
-        if (obb_overlaps_cluster(k)) mask |= 1u << c;
+    uint32_t w = 0u;
+    for (uint32_t k = 0; k < l; k++) w += level_words(k);
+    return w;
+}
+
+/* Counters of a build (u32): pairs of level l at l, then the summary the host
+ * reads: first node of level l at SVO_CNT_BASE + l, all nodes after the last;
+ * leaves that an update took over at SVO_CNT_REUSED. */
+#define SVO_CNT_BASE 16u
+#define SVO_CNT_REUSED 31u
+#define SVO_CNT_N    32u
+
+/* Children of the level's (node, cluster pointer) pairs: eight lanes per pair,
+ * one child each (tg_intersect_aabb_obb_ignore_contact). The survivors are
+ * appended to the next level's pairs, in no order (the leaf level's are sorted
+ * once), up to cap of them; *n_out counts all. Their cells, one byte per pair,
+ * are set in the level's bitmap. Level 0 takes the non-empty cluster pointers
+ * themselves (coord null).
+ * What bounds it is the bitmap's atomics, which leave the XCD: at depth 11
+ * and 60 k leaf pairs the last level takes 77 us with an atomic per child, 60
+ * with one per pair, and 25 where each block gathers them in LDS and adds the
+ * words that are not yet set. That is done up to 8192 words (level 6); beyond,
+ * a block would clear and read more words than it has pairs. Two blocks of 16
+ * waves per CU loop over the pairs, so that there are few maps to add. All
+ * levels: 116 us, and no host round trip, for what took 145 us in the tests
+ * alone (a lane per pair, its eight children in turn) and 295 us in scans and
+ * sorts. */
+#define EXPAND_BLOCK 1024u
+#define EXPAND_PAIRS (EXPAND_BLOCK / 8u)
+#define EXPAND_LDS_WORDS 8192u
+#define EXPAND_BLOCKS 512u
+__global__ __launch_bounds__(EXPAND_BLOCK) void svo_expand_k(const uint32_t* __restrict__ coord,
+                                                             const uint32_t* __restrict__ cptr,
+                                                             const uint32_t* __restrict__ nonempty,
+                                                             const uint32_t* __restrict__ n_in, uint32_t n_max,
+                                                             const svo_frame* __restrict__ frames, float mnx, float mny,
+                                                             float mnz, float side, uint32_t* __restrict__ n_out,
+                                                             uint32_t* __restrict__ out_coord,
+                                                             uint32_t* __restrict__ out_cptr, uint32_t cap,
+                                                             uint32_t* __restrict__ map, uint32_t map_words)
+{
+    __shared__ uint32_t s_map[EXPAND_LDS_WORDS];
+    const bool lds = map_words <= EXPAND_LDS_WORDS;
+    const uint32_t n_all = coord ? *n_in : n_max, n = n_all < n_max ? n_all : n_max;
+    if (blockIdx.x * EXPAND_PAIRS >= n) return;
+    if (lds) {
+        for (uint32_t w = threadIdx.x; w < map_words; w += EXPAND_BLOCK) s_map[w] = 0u;
+        __syncthreads();
     }
-    masks[i] = mask;
-    counts[i] = (uint32_t)__popc(mask);
-}
-
-__global__ void svo_emit_k(const uint32_t* __restrict__ coord, const uint32_t* __restrict__ cptr, uint32_t n,
-                           const uint32_t* __restrict__ masks, const uint32_t* __restrict__ off,
-                           uint32_t* __restrict__ out_coord, uint32_t* __restrict__ out_cptr)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t x, y, z;
-    unpack(coord[i], x, y, z);
-    const uint32_t mask = masks[i];
-    uint32_t o = off[i];
-    for (uint32_t c = 0; c < 8; c++) {
-        if (!(mask & (1u << c))) continue;
-        const uint32_t cx = 2u * x + (c & 1u), cy = 2u * y + ((c >> 1) & 1u), cz = 2u * z + ((c >> 2) & 1u);
-        out_coord[o] = cx | (cy << 10) | (cz << 20);
-        out_cptr[o] = cptr[i];
-        o++;
+    const uint32_t c = threadIdx.x & 7u;
+    for (uint32_t base = blockIdx.x * EXPAND_PAIRS; base < n; base += gridDim.x * EXPAND_PAIRS) {
+        const uint32_t i = base + (threadIdx.x >> 3);
+        bool in = i < n && (coord || nonempty[i]);
+        uint32_t x = 0u, y = 0u, z = 0u, cp = 0u;
+        if (in) {
+            cp = coord ? cptr[i] : i;
+            unpack(coord ? coord[i] : 0u, x, y, z);
+            /* Parent box in world space: exact integers (tg_sparse_voxel_octree.c:344,359-365). */
+            const float pminx = mnx + (float)x * side, pminy = mny + (float)y * side, pminz = mnz + (float)z * side;
+            const float pmaxx = pminx + side, pmaxy = pminy + side, pmaxz = pminz + side;
+            const float cex = (pmaxx - pminx) * 0.5f, cey = (pmaxy - pminy) * 0.5f, cez = (pmaxz - pminz) * 0.5f;
+            const float cminx = pminx + (float)(c % 2) * cex;
+            const float cminy = pminy + (float)((c / 2) % 2) * cey;
+            const float cminz = pminz + (float)((c / 4) % 2) * cez;
+            const float cmaxx = cminx + cex, cmaxy = cminy + cey, cmaxz = cminz + cez;
+            const float* m = frames[cp].ws2ms;
+            f3 k[8];
+            for (int j = 0; j < 8; j++)
+                k[j] = mulv(m, (j & 1) ? cmaxx : cminx, (j & 2) ? cmaxy : cminy, (j & 4) ? cmaxz : cminz, 1.0f);
+            in = obb_overlaps_cluster(k);
+        }
+        const uint32_t slot = block_append<EXPAND_BLOCK>(n_out, in ? 1u : 0u);
+        if (in) {
+            const uint32_t cx = 2u * x + (c & 1u), cy = 2u * y + ((c >> 1) & 1u), cz = 2u * z + (c >> 2);
+            if (slot < cap) {
+                out_coord[slot] = cx | (cy << 10) | (cz << 20);
+                out_cptr[slot] = cp;
+            }
+        }
+        /* a pair's children are one byte of the bitmap */
+        const uint32_t kids = (uint32_t)(__ballot(in) >> (threadIdx.x & 56u)) & 0xFFu;
+        if (c == 0u && kids) {
+            const uint32_t mc = 8u * morton3(x, y, z), v = kids << (mc & 31u);
+            if (lds) atomicOr(&s_map[mc >> 5], v);
+            else if (v & ~__hip_atomic_load(&map[mc >> 5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicOr(&map[mc >> 5], v);
+        }
+        __syncthreads(); /* block_append's shared words and s_map */
     }
+    if (lds)
+        for (uint32_t w = threadIdx.x; w < map_words; w += EXPAND_BLOCK) {
+            const uint32_t v = s_map[w];
+            if (v & ~__hip_atomic_load(&map[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&map[w], v);
+        }
 }
 
-__global__ void svo_morton_k(const uint32_t* __restrict__ coord, uint32_t n, uint32_t* __restrict__ key)
+/* Counters and bitmap cleared, but for the root's bit. */
+__global__ __launch_bounds__(256) void svo_levels_init_k(uint32_t* __restrict__ cnt, uint32_t n)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t x, y, z;
-    unpack(coord[i], x, y, z);
-    key[i] = morton3(x, y, z);
+    if (i < n) cnt[i] = i == SVO_CNT_N ? 1u : 0u;
 }
 
-__global__ void svo_unique_flags_k(const uint32_t* __restrict__ key, uint32_t n, uint32_t* __restrict__ flag)
+/* Exclusive scan of count(i), i < n, by one block of 1024 threads that take
+ * eight counts each. Returns the total. */
+template <typename F>
+__device__ static inline uint32_t one_block_scan(uint32_t n, F count, uint32_t* __restrict__ out)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    flag[i] = (i == 0 || key[i] != key[i - 1]) ? 1u : 0u;
+    __shared__ uint32_t s_wave[16];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t before = 0u;
+    for (uint32_t base = 0; base < n; base += 8192u) {
+        const uint32_t i = base + 8u * threadIdx.x;
+        uint32_t c[8], sum = 0u;
+        for (uint32_t k = 0; k < 8u; k++) {
+            c[k] = sum;
+            sum += i + k < n ? count(i + k) : 0u;
+        }
+        uint32_t incl = sum;
+        for (uint32_t off = 1; off < 64u; off <<= 1) {
+            const uint32_t v = __shfl_up(incl, off);
+            if (lane >= off) incl += v;
+        }
+        if (lane == 63u) s_wave[wave] = incl;
+        __syncthreads();
+        uint32_t total = 0u, mine = before + incl - sum;
+        for (uint32_t w = 0; w < 16u; w++) {
+            if (w < wave) mine += s_wave[w];
+            total += s_wave[w];
+        }
+        for (uint32_t k = 0; k < 8u; k++)
+            if (i + k < n) out[i + k] = mine + c[k];
+        before += total;
+        __syncthreads();
+    }
+    return before;
 }
 
-/* One thread per pair starting a node: creates the node (canonical index
- * base + rank) and links it to its parent one level up. */
-__global__ void svo_nodes_k(const uint32_t* __restrict__ key, const uint32_t* __restrict__ flag,
-                            const uint32_t* __restrict__ rank, uint32_t n, uint32_t level, uint32_t base,
-                            uint32_t is_leaf_level, const uint32_t* __restrict__ parent_keys, uint32_t n_parent,
-                            uint32_t parent_base, svo_gnode* __restrict__ nodes, uint32_t* __restrict__ first_pair)
+__global__ __launch_bounds__(256) void svo_popc_k(const uint32_t* __restrict__ map, uint32_t n,
+                                                  uint32_t* __restrict__ count)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    const uint32_t r = rank[i];
-    const uint32_t idx = base + r;
-    const uint32_t k = key[i];
-    first_pair[r] = i;
+    if (i < n) count[i] = (uint32_t)__popc(map[i]);
+}
+
+/* Numbers the nodes (pre: nodes before each bitmap word, unless scanned
+ * already) and tells the host, in its own memory, the pairs and the first node
+ * of every level. One block, 5 us per 8192 words: the 9 k words of depth 11
+ * take it 10 us, where counting, a scan over the chip, the sums and a copy were
+ * five launches and 23 us. Beyond SVO_ONE_BLOCK_MAX it is those. */
+#define SVO_ONE_BLOCK_MAX 16384u
+__global__ __launch_bounds__(1024) void svo_number_k(const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ map,
+                                                     uint32_t map_words, uint32_t leaf_level, uint32_t scanned,
+                                                     uint32_t* pre, uint32_t* __restrict__ host)
+{
+    const uint32_t total = scanned ? pre[map_words - 1u] + (uint32_t)__popc(map[map_words - 1u])
+                                   : one_block_scan(map_words, [&](uint32_t i) { return (uint32_t)__popc(map[i]); }, pre);
+    const uint32_t l = threadIdx.x;
+    __threadfence_block();
+    __syncthreads();
+    if (l > leaf_level + 1u) return;
+    host[SVO_CNT_BASE + l] = l <= leaf_level ? pre[node_word(l)] : total;
+    host[l] = cnt[l];
+}
+
+/* Canonical index of the node of Morton cell m on the level whose bitmap
+ * starts at word w0 (its bit must be set). */
+__device__ static inline uint32_t node_index(const uint32_t* __restrict__ map, const uint32_t* __restrict__ pre,
+                                             uint32_t w0, uint32_t m)
+{
+    const uint32_t w = w0 + (m >> 5);
+    return pre[w] + (uint32_t)__popc(map[w] & ((1u << (m & 31u)) - 1u));
+}
+
+/* All nodes from the bitmap, a thread per cell. */
+__global__ __launch_bounds__(256) void svo_nodes_k(const uint32_t* __restrict__ map, const uint32_t* __restrict__ pre,
+                                                   uint32_t map_words, uint32_t leaf_level, uint32_t leaf_base,
+                                                   svo_gnode* __restrict__ nodes, uint32_t* __restrict__ leaf_keys)
+{
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, w = t >> 5;
+    if (w >= map_words || !((map[w] >> (t & 31u)) & 1u)) return;
+    uint32_t level = 0u, w0 = 0u;
+    while (w >= w0 + level_words(level)) w0 += level_words(level++);
+    const uint32_t m = t - (w0 << 5);
+    const uint32_t idx = node_index(map, pre, w0, m);
     svo_gnode nd;
     nd.first_child = SVO_NONE;
-    nd.leaf_idx = is_leaf_level ? r : SVO_NONE;
+    nd.parent = level ? node_index(map, pre, node_word(level - 1u), m >> 3) : SVO_NONE;
+    nd.leaf_idx = SVO_NONE;
     nd.masks = level << 16;
-    nd.cx = compact3(k);
-    nd.cy = compact3(k >> 1);
-    nd.cz = compact3(k >> 2);
-    nd.leaf_n = 0;
-    /* parent: Morton code >> 3 among the sorted keys of the level above */
-    const uint32_t pk = k >> 3;
-    uint32_t lo = 0, hi = n_parent;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (parent_keys[mid] < pk) lo = mid + 1; else hi = mid;
+    if (level < leaf_level) {
+        const uint32_t w1 = w0 + level_words(level);
+        const uint32_t kids = (map[w1 + ((8u * m) >> 5)] >> ((8u * m) & 31u)) & 0xFFu;
+        if (kids) {
+            nd.first_child = node_index(map, pre, w1, 8u * m + (uint32_t)__ffs((int)kids) - 1u);
+            nd.masks |= kids | (level + 1u == leaf_level ? kids << 8 : 0u);
+        }
+    } else {
+        nd.leaf_idx = idx - leaf_base;
+        leaf_keys[nd.leaf_idx] = m;
     }
-    const uint32_t parent = parent_base + lo;
-    nd.parent = parent;
+    nd.cx = compact3(m);
+    nd.cy = compact3(m >> 1);
+    nd.cz = compact3(m >> 2);
+    nd.leaf_n = 0;
     nodes[idx] = nd;
-    const uint32_t bit = 1u << (k & 7u);
-    atomicOr(&nodes[parent].masks, is_leaf_level ? (bit | (bit << 8)) : bit);
-    atomicMin(&nodes[parent].first_child, idx);
 }
 
-/* Keys of the distinct nodes of a level, in order. */
-__global__ void svo_node_keys_k(const uint32_t* __restrict__ key, const uint32_t* __restrict__ flag,
-                                const uint32_t* __restrict__ rank, uint32_t n, uint32_t* __restrict__ node_keys)
+/* Sort keys of the leaf level's pairs: leaf index << cptr_bits | cluster
+ * pointer, so that each leaf's clusters come in pointer order (the
+ * reference's list order). */
+__global__ __launch_bounds__(256) void svo_pair_keys_k(const uint32_t* __restrict__ coord, const uint32_t* __restrict__ cptr,
+                                                       uint32_t n, const uint32_t* __restrict__ map,
+                                                       const uint32_t* __restrict__ pre, uint32_t leaf_level,
+                                                       uint32_t leaf_base, uint32_t cptr_bits,
+                                                       uint64_t* __restrict__ key)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && flag[i]) node_keys[rank[i]] = key[i];
+    if (i >= n) return;
+    uint32_t x, y, z;
+    unpack(coord[i], x, y, z);
+    const uint32_t leaf = node_index(map, pre, node_word(leaf_level), morton3(x, y, z)) - leaf_base;
+    key[i] = ((uint64_t)leaf << cptr_bits) | cptr[i];
+}
+
+/* Cluster pointers of the sorted pairs and each leaf's first pair. */
+__global__ __launch_bounds__(256) void svo_pair_split_k(const uint64_t* __restrict__ key, uint32_t n, uint32_t cptr_bits,
+                                                        uint32_t* __restrict__ cptr, uint32_t* __restrict__ first_pair)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t leaf = (uint32_t)(key[i] >> cptr_bits);
+    cptr[i] = (uint32_t)(key[i] & ((1ull << cptr_bits) - 1ull));
+    if (i == 0u || (uint32_t)(key[i - 1u] >> cptr_bits) != leaf) first_pair[leaf] = i;
+}
+
+/* Totals of two exclusive scans over n counts, written behind the offsets
+ * and to the host's out[0..1]; out[2] takes *extra (null: 0). */
+__global__ void svo_totals_k(const uint32_t* __restrict__ count0, uint32_t* __restrict__ off0,
+                             const uint32_t* __restrict__ count1, uint32_t* __restrict__ off1, uint32_t n,
+                             const uint32_t* __restrict__ extra, uint32_t* __restrict__ out)
+{
+    if (threadIdx.x == 2u) out[2] = extra ? *extra : 0u;
+    if (threadIdx.x > 1u) return;
+    const uint32_t* c = threadIdx.x ? count1 : count0;
+    uint32_t* o = threadIdx.x ? off1 : off0;
+    const uint32_t t = n ? o[n - 1u] + c[n - 1u] : 0u;
+    o[n] = t;
+    out[threadIdx.x] = t;
+}
+
+/* Both scans with their totals in one launch, a block each: 5 us at 3.4 k
+ * leaves, against 14 in three launches, which are what longer counts take. */
+__global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict__ count0, uint32_t* __restrict__ off0,
+                                                      const uint32_t* __restrict__ count1, uint32_t* __restrict__ off1,
+                                                      uint32_t n, const uint32_t* __restrict__ extra,
+                                                      uint32_t* __restrict__ out)
+{
+    const uint32_t* c = blockIdx.x ? count1 : count0;
+    uint32_t* o = blockIdx.x ? off1 : off0;
+    const uint32_t t = one_block_scan(n, [&](uint32_t i) { return c[i]; }, o);
+    if (threadIdx.x == 0u) {
+        o[n] = t;
+        out[blockIdx.x] = t;
+        if (blockIdx.x) out[2] = extra ? *extra : 0u;
+    }
 }
 
 /* Leaf sampling. A leaf's candidate clusters are staged LEAF_STAGE at a time:
@@ -654,22 +803,47 @@ __global__ __launch_bounds__(256) void svo_match_k(const uint32_t* __restrict__ 
     }
 }
 
-/* candidate cluster pointers -> cluster indices (kept for the next update) */
-__global__ void svo_cand_k(const uint32_t* __restrict__ pair_cptr, uint32_t n, const svo_frame* __restrict__ frames,
-                           uint32_t* __restrict__ out)
+/* What the next update compares against: leaf keys, first pairs, candidate
+ * cluster indices; and no cluster is dirty any more. */
+__global__ __launch_bounds__(256) void svo_keep_k(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ first,
+                                                  uint32_t n_leaves, const uint32_t* __restrict__ pair_cptr,
+                                                  uint32_t n_pairs, const svo_frame* __restrict__ frames,
+                                                  uint32_t dirty_words, uint32_t* __restrict__ prev_keys,
+                                                  uint32_t* __restrict__ prev_off, uint32_t* __restrict__ prev_cand,
+                                                  uint32_t* __restrict__ dirty)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = frames[pair_cptr[i]].cidx;
+    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;; i += step) {
+        if (i < n_leaves) prev_keys[i] = keys[i];
+        if (i <= n_leaves) prev_off[i] = i < n_leaves ? first[i] : n_pairs;
+        if (i < n_pairs) prev_cand[i] = frames[pair_cptr[i]].cidx;
+        if (i < dirty_words) dirty[i] = 0u;
+        if (i >= n_leaves && i >= n_pairs && i >= dirty_words) return;
+    }
 }
 
-__global__ void svo_list_compact_k(const uint32_t* __restrict__ leaf_first_pair, const uint32_t* __restrict__ leaf_n,
-                                   const uint32_t* __restrict__ list_off, uint32_t n_leaves,
-                                   const uint32_t* __restrict__ list_tmp, uint32_t* __restrict__ list)
+/* A wave per leaf: one bit per 8^3 brick (bx + 4 by + 16 bz, a lane each) that
+ * holds a solid voxel; and with list_tmp the leaf's list from its first
+ * pair's place to its offset. */
+__global__ __launch_bounds__(256) void svo_bricks_k(const uint32_t* __restrict__ leaf_bits, uint32_t n_leaves,
+                                                    unsigned long long* __restrict__ bricks,
+                                                    const uint32_t* __restrict__ list_tmp,
+                                                    const uint32_t* __restrict__ first_pair,
+                                                    const uint32_t* __restrict__ leaf_n,
+                                                    const uint32_t* __restrict__ list_off, uint32_t* __restrict__ list)
 {
-    const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t l = blockIdx.x * 4u + (threadIdx.x >> 6), t = threadIdx.x & 63u;
     if (l >= n_leaves) return;
-    const uint32_t b = leaf_first_pair[l], o = list_off[l];
-    for (uint32_t i = 0; i < leaf_n[l]; i++) list[o + i] = list_tmp[b + i];
+    const uint32_t bx = t & 3u, by = (t >> 2) & 3u, bz = t >> 4;
+    const uint32_t* g = leaf_bits + (size_t)l * TGX_SVO_BLOCK_WORDS;
+    uint32_t acc = 0;
+    for (uint32_t z = 8u * bz; z < 8u * bz + 8u; z++)
+        for (uint32_t y = 8u * by; y < 8u * by + 8u; y++) acc |= (g[32u * z + y] >> (8u * bx)) & 0xFFu;
+    const unsigned long long m = __ballot(acc != 0u);
+    if (t == 0) bricks[l] = m;
+    if (!list_tmp) return;
+    const uint32_t b = first_pair[l], o = list_off[l], n = leaf_n[l];
+    for (uint32_t i = t; i < n; i += 64u) list[o + i] = list_tmp[b + i];
 }
 
 /* Leaf grid for traversal, one entry per 32^3 cell of the root (cell x | y
@@ -697,21 +871,6 @@ __global__ __launch_bounds__(256) void svo_grid_k(const svo_gnode* __restrict__ 
     }
     const uint32_t leaf = nodes[node].leaf_idx;
     grid[i] = bricks[leaf] ? leaf : SVO_GRID_EMPTY;
-}
-
-/* Per leaf, one bit per 8^3 brick (bx + 4 by + 16 bz) that holds a solid
- * voxel. One wave per leaf, one lane per brick. */
-__global__ __launch_bounds__(64) void svo_bricks_k(const uint32_t* __restrict__ leaf_bits,
-                                                   unsigned long long* __restrict__ bricks)
-{
-    const uint32_t t = threadIdx.x;
-    const uint32_t bx = t & 3u, by = (t >> 2) & 3u, bz = t >> 4;
-    const uint32_t* g = leaf_bits + (size_t)blockIdx.x * TGX_SVO_BLOCK_WORDS;
-    uint32_t acc = 0;
-    for (uint32_t z = 8u * bz; z < 8u * bz + 8u; z++)
-        for (uint32_t y = 8u * by; y < 8u * by + 8u; y++) acc |= (g[32u * z + y] >> (8u * bx)) & 0xFFu;
-    const unsigned long long m = __ballot(acc != 0u);
-    if (t == 0) bricks[blockIdx.x] = m;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -790,27 +949,17 @@ struct arena_scope {
         }
     }
 };
-/* Pinned scratch of the SVO code: bytes [64, 128) of the context's pinned
+/* Pinned scratch of the SVO code: bytes [64, 192) of the context's pinned
  * page (bytes [0, 64) hold the visibility statistics readback). */
 inline uint32_t* svo_pinned(tgx_context* ctx) { return (uint32_t*)((char*)ctx->host_pinned + 64); }
-int read_u32(tgx_context* ctx, const uint32_t* dev, uint32_t* out)
-{
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync(svo_pinned(ctx), dev, 4, hipMemcpyDeviceToHost, ctx->stream));
-    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    *out = *svo_pinned(ctx);
-    return TGX_OK;
-}
-/* total of an exclusive scan = last offset + last count */
-int scan_total(tgx_context* ctx, const uint32_t* counts, const uint32_t* offs, uint32_t n, uint32_t* total)
-{
-    if (n == 0) { *total = 0; return TGX_OK; }
-    uint32_t* h = svo_pinned(ctx);
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync(h, offs + n - 1, 4, hipMemcpyDeviceToHost, ctx->stream));
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync(h + 1, counts + n - 1, 4, hipMemcpyDeviceToHost, ctx->stream));
-    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    *total = h[0] + h[1];
-    return TGX_OK;
-}
+/* The arena as it was at construction, for a step that is run again with
+ * larger arrays (what spilled stays until the build ends). */
+struct arena_mark {
+    tgx_context* ctx;
+    size_t       used;
+    explicit arena_mark(tgx_context* c) : ctx(c), used(c->svo_arena_used) {}
+    void release() const { ctx->svo_arena_used = used; }
+};
 }  // namespace
 
 extern "C" {
@@ -872,8 +1021,8 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
 
     if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_frames, sizeof(svo_frame) * (size_t)n_cptr, "svo frames"))) return rc;
     svo_frame* frames = (svo_frame*)ctx->svo_frames.ptr;
-    dbuf nonempty, pos;
-    if ((rc = dalloc(ctx, nonempty, 4ull * n_cptr, "svo flags")) || (rc = dalloc(ctx, pos, 4ull * n_cptr, "svo positions"))) return rc;
+    dbuf nonempty;
+    if ((rc = dalloc(ctx, nonempty, 4ull * n_cptr, "svo flags"))) return rc;
     {
         tgx_launch_scope s(ctx, "svo_frames_k");
         hipLaunchKernelGGL(svo_frames_k, dim3(blocks_for(n_cptr)), dim3(256), 0, ctx->stream,
@@ -882,106 +1031,101 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
                            frames, nonempty.as<uint32_t>());
     }
     TGX_LAUNCH_CHECK(ctx, "svo_frames_k");
-    if ((rc = tgx_prim_exclusive_scan_u32(ctx, nonempty.as<uint32_t>(), pos.as<uint32_t>(), n_cptr))) return rc;
-    uint32_t n_pairs = 0;
-    if ((rc = scan_total(ctx, nonempty.as<uint32_t>(), pos.as<uint32_t>(), n_cptr, &n_pairs))) return rc;
 
-    /* Per level: pairs (coords, cptr) in emission order, then sorted. */
-    std::vector<dbuf> lvl_coord(leaf_level + 1), lvl_cptr(leaf_level + 1);
-    std::vector<uint32_t> lvl_n(leaf_level + 1, 0);
-    if ((rc = dalloc(ctx, lvl_coord[0], 4ull * n_pairs, "svo pairs")) || (rc = dalloc(ctx, lvl_cptr[0], 4ull * n_pairs, "svo pairs"))) return rc;
-    lvl_n[0] = n_pairs;
-    hipLaunchKernelGGL(svo_compact_k, dim3(blocks_for(n_cptr)), dim3(256), 0, ctx->stream, nonempty.as<uint32_t>(),
-                       pos.as<uint32_t>(), n_cptr, lvl_coord[0].as<uint32_t>(), lvl_cptr[0].as<uint32_t>());
-    TGX_LAUNCH_CHECK(ctx, "svo_compact_k");
-
-    for (uint32_t l = 0; l < leaf_level; l++) {
-        const uint32_t n = lvl_n[l];
-        dbuf masks, counts, offs;
-        if ((rc = dalloc(ctx, masks, 4ull * n, "svo masks")) || (rc = dalloc(ctx, counts, 4ull * n, "svo counts")) ||
-            (rc = dalloc(ctx, offs, 4ull * n, "svo offsets")))
+    /* Levels: the pairs of one level give the next one's, in two arrays that
+     * take turns, and the nodes' bitmap. No count comes back in between: the
+     * arrays hold 3 pairs per cluster pointer (rotated boxes on a noise scene
+     * need 1.8) or what the last build needed, and a level that needs more is
+     * found afterwards and the levels run again. */
+    const uint32_t map_words = node_word(leaf_level + 1u);
+    dbuf map;
+    if ((rc = dalloc(ctx, map, 4ull * (SVO_CNT_N + 3ull * map_words), "svo node bitmap"))) return rc;
+    uint32_t* cnt = map.as<uint32_t>();
+    uint32_t* bits_of = cnt + SVO_CNT_N;
+    uint32_t* pre = bits_of + map_words;
+    uint32_t* popc = pre + map_words;
+    uint32_t* h = svo_pinned(ctx);
+    uint32_t leaf_cnt[2 * SVO_CNT_BASE];
+    const uint32_t *leaf_coord = nullptr, *leaf_cptr = nullptr;
+    uint64_t cap = 3ull * n_cptr + 4096ull;
+    if (cap < ctx->svo_pairs_need) cap = ctx->svo_pairs_need + ctx->svo_pairs_need / 4u;
+    for (;;) {
+        if (cap > 0xF0000000ull) return tgx_fail(ctx, TGX_ERR_CAPACITY, "too many (node, cluster) pairs");
+        const arena_mark mark(ctx);
+        dbuf pairs[2];
+        if ((rc = dalloc(ctx, pairs[0], 8ull * cap, "svo pairs")) || (rc = dalloc(ctx, pairs[1], 8ull * cap, "svo pairs")))
             return rc;
-        const float side = (float)(1u << (depth - l));
-        if (n) {
-            tgx_launch_scope s(ctx, "svo_children_k");
-            hipLaunchKernelGGL(svo_children_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, lvl_coord[l].as<uint32_t>(),
-                               lvl_cptr[l].as<uint32_t>(), n, frames, mn[0], mn[1], mn[2], side, masks.as<uint32_t>(),
-                               counts.as<uint32_t>());
+        hipLaunchKernelGGL(svo_levels_init_k, dim3(blocks_for(SVO_CNT_N + map_words)), dim3(256), 0, ctx->stream, cnt,
+                           SVO_CNT_N + map_words);
+        for (uint32_t l = 0; l < leaf_level; l++) {
+            const uint32_t n_max = l ? (uint32_t)cap : n_cptr;
+            const uint64_t blocks = ((uint64_t)n_max + EXPAND_PAIRS - 1u) / EXPAND_PAIRS;
+            const uint32_t* in = pairs[l & 1u].as<uint32_t>();
+            uint32_t* out = pairs[(l + 1u) & 1u].as<uint32_t>();
+            tgx_launch_scope s(ctx, "svo_expand_k");
+            hipLaunchKernelGGL(svo_expand_k, dim3((uint32_t)(blocks < EXPAND_BLOCKS ? blocks : EXPAND_BLOCKS)), dim3(EXPAND_BLOCK), 0,
+                               ctx->stream, l ? in : (const uint32_t*)nullptr, in + cap, nonempty.as<uint32_t>(), cnt + l,
+                               n_max, frames, mn[0], mn[1], mn[2], (float)(1u << (depth - l)), cnt + l + 1u, out,
+                               out + cap, (uint32_t)cap, bits_of + node_word(l + 1u), level_words(l + 1u));
         }
-        TGX_LAUNCH_CHECK(ctx, "svo_children_k");
-        if ((rc = tgx_prim_exclusive_scan_u32(ctx, counts.as<uint32_t>(), offs.as<uint32_t>(), n))) return rc;
-        uint32_t next = 0;
-        if ((rc = scan_total(ctx, counts.as<uint32_t>(), offs.as<uint32_t>(), n, &next))) return rc;
-        if ((rc = dalloc(ctx, lvl_coord[l + 1], 4ull * next, "svo pairs")) || (rc = dalloc(ctx, lvl_cptr[l + 1], 4ull * next, "svo pairs"))) return rc;
-        if (n)
-            hipLaunchKernelGGL(svo_emit_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, lvl_coord[l].as<uint32_t>(),
-                               lvl_cptr[l].as<uint32_t>(), n, masks.as<uint32_t>(), offs.as<uint32_t>(),
-                               lvl_coord[l + 1].as<uint32_t>(), lvl_cptr[l + 1].as<uint32_t>());
-        TGX_LAUNCH_CHECK(ctx, "svo_emit_k");
-        lvl_n[l + 1] = next;
+        TGX_LAUNCH_CHECK(ctx, "svo_expand_k");
+        const bool wide = map_words > SVO_ONE_BLOCK_MAX;
+        if (wide) {
+            hipLaunchKernelGGL(svo_popc_k, dim3(blocks_for(map_words)), dim3(256), 0, ctx->stream, bits_of, map_words, popc);
+            if ((rc = tgx_prim_exclusive_scan_u32(ctx, popc, pre, map_words))) return rc;
+        }
+        hipLaunchKernelGGL(svo_number_k, dim3(1), dim3(1024), 0, ctx->stream, cnt, bits_of, map_words, leaf_level,
+                           wide ? 1u : 0u, pre, h);
+        TGX_LAUNCH_CHECK(ctx, "svo_number_k");
+        TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        uint64_t need = 0;
+        for (uint32_t l = 1; l <= leaf_level && need <= cap; l++) need = h[l] > need ? h[l] : need;
+        ctx->svo_pairs_need = need;
+        if (need <= cap) {
+            memcpy(leaf_cnt, h, sizeof(leaf_cnt));
+            leaf_coord = pairs[leaf_level & 1u].as<uint32_t>();
+            leaf_cptr = leaf_coord + cap;
+            break;
+        }
+        cap = need + need / 4u;
+        mark.release();
     }
-
-    /* Sort each level by Morton code (stable: clusters stay in pointer
-     * order within a node) and count the distinct nodes. */
-    std::vector<dbuf> lvl_keys(leaf_level + 1), lvl_scptr(leaf_level + 1), lvl_flag(leaf_level + 1),
-        lvl_rank(leaf_level + 1), lvl_node_keys(leaf_level + 1);
-    std::vector<uint32_t> lvl_nodes(leaf_level + 1, 0), lvl_base(leaf_level + 1, 0);
-    lvl_nodes[0] = 1;
-    uint32_t total_nodes = 1;
-    for (uint32_t l = 1; l <= leaf_level; l++) {
-        const uint32_t n = lvl_n[l];
-        dbuf raw;
-        if ((rc = dalloc(ctx, raw, 4ull * n, "svo keys")) || (rc = dalloc(ctx, lvl_keys[l], 4ull * n, "svo keys")) ||
-            (rc = dalloc(ctx, lvl_scptr[l], 4ull * n, "svo cptr")) || (rc = dalloc(ctx, lvl_flag[l], 4ull * n, "svo flags")) ||
-            (rc = dalloc(ctx, lvl_rank[l], 4ull * n, "svo ranks")))
-            return rc;
-        if (n) hipLaunchKernelGGL(svo_morton_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, lvl_coord[l].as<uint32_t>(), n, raw.as<uint32_t>());
-        TGX_LAUNCH_CHECK(ctx, "svo_morton_k");
-        if ((rc = tgx_prim_sort_pairs_u32(ctx, raw.as<uint32_t>(), lvl_keys[l].as<uint32_t>(), lvl_cptr[l].as<uint32_t>(),
-                                          lvl_scptr[l].as<uint32_t>(), n, 3u * l)))
-            return rc;
-        if (n) hipLaunchKernelGGL(svo_unique_flags_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, lvl_keys[l].as<uint32_t>(), n, lvl_flag[l].as<uint32_t>());
-        TGX_LAUNCH_CHECK(ctx, "svo_unique_flags_k");
-        if ((rc = tgx_prim_exclusive_scan_u32(ctx, lvl_flag[l].as<uint32_t>(), lvl_rank[l].as<uint32_t>(), n))) return rc;
-        uint32_t cnt = 0;
-        if ((rc = scan_total(ctx, lvl_flag[l].as<uint32_t>(), lvl_rank[l].as<uint32_t>(), n, &cnt))) return rc;
-        lvl_nodes[l] = cnt;
-        lvl_base[l] = total_nodes;
-        total_nodes += cnt;
-        if ((rc = dalloc(ctx, lvl_node_keys[l], 4ull * cnt, "svo node keys"))) return rc;
-        if (n) hipLaunchKernelGGL(svo_node_keys_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, lvl_keys[l].as<uint32_t>(),
-                                  lvl_flag[l].as<uint32_t>(), lvl_rank[l].as<uint32_t>(), n, lvl_node_keys[l].as<uint32_t>());
-        TGX_LAUNCH_CHECK(ctx, "svo_node_keys_k");
-    }
-    const uint32_t n_leaves = lvl_nodes[leaf_level];
+    const uint32_t n_leaf_pairs = leaf_cnt[leaf_level];
+    const uint32_t leaf_base = leaf_cnt[SVO_CNT_BASE + leaf_level];
+    const uint32_t total_nodes = leaf_cnt[SVO_CNT_BASE + leaf_level + 1u];
+    const uint32_t n_leaves = total_nodes - leaf_base;
 
     if (total_nodes >= 0xFFFFFFu)
-        return tgx_fail(ctx, TGX_ERR_CAPACITY, "the SVO has %u nodes; traversal holds node indices in 24 bits", total_nodes);
-    /* Nodes: root, then each level linked to its parents. */
+        return tgx_fail(ctx, TGX_ERR_CAPACITY, "the SVO has %u nodes; the limit is 2^24 - 2", total_nodes);
     if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_nodes, sizeof(svo_gnode) * (size_t)total_nodes, "svo nodes"))) return rc;
     svo_gnode* nodes = (svo_gnode*)ctx->svo_nodes.ptr;
+    dbuf leaf_keys, keys, keys2, pair_cptr, first;
+    if ((rc = dalloc(ctx, leaf_keys, 4ull * n_leaves, "svo leaf keys")) ||
+        (rc = dalloc(ctx, keys, 8ull * n_leaf_pairs, "svo pair keys")) ||
+        (rc = dalloc(ctx, keys2, 8ull * n_leaf_pairs, "svo pair keys")) ||
+        (rc = dalloc(ctx, pair_cptr, 4ull * n_leaf_pairs, "svo pairs")) ||
+        (rc = dalloc(ctx, first, 4ull * (n_leaves + 1ull), "svo first pair")))
+        return rc;
     {
-        const svo_gnode root = {SVO_NONE, SVO_NONE, SVO_NONE, 0u, 0u, 0u, 0u, 0u};
-        TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-        memcpy((char*)ctx->host_pinned + 256, &root, sizeof(root));
-        TGX_HIP_CHECK(ctx, hipMemcpyAsync(nodes, (char*)ctx->host_pinned + 256, sizeof(root), hipMemcpyHostToDevice, ctx->stream));
+        tgx_launch_scope s(ctx, "svo_nodes_k");
+        hipLaunchKernelGGL(svo_nodes_k, dim3(blocks_for(32ull * map_words)), dim3(256), 0, ctx->stream, bits_of, pre,
+                           map_words, leaf_level, leaf_base, nodes, leaf_keys.as<uint32_t>());
     }
-    dbuf root_key;
-    if ((rc = dalloc(ctx, root_key, 4, "svo root key"))) return rc;
-    hipLaunchKernelGGL(svo_fill_k, dim3(1), dim3(64), 0, ctx->stream, root_key.as<uint32_t>(), 1ull, 0u);
-    std::vector<dbuf> lvl_first(leaf_level + 1);
-    for (uint32_t l = 1; l <= leaf_level; l++) {
-        const uint32_t n = lvl_n[l];
-        if ((rc = dalloc(ctx, lvl_first[l], 4ull * (lvl_nodes[l] + 1), "svo first pair"))) return rc;
-        const uint32_t* pkeys = l == 1 ? root_key.as<uint32_t>() : lvl_node_keys[l - 1].as<uint32_t>();
-        if (n) {
-            tgx_launch_scope s(ctx, "svo_nodes_k");
-            hipLaunchKernelGGL(svo_nodes_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, lvl_keys[l].as<uint32_t>(),
-                               lvl_flag[l].as<uint32_t>(), lvl_rank[l].as<uint32_t>(), n, l, lvl_base[l],
-                               l == leaf_level ? 1u : 0u, pkeys, lvl_nodes[l - 1], lvl_base[l - 1], nodes,
-                               lvl_first[l].as<uint32_t>());
-        }
-        TGX_LAUNCH_CHECK(ctx, "svo_nodes_k");
+    TGX_LAUNCH_CHECK(ctx, "svo_nodes_k");
+    if (n_leaf_pairs) {
+        uint32_t cptr_bits = 1u, leaf_bits_n = 1u;
+        while (cptr_bits < 32u && (n_cptr - 1u) >> cptr_bits) cptr_bits++;
+        while ((n_leaves - 1u) >> leaf_bits_n) leaf_bits_n++;
+        hipLaunchKernelGGL(svo_pair_keys_k, dim3(blocks_for(n_leaf_pairs)), dim3(256), 0, ctx->stream, leaf_coord,
+                           leaf_cptr, n_leaf_pairs, bits_of, pre, leaf_level, leaf_base, cptr_bits, keys.as<uint64_t>());
+        TGX_LAUNCH_CHECK(ctx, "svo_pair_keys_k");
+        if ((rc = tgx_prim_sort_keys_u64(ctx, keys.as<uint64_t>(), keys2.as<uint64_t>(), n_leaf_pairs,
+                                         cptr_bits + leaf_bits_n)))
+            return rc;
+        hipLaunchKernelGGL(svo_pair_split_k, dim3(blocks_for(n_leaf_pairs)), dim3(256), 0, ctx->stream,
+                           keys2.as<uint64_t>(), n_leaf_pairs, cptr_bits, pair_cptr.as<uint32_t>(),
+                           first.as<uint32_t>());
+        TGX_LAUNCH_CHECK(ctx, "svo_pair_split_k");
     }
 
     /* Leaves. */
@@ -992,23 +1136,19 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_n, 4ull * nl, "svo leaf n")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_list_off, 4ull * (nl + 1), "svo list offsets")))
         return rc;
-    const uint32_t n_leaf_pairs = lvl_n[leaf_level];
     dbuf list_tmp, solid;
     if ((rc = dalloc(ctx, list_tmp, 4ull * (n_leaf_pairs ? n_leaf_pairs : 1), "svo list")) ||
         (rc = dalloc(ctx, solid, 4ull * nl, "svo solid counts")))
         return rc;
     dbuf reuse;
     if (update && n_leaves) {
-        if ((rc = dalloc(ctx, reuse, 4ull * n_leaves + 4, "svo reuse"))) return rc;
-        uint32_t* n_reused = reuse.as<uint32_t>() + n_leaves;
-        hipLaunchKernelGGL(svo_fill_k, dim3(1), dim3(64), 0, ctx->stream, n_reused, 1ull, 0u);
+        if ((rc = dalloc(ctx, reuse, 4ull * n_leaves, "svo reuse"))) return rc;
         hipLaunchKernelGGL(svo_match_k, dim3((n_leaves + 3u) / 4u), dim3(256), 0, ctx->stream,
-                           lvl_node_keys[leaf_level].as<uint32_t>(), lvl_first[leaf_level].as<uint32_t>(), n_leaf_pairs,
-                           n_leaves, lvl_scptr[leaf_level].as<uint32_t>(), frames, (const uint8_t*)ctx->cl_dirty.ptr, (const uint32_t*)ctx->svo_prev_keys.ptr,
+                           leaf_keys.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs,
+                           n_leaves, pair_cptr.as<uint32_t>(), frames, (const uint8_t*)ctx->cl_dirty.ptr, (const uint32_t*)ctx->svo_prev_keys.ptr,
                            ctx->svo_prev_leaves, (const uint32_t*)ctx->svo_prev_off.ptr,
-                           (const uint32_t*)ctx->svo_prev_cand.ptr, reuse.as<uint32_t>(), n_reused);
+                           (const uint32_t*)ctx->svo_prev_cand.ptr, reuse.as<uint32_t>(), cnt + SVO_CNT_REUSED);
         TGX_LAUNCH_CHECK(ctx, "svo_match_k");
-        if ((rc = read_u32(ctx, n_reused, &ctx->svo_reused))) return rc;
     }
     /* Leaf sampling in two passes: bits, lists and solid counts; then,
      * with the counts scanned into material offsets, the materials of the
@@ -1017,8 +1157,8 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
     const uint32_t* rz = update ? reuse.as<uint32_t>() : nullptr;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_k");
-        hipLaunchKernelGGL(svo_leaf_k, dim3(n_leaves), dim3(LEAF_BLOCK), 0, ctx->stream, nodes, lvl_base[leaf_level],
-                           lvl_scptr[leaf_level].as<uint32_t>(), lvl_first[leaf_level].as<uint32_t>(), n_leaf_pairs,
+        hipLaunchKernelGGL(svo_leaf_k, dim3(n_leaves), dim3(LEAF_BLOCK), 0, ctx->stream, nodes, leaf_base,
+                           pair_cptr.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs,
                            n_leaves, frames, (const uint32_t*)ctx->bits.ptr, mn[0], mn[1], mn[2], quirk,
                            (uint32_t*)ctx->svo_leaf_bits.ptr, solid.as<uint32_t>(), (uint16_t*)ctx->svo_leaf_wpre.ptr,
                            (uint32_t*)ctx->svo_leaf_n.ptr, list_tmp.as<uint32_t>(), nodes, rz,
@@ -1027,47 +1167,49 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
                            (const uint32_t*)ctx->svo_old_list_off.ptr, (const uint32_t*)ctx->svo_old_list.ptr);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_k");
-    if ((rc = tgx_prim_exclusive_scan_u32(ctx, solid.as<uint32_t>(), (uint32_t*)ctx->svo_leaf_moff.ptr, n_leaves))) return rc;
-    uint32_t n_solid = 0;
-    if ((rc = scan_total(ctx, solid.as<uint32_t>(), (const uint32_t*)ctx->svo_leaf_moff.ptr, n_leaves, &n_solid))) return rc;
-    *(uint32_t*)((char*)ctx->host_pinned + 336) = n_solid;
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync((uint32_t*)ctx->svo_leaf_moff.ptr + n_leaves, (char*)ctx->host_pinned + 336, 4,
-                                      hipMemcpyHostToDevice, ctx->stream));
-    if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_mats, 2ull * (n_solid ? n_solid : 1), "svo leaf materials"))) return rc;
+    /* material offsets and list offsets, their totals read back together */
+    const uint32_t* n_reused = update && n_leaves ? cnt + SVO_CNT_REUSED : (const uint32_t*)nullptr;
+    uint32_t* moff = (uint32_t*)ctx->svo_leaf_moff.ptr;
+    uint32_t* list_off = (uint32_t*)ctx->svo_list_off.ptr;
+    const uint32_t* leaf_n = (const uint32_t*)ctx->svo_leaf_n.ptr;
+    if (n_leaves <= SVO_ONE_BLOCK_MAX) {
+        hipLaunchKernelGGL(svo_offsets_k, dim3(2), dim3(1024), 0, ctx->stream, solid.as<uint32_t>(), moff, leaf_n, list_off,
+                           n_leaves, n_reused, h);
+    } else {
+        if ((rc = tgx_prim_exclusive_scan_u32(ctx, solid.as<uint32_t>(), moff, n_leaves)) ||
+            (rc = tgx_prim_exclusive_scan_u32(ctx, leaf_n, list_off, n_leaves)))
+            return rc;
+        hipLaunchKernelGGL(svo_totals_k, dim3(1), dim3(64), 0, ctx->stream, solid.as<uint32_t>(), moff, leaf_n, list_off,
+                           n_leaves, n_reused, h);
+    }
+    TGX_LAUNCH_CHECK(ctx, "svo_offsets_k");
+    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    const uint32_t n_solid = h[0], n_list = h[1];
+    ctx->svo_reused = h[2];
+    if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_mats, 2ull * (n_solid ? n_solid : 1), "svo leaf materials")) ||
+        (rc = tgx_buffer_reserve(ctx, &ctx->svo_list, 4ull * (n_list ? n_list : 1), "svo list")))
+        return rc;
     ctx->svo_n_solid = n_solid;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_mats_k");
         hipLaunchKernelGGL(svo_leaf_mats_k, dim3(n_leaves * LEAF_PARTS), dim3(LEAF_BLOCK), 0, ctx->stream, nodes,
-                           lvl_base[leaf_level], lvl_scptr[leaf_level].as<uint32_t>(),
-                           lvl_first[leaf_level].as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
+                           leaf_base, pair_cptr.as<uint32_t>(),
+                           first.as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
                            (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx), mn[0], mn[1], mn[2], quirk,
                            (const uint32_t*)ctx->svo_leaf_bits.ptr, (const uint16_t*)ctx->svo_leaf_wpre.ptr,
                            (const uint32_t*)ctx->svo_leaf_moff.ptr, (uint16_t*)ctx->svo_leaf_mats.ptr, rz,
                            (const uint32_t*)ctx->svo_old_moff.ptr, (const uint16_t*)ctx->svo_old_mats.ptr);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_mats_k");
-    if ((rc = tgx_prim_exclusive_scan_u32(ctx, (const uint32_t*)ctx->svo_leaf_n.ptr, (uint32_t*)ctx->svo_list_off.ptr, n_leaves))) return rc;
-    uint32_t n_list = 0;
-    if ((rc = scan_total(ctx, (const uint32_t*)ctx->svo_leaf_n.ptr, (const uint32_t*)ctx->svo_list_off.ptr, n_leaves, &n_list))) return rc;
-    *(uint32_t*)((char*)ctx->host_pinned + 320) = n_list;
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync((uint32_t*)ctx->svo_list_off.ptr + n_leaves, (char*)ctx->host_pinned + 320, 4,
-                                      hipMemcpyHostToDevice, ctx->stream));
-    if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_list, 4ull * (n_list ? n_list : 1), "svo list"))) return rc;
-    if (n_leaves)
-        hipLaunchKernelGGL(svo_list_compact_k, dim3(blocks_for(n_leaves)), dim3(256), 0, ctx->stream,
-                           lvl_first[leaf_level].as<uint32_t>(), (const uint32_t*)ctx->svo_leaf_n.ptr,
-                           (const uint32_t*)ctx->svo_list_off.ptr, n_leaves, list_tmp.as<uint32_t>(),
-                           (uint32_t*)ctx->svo_list.ptr);
-    TGX_LAUNCH_CHECK(ctx, "svo_list_compact_k");
-
-    /* Traversal layout: leaf brick masks and the leaf grid. */
-    const uint32_t n_inner = lvl_base[leaf_level];
+    /* Lists; and the traversal layout: leaf brick masks and the leaf grid. */
+    const uint32_t n_inner = leaf_base;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_grid, 4ull << (3u * leaf_level), "svo leaf grid")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_bricks, 8ull * nl, "svo leaf bricks")))
         return rc;
     if (n_leaves)
-        hipLaunchKernelGGL(svo_bricks_k, dim3(n_leaves), dim3(64), 0, ctx->stream, (const uint32_t*)ctx->svo_leaf_bits.ptr,
-                           (unsigned long long*)ctx->svo_bricks.ptr);
+        hipLaunchKernelGGL(svo_bricks_k, dim3((n_leaves + 3u) / 4u), dim3(256), 0, ctx->stream,
+                           (const uint32_t*)ctx->svo_leaf_bits.ptr, n_leaves, (unsigned long long*)ctx->svo_bricks.ptr,
+                           list_tmp.as<uint32_t>(), first.as<uint32_t>(), leaf_n, list_off, (uint32_t*)ctx->svo_list.ptr);
     TGX_LAUNCH_CHECK(ctx, "svo_bricks_k");
     hipLaunchKernelGGL(svo_grid_k, dim3(blocks_for(1ull << (3u * leaf_level))), dim3(256), 0, ctx->stream,
                        (const svo_gnode*)nodes, leaf_level, (const unsigned long long*)ctx->svo_bricks.ptr,
@@ -1079,23 +1221,13 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
             (rc = tgx_buffer_reserve(ctx, &ctx->svo_prev_off, 4ull * (nl + 1), "svo previous offsets")) ||
             (rc = tgx_buffer_reserve(ctx, &ctx->svo_prev_cand, 4ull * (n_leaf_pairs ? n_leaf_pairs : 1), "svo previous candidates")))
             return rc;
-        if (n_leaves) {
-            TGX_HIP_CHECK(ctx, hipMemcpyAsync(ctx->svo_prev_keys.ptr, lvl_node_keys[leaf_level].p, 4ull * n_leaves,
-                                              hipMemcpyDeviceToDevice, ctx->stream));
-            TGX_HIP_CHECK(ctx, hipMemcpyAsync(ctx->svo_prev_off.ptr, lvl_first[leaf_level].p, 4ull * n_leaves,
-                                              hipMemcpyDeviceToDevice, ctx->stream));
-        }
-        hipLaunchKernelGGL(svo_fill_k, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)ctx->svo_prev_off.ptr + n_leaves,
-                           1ull, n_leaf_pairs);
-        if (n_leaf_pairs)
-            hipLaunchKernelGGL(svo_cand_k, dim3(blocks_for(n_leaf_pairs)), dim3(256), 0, ctx->stream,
-                               lvl_scptr[leaf_level].as<uint32_t>(), n_leaf_pairs, frames,
-                               (uint32_t*)ctx->svo_prev_cand.ptr);
-        TGX_LAUNCH_CHECK(ctx, "svo_cand_k");
         const uint64_t dirty_words = (ctx->n_clusters + 3ull) / 4ull;
-        hipLaunchKernelGGL(svo_fill_k, dim3((uint32_t)((dirty_words + 255) / 256)), dim3(256), 0, ctx->stream,
-                           (uint32_t*)ctx->cl_dirty.ptr, dirty_words, 0u);
-        TGX_LAUNCH_CHECK(ctx, "svo_fill_k");
+        const uint64_t most = n_leaf_pairs > dirty_words ? n_leaf_pairs : dirty_words;
+        hipLaunchKernelGGL(svo_keep_k, dim3(blocks_for(most + 1u)), dim3(256), 0, ctx->stream, leaf_keys.as<uint32_t>(),
+                           first.as<uint32_t>(), n_leaves, pair_cptr.as<uint32_t>(), n_leaf_pairs, frames,
+                           (uint32_t)dirty_words, (uint32_t*)ctx->svo_prev_keys.ptr, (uint32_t*)ctx->svo_prev_off.ptr,
+                           (uint32_t*)ctx->svo_prev_cand.ptr, (uint32_t*)ctx->cl_dirty.ptr);
+        TGX_LAUNCH_CHECK(ctx, "svo_keep_k");
         ctx->svo_prev_leaves = n_leaves;
     }
     TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -1415,8 +1547,10 @@ int tgx_svo_load(tgx_context* ctx, const char* path)
     if (!list.empty())
         TGX_HIP_CHECK(ctx, hipMemcpy(ctx->svo_list.ptr, list.data(), 4ull * list.size(), hipMemcpyHostToDevice));
     if (nl)
-        hipLaunchKernelGGL(svo_bricks_k, dim3(nl), dim3(64), 0, ctx->stream, (const uint32_t*)ctx->svo_leaf_bits.ptr,
-                           (unsigned long long*)ctx->svo_bricks.ptr);
+        hipLaunchKernelGGL(svo_bricks_k, dim3((nl + 3u) / 4u), dim3(256), 0, ctx->stream,
+                           (const uint32_t*)ctx->svo_leaf_bits.ptr, nl, (unsigned long long*)ctx->svo_bricks.ptr,
+                           (const uint32_t*)nullptr, (const uint32_t*)nullptr, (const uint32_t*)nullptr,
+                           (const uint32_t*)nullptr, (uint32_t*)nullptr);
     TGX_LAUNCH_CHECK(ctx, "svo_bricks_k");
     hipLaunchKernelGGL(svo_grid_k, dim3(blocks_for(1ull << (3u * (in.depth - 5u)))), dim3(256), 0, ctx->stream,
                        (const svo_gnode*)ctx->svo_nodes.ptr, in.depth - 5u,
