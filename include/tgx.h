@@ -801,6 +801,11 @@ int tgx_visibility_last_stats(tgx_context* ctx, tgx_visibility_stats* out);
  * reference counterpart (tg rasterises instead of binning). */
 int tgx_visibility_set_list_capacity(tgx_context* ctx, uint32_t entries);
 
+/* Compares the device's short reciprocal and square root with IEEE ones over
+ * every float in [2^-100, 2^100], which the kernels' exact results rely on:
+ * mismatches[0] of 1 / d, [1] of sqrt(d). No reference counterpart. */
+int tgx_arith_check(tgx_context* ctx, uint64_t mismatches[2]);
+
 #ifdef __cplusplus
 }
 #endif

@@ -212,6 +212,7 @@ def load_library() -> ctypes.CDLL:
         "tgx_visibility_decode": (i32, [u64, ctypes.POINTER(ctypes.c_float), ctypes.POINTER(u32), ctypes.POINTER(u32)]),
         "tgx_visibility_last_stats": (i32, [vp, ctypes.POINTER(VisibilityStats)]),
         "tgx_visibility_set_list_capacity": (i32, [vp, u32]),
+        "tgx_arith_check": (i32, [vp, vp]),
         "tgx_device_alloc": (i32, [vp, ctypes.c_size_t, ctypes.POINTER(vp)]),
         "tgx_device_free": (i32, [vp, vp]),
         "tgx_memcpy_d2h": (i32, [vp, vp, vp, ctypes.c_size_t]),
@@ -500,6 +501,12 @@ class Context:
 
     def set_list_capacity(self, entries: int) -> None:
         self._check(self.lib.tgx_visibility_set_list_capacity(self.h, entries), "tgx_visibility_set_list_capacity")
+
+    def arith_check(self) -> tuple[int, int]:
+        """tgx_arith_check: mismatches of the device's short 1 / d and sqrt(d)."""
+        out = np.zeros(2, np.uint64)
+        self._check(self.lib.tgx_arith_check(self.h, _ptr(out)), "tgx_arith_check")
+        return int(out[0]), int(out[1])
 
     # -- sparse voxel octree ------------------------------------------------
 

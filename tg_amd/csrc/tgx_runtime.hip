@@ -3,6 +3,7 @@
  * entry points of the C ABI (declared in include/tgx.h).
  */
 #include "tgx_internal.h"
+#include "tgx_exact.h"
 
 #include <algorithm>
 
@@ -355,6 +356,41 @@ int tgx_profile_get(tgx_context* ctx, tgx_kernel_stat* out, uint32_t capacity, u
     const uint32_t n = (uint32_t)ctx->stats.size();
     for (uint32_t i = 0; i < n && i < capacity && out; i++) out[i] = ctx->stats[i];
     *out_n = n;
+    return TGX_OK;
+}
+
+/* Every float of [2^-100, 2^100]: bits lo..hi. */
+static __global__ __launch_bounds__(256) void arith_check_k(uint32_t lo, uint32_t hi, unsigned long long* __restrict__ bad)
+{
+    uint32_t n_recip = 0u, n_root = 0u;
+    for (uint32_t u = lo + blockIdx.x * blockDim.x + threadIdx.x; u <= hi; u += gridDim.x * blockDim.x) {
+        const float d = __uint_as_float(u);
+        n_recip += exact_recip(d) != 1.0f / d ? 1u : 0u;
+        n_root += exact_root(d) != sqrtf(d) ? 1u : 0u;
+    }
+    if (n_recip) atomicAdd(&bad[0], (unsigned long long)n_recip);
+    if (n_root) atomicAdd(&bad[1], (unsigned long long)n_root);
+}
+
+int tgx_arith_check(tgx_context* ctx, uint64_t mismatches[2])
+{
+    if (!ctx || !mismatches) return TGX_ERR_INVALID_ARG;
+    ctx->last_error.clear();
+    TGX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    tgx_buffer b;
+    int rc;
+    if ((rc = tgx_buffer_reserve(ctx, &b, 16, "arithmetic check"))) return rc;
+    const uint64_t zero[2] = {0, 0};
+    hipError_t e = hipMemcpyAsync(b.ptr, zero, 16, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(arith_check_k, dim3(2048), dim3(256), 0, ctx->stream, 27u << 23, 227u << 23,
+                           (unsigned long long*)b.ptr);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(mismatches, b.ptr, 16, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    tgx_buffer_release(&b);
+    if (e != hipSuccess) return tgx_fail(ctx, TGX_ERR_HIP, "arithmetic check: %s", hipGetErrorString(e));
     return TGX_OK;
 }
 

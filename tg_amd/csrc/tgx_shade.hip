@@ -14,6 +14,7 @@
  * (and in the oracle) as ((x x)(x x)) x.
  */
 #include "tgx_internal.h"
+#include "tgx_exact.h"
 #include "tgx_m4.h"
 
 struct shade_cam {
@@ -55,8 +56,7 @@ __device__ static inline float3 sh_ggx(float3 n, float3 v, float3 l, float3 alb,
                                        float roughness, float radiance)
 {
     float hx = v.x + l.x, hy = v.y + l.y, hz = v.z + l.z;
-    const float hm = sqrtf(hx * hx + hy * hy + hz * hz);
-    hx = hx / hm; hy = hy / hm; hz = hz / hm;
+    exact_normalize3(hx, hy, hz);
     const float h_dot_n = hx * n.x + hy * n.y + hz * n.z;
     const float l_dot_n = n.x * l.x + n.y * l.y + n.z * l.z;
     const float n_dot_v = n.x * v.x + n.y * v.y + n.z * v.z;
@@ -93,14 +93,15 @@ __global__ __launch_bounds__(256) void shade_k(const tgx_object* __restrict__ ob
                                                const uint32_t* __restrict__ cptrs, const uint32_t* __restrict__ c2o,
                                                const uint8_t* __restrict__ materials,
                                                const tgx_lut_entry* __restrict__ luts, shade_cam cam, uint32_t W,
-                                               uint32_t H, const uint64_t* __restrict__ vis, shade_consts k,
+                                               uint32_t H, float inv_w, float inv_h, exact_div div_w,
+                                               const uint64_t* __restrict__ vis, shade_consts k,
                                                float4* __restrict__ out)
 {
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
     if (pix >= W * H) return;
-    const uint32_t px = pix % W, py = pix / W;
+    const uint32_t py = exact_div_floor(pix, div_w), px = pix - py * W;
     const uint64_t word = vis[pix];
-    const float depth = (float)(word >> 40) / 16777215.0f;
+    const float depth = exact_quot((float)(word >> 40), 16777215.0f, 1.0f / 16777215.0f);
     if (!(depth < 1.0f)) {
         out[pix] = make_float4(k.miss[0], k.miss[1], k.miss[2], k.miss[3]);
         return;
@@ -114,11 +115,11 @@ __global__ __launch_bounds__(256) void shade_k(const tgx_object* __restrict__ ob
     const tgx_lut_entry e = luts[(size_t)ob.lut_idx * TGX_LUT_ENTRIES + mat];
 
     /* ray in cluster space and the hit voxel's face normal (shading.frag:141-229) */
-    const float fx = ((float)px + 0.5f) / (float)W;
-    const float fy = 1.0f - ((float)py + 0.5f) / (float)H;
+    const float fx = exact_quot((float)px + 0.5f, (float)W, inv_w);
+    const float fy = 1.0f - exact_quot((float)py + 0.5f, (float)H, inv_h);
     const uint32_t rel = cptr - ob.first_cluster_pointer;
     const uint32_t nx = ob.n_cluster_pointers_per_dim[0], ny = ob.n_cluster_pointers_per_dim[1];
-    const uint32_t rx = rel % nx, ry = (rel / nx) % ny, rz = rel / (nx * ny);
+    const uint32_t row = rel / nx, rx = rel - row * nx, rz = row / ny, ry = row - rz * ny;
     const tgx_m4 w2c = tgx_world_to_cluster(ob.rotation, ob.translation, ob.n_cluster_pointers_per_dim, rx, ry, rz);
     const tgx_v4 o4 = tgx_m4_mulv4(w2c, cam.pos[0], cam.pos[1], cam.pos[2], 1.0f);
     const float omy = 1.0f - fy, omx = 1.0f - fx;
@@ -126,20 +127,15 @@ __global__ __launch_bounds__(256) void shade_k(const tgx_object* __restrict__ ob
     const float qx = cam.br[0] * omy + cam.tr[0] * fy, qy = cam.br[1] * omy + cam.tr[1] * fy, qz = cam.br[2] * omy + cam.tr[2] * fy;
     const float dwx = lx * omx + qx * fx, dwy = ly * omx + qy * fx, dwz = lz * omx + qz * fx;
     const tgx_v4 d4 = tgx_m4_mulv4(w2c, dwx, dwy, dwz, 0.0f);
-    const float dm = sqrtf(d4.x * d4.x + d4.y * d4.y + d4.z * d4.z);
-    const float ddx = d4.x / dm, ddy = d4.y / dm, ddz = d4.z / dm;
+    float ddx = d4.x, ddy = d4.y, ddz = d4.z;
+    exact_normalize3(ddx, ddy, ddz);
     const float vmx = (float)(v % 8u), vmy = (float)((v / 8u) % 8u), vmz = (float)(v / 64u);
     /* tg_intersect_ray_aabb (collide.inc:3-24) with the voxel box */
-    const float ax0 = ddx == 0.0f ? -3.402823466e+38f : (vmx - o4.x) / ddx;
-    const float ay0 = ddy == 0.0f ? -3.402823466e+38f : (vmy - o4.y) / ddy;
-    const float az0 = ddz == 0.0f ? -3.402823466e+38f : (vmz - o4.z) / ddz;
-    const float bx0 = ddx == 0.0f ? 3.402823466e+38f : ((vmx + 1.0f) - o4.x) / ddx;
-    const float by0 = ddy == 0.0f ? 3.402823466e+38f : ((vmy + 1.0f) - o4.y) / ddy;
-    const float bz0 = ddz == 0.0f ? 3.402823466e+38f : ((vmz + 1.0f) - o4.z) / ddz;
-    const float enter = sh_max(sh_max(sh_min(ax0, bx0), sh_min(ay0, by0)), sh_min(az0, bz0));
-    const float exit_ = sh_min(sh_min(sh_max(ax0, bx0), sh_max(ay0, by0)), sh_max(az0, bz0));
+    float enter, exit_;
+    const bool face = exact_slab(o4.x, o4.y, o4.z, ddx, ddy, ddz, vmx, vmy, vmz, vmx + 1.0f, vmy + 1.0f, vmz + 1.0f, enter,
+                                 exit_);
     float3 n = make_float3(0.0f, 0.0f, 0.0f);
-    if (exit_ > 0.0f && enter <= exit_) {
+    if (face) {
         float hx = o4.x, hy = o4.y, hz = o4.z;
         if (enter > 0.0f) { hx = o4.x + enter * ddx; hy = o4.y + enter * ddy; hz = o4.z + enter * ddz; }
         float mx = hx - (vmx + 0.5f), my = hy - (vmy + 0.5f), mz = hz - (vmz + 0.5f);
@@ -153,8 +149,8 @@ __global__ __launch_bounds__(256) void shade_k(const tgx_object* __restrict__ ob
         tgx_m4 rot;
         for (int i = 0; i < 16; i++) rot.m[i] = ob.rotation[i];
         const tgx_v4 n4 = tgx_m4_mulv4(rot, mx, my, mz, 0.0f);
-        const float nm = sqrtf(n4.x * n4.x + n4.y * n4.y + n4.z * n4.z);
-        n = make_float3(n4.x / nm, n4.y / nm, n4.z / nm);
+        n = make_float3(n4.x, n4.y, n4.z);
+        exact_normalize3(n.x, n.y, n.z);
     }
 
     float4 c;
@@ -179,8 +175,7 @@ __global__ __launch_bounds__(256) void shade_k(const tgx_object* __restrict__ ob
         const float t = depth * cam.far_plane;
         const float hpx = cam.pos[0] + t * dwx, hpy = cam.pos[1] + t * dwy, hpz = cam.pos[2] + t * dwz;
         float vx = cam.pos[0] - hpx, vy = cam.pos[1] - hpy, vz = cam.pos[2] - hpz;
-        const float vm = sqrtf(vx * vx + vy * vy + vz * vz);
-        vx = vx / vm; vy = vy / vm; vz = vz / vm;
+        exact_normalize3(vx, vy, vz);
         const float om = 1.0f - k.metallic;
         const float3 spec = make_float3(0.04f * om + alb.x * k.metallic, 0.04f * om + alb.y * k.metallic,
                                         0.04f * om + alb.z * k.metallic);
@@ -307,7 +302,8 @@ int tgx_shade_device(tgx_context* ctx, const tgx_camera* cam, uint32_t w, uint32
         hipLaunchKernelGGL(shade_k, dim3((n + 255) / 256), dim3(256), 0, ctx->stream,
                            (const tgx_object*)ctx->objects.ptr, (const uint32_t*)ctx->cluster_pointers.ptr,
                            (const uint32_t*)ctx->cluster_idx_to_object.ptr, tgx_scene_materials(ctx),
-                           (const tgx_lut_entry*)ctx->luts.ptr, sc, w, h, vis_dev, k, (float4*)rgba_dev);
+                           (const tgx_lut_entry*)ctx->luts.ptr, sc, w, h, 1.0f / (float)w, 1.0f / (float)h, exact_div_of(w),
+                           vis_dev, k, (float4*)rgba_dev);
     }
     TGX_LAUNCH_CHECK(ctx, "shade_k");
     return TGX_OK;
