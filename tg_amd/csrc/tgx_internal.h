@@ -62,8 +62,6 @@ struct tgx_context {
     tgx_buffer   vis_stats_dev;  /* frame statistics (records, entries, max)*/
     uint32_t     vis_list_capacity = 0;   /* tile-list entries allocated    */
     uint32_t     vis_list_capacity_fixed = 0; /* caller override, 0 = auto */
-    hipEvent_t   vis_stats_event = nullptr;
-    bool         vis_stats_pending = false;
     void*        host_pinned = nullptr; /* small pinned readback area       */
     tgx_visibility_stats vis_stats = {};
 

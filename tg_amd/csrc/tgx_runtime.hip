@@ -123,6 +123,7 @@ int tgx_create(int device, tgx_context** out_ctx)
         delete ctx;
         return TGX_ERR_HIP;
     }
+    memset(ctx->host_pinned, 0, 4096);
     if (tgx_vis_scratch_init(ctx) != TGX_OK) {
         (void)hipHostFree(ctx->host_pinned);
         (void)hipStreamDestroy(ctx->stream);
@@ -153,7 +154,6 @@ int tgx_destroy(tgx_context* ctx)
     tgx_svo_release(ctx);
     tgx_nrc_release(ctx);
     if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
-    if (ctx->vis_stats_event) (void)hipEventDestroy(ctx->vis_stats_event);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return TGX_OK;

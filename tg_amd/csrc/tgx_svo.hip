@@ -293,10 +293,20 @@ __device__ static inline uint32_t one_block_scan(uint32_t n, F count, uint32_t* 
     uint32_t before = 0u;
     for (uint32_t base = 0; base < n; base += 8192u) {
         const uint32_t i = base + 8u * threadIdx.x;
+        const bool full = i + 8u <= n; /* without a test per element the accesses are 16 bytes */
         uint32_t c[8], sum = 0u;
+        if (full) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) c[k] = count(i + k);
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) c[k] = i + k < n ? count(i + k) : 0u;
+        }
+#pragma unroll
         for (uint32_t k = 0; k < 8u; k++) {
+            const uint32_t v = c[k];
             c[k] = sum;
-            sum += i + k < n ? count(i + k) : 0u;
+            sum += v;
         }
         uint32_t incl = sum;
         for (uint32_t off = 1; off < 64u; off <<= 1) {
@@ -310,8 +320,14 @@ __device__ static inline uint32_t one_block_scan(uint32_t n, F count, uint32_t* 
             if (w < wave) mine += s_wave[w];
             total += s_wave[w];
         }
-        for (uint32_t k = 0; k < 8u; k++)
-            if (i + k < n) out[i + k] = mine + c[k];
+        if (full) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) out[i + k] = mine + c[k];
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++)
+                if (i + k < n) out[i + k] = mine + c[k];
+        }
         before += total;
         __syncthreads();
     }
@@ -327,8 +343,7 @@ __global__ __launch_bounds__(256) void svo_popc_k(const uint32_t* __restrict__ m
 
 /* Numbers the nodes (pre: nodes before each bitmap word, unless scanned
  * already) and tells the host, in its own memory, the pairs and the first node
- * of every level. One block, 5 us per 8192 words: the 9 k words of depth 11
- * take it 10 us, where counting, a scan over the chip, the sums and a copy were
+ * of every level. One block: the 9 k words of depth 11 take it 5 us, where counting, a scan over the chip, the sums and a copy were
  * five launches and 23 us. Beyond SVO_ONE_BLOCK_MAX it is those. */
 #define SVO_ONE_BLOCK_MAX 16384u
 __global__ __launch_bounds__(1024) void svo_number_k(const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ map,

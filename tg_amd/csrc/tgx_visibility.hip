@@ -342,15 +342,9 @@ __device__ static bool cluster_rect(const vis_cam& cam, const tgx_object& ob, ui
  * of the grown box) lies beyond the far plane, by a margin of 0.1 % and one
  * voxel for the rounding of the pair's slab distance, holds no hit with
  * depth <= 1 and is culled for every camera. */
-__global__ __launch_bounds__(256) void vis_objcull_k(const tgx_object* __restrict__ objects, uint32_t n_objects,
-                                                     const uint2* __restrict__ obj_occ,
-                                                     const vis_cam* __restrict__ cams, uint32_t W, uint32_t H,
-                                                     uint32_t* __restrict__ objcnt)
+__device__ static uint32_t objcull_one(const tgx_object* __restrict__ objects, const uint2* __restrict__ obj_occ,
+                                       uint32_t o, const vis_cam& cam, uint32_t W, uint32_t H)
 {
-    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t ci = blockIdx.y;
-    if (o >= n_objects) return;
-    const vis_cam& cam = cams[ci];
     const tgx_object ob = objects[o];
     /* the object's cluster pointers to clusters with a solid voxel */
     const uint32_t n = obj_occ[o].y;
@@ -401,7 +395,18 @@ __global__ __launch_bounds__(256) void vis_objcull_k(const tgx_object* __restric
         const bool behind = hi[0] < VIS_RECT_EPS - 1.0f;
         if (!near_cube && (behind || left || right || below || above)) keep = 0u;
     }
-    objcnt[(size_t)ci * 3u * n_objects + o] = keep ? n : 0u;
+    return keep ? n : 0u;
+}
+
+__global__ __launch_bounds__(256) void vis_objcull_k(const tgx_object* __restrict__ objects, uint32_t n_objects,
+                                                     const uint2* __restrict__ obj_occ,
+                                                     const vis_cam* __restrict__ cams, uint32_t W, uint32_t H,
+                                                     uint32_t* __restrict__ objcnt)
+{
+    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t ci = blockIdx.y;
+    if (o >= n_objects) return;
+    objcnt[(size_t)ci * 3u * n_objects + o] = objcull_one(objects, obj_occ, o, cams[ci], W, H);
 }
 
 /* Per camera (one workgroup each): the kept objects (nonzero counts) in
@@ -409,20 +414,19 @@ __global__ __launch_bounds__(256) void vis_objcull_k(const tgx_object* __restric
  * pointers (the camera's block of objcnt holds counts, ids, offsets, n_objects
  * u32 each); total[ci] the number of cluster pointers of kept objects and
  * n_kept[ci] the number of kept objects. */
-__global__ __launch_bounds__(1024) void vis_objscan_k(uint32_t* __restrict__ objcnt, uint32_t n_objects,
-                                                      uint32_t* __restrict__ total, uint32_t* __restrict__ n_kept)
+template <typename F>
+__device__ static inline void objscan_block(F count, uint32_t* __restrict__ kid, uint32_t n_objects,
+                                            uint32_t* __restrict__ total, uint32_t* __restrict__ n_kept)
 {
     __shared__ uint32_t wsum[16], wnum[16];
     __shared__ uint32_t carry, carry_n;
     const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
-    const uint32_t* cnt = objcnt + (size_t)blockIdx.x * 3u * n_objects;
-    uint32_t* kid = objcnt + (size_t)blockIdx.x * 3u * n_objects + n_objects;
     uint32_t* koff = kid + n_objects;
     if (t == 0) { carry = 0u; carry_n = 0u; }
     __syncthreads();
     for (uint32_t base = 0; base < n_objects; base += 1024u) {
         const uint32_t i = base + t;
-        const uint32_t v = i < n_objects ? cnt[i] : 0u;
+        const uint32_t v = i < n_objects ? count(i) : 0u;
         const uint32_t f = v ? 1u : 0u;
         uint32_t incl = v, ninc = f;
 #pragma unroll
@@ -449,7 +453,63 @@ __global__ __launch_bounds__(1024) void vis_objscan_k(uint32_t* __restrict__ obj
         if (t == 0) { carry = c0 + blk; carry_n = n0 + blkn; }
         __syncthreads();
     }
-    if (t == 0) { total[blockIdx.x] = carry; n_kept[blockIdx.x] = carry_n; }
+    if (t == 0) { *total = carry; *n_kept = carry_n; }
+}
+
+__global__ __launch_bounds__(1024) void vis_objscan_k(uint32_t* __restrict__ objcnt, uint32_t n_objects,
+                                                      uint32_t* __restrict__ total, uint32_t* __restrict__ n_kept)
+{
+    uint32_t* block = objcnt + (size_t)blockIdx.x * 3u * n_objects;
+    objscan_block([&](uint32_t i) { return block[i]; }, block + n_objects, n_objects, total + blockIdx.x,
+                  n_kept + blockIdx.x);
+}
+
+/* Camera records passed by value (kernel arguments), so that a call can
+ * place them in device memory without a copy from host memory. */
+#define VIS_ARG_CAMS 16u
+struct vis_cam_pack {
+    vis_cam c[VIS_ARG_CAMS];
+};
+
+/* Begins a batch, a workgroup per camera: the camera's record (from_args:
+ * to its place in cams), cleared tile counts and counters, the call's cleared
+ * statistics, and with `cull` the object lists (objects culled and scanned by
+ * the one workgroup). One launch of 4 us in place of three fills, a copy and two
+ * passes: a call over one object at 256x256 is bound by its launches (66 us with
+ * those, a scan in three and statistics copied back; 37 so). Above VIS_CULL_ONE
+ * objects (4 culled per lane) the cull takes its own grid. */
+#define VIS_CULL_ONE 4096u
+__global__ __launch_bounds__(1024) void vis_begin_k(vis_cam_pack pack, uint32_t from_args, vis_cam* __restrict__ cams,
+                                                    const tgx_object* __restrict__ objects, uint32_t n_objects,
+                                                    const uint2* __restrict__ obj_occ, uint32_t W, uint32_t H,
+                                                    uint32_t cull, uint32_t* __restrict__ objcnt,
+                                                    uint32_t* __restrict__ tile_count, uint32_t tiles_per_cam,
+                                                    uint32_t* __restrict__ counters, uint32_t n_cams,
+                                                    uint32_t* __restrict__ stats)
+{
+    const uint32_t ci = blockIdx.x, t = threadIdx.x;
+    __shared__ vis_cam cam;
+    if (from_args) {
+        if (t < sizeof(vis_cam) / 4u) {
+            const uint32_t v = ((const uint32_t*)&pack.c[ci])[t];
+            ((uint32_t*)&cams[ci])[t] = v;
+            ((uint32_t*)&cam)[t] = v;
+        }
+    } else if (t < sizeof(vis_cam) / 4u) {
+        ((uint32_t*)&cam)[t] = ((const uint32_t*)&cams[ci])[t];
+    }
+    uint32_t* tc = tile_count + (size_t)ci * tiles_per_cam;
+    for (uint32_t i = t; i < tiles_per_cam; i += 1024u) tc[i] = 0u;
+    if (t == 0u) {
+        counters[ci] = 0u;               /* records */
+        counters[n_cams + 8u + ci] = 0u; /* global records */
+    }
+    if (ci == 0u && stats && t < 8u) stats[t] = 0u;
+    if (!cull) return;
+    __syncthreads();
+    objscan_block([&](uint32_t i) { return objcull_one(objects, obj_occ, i, cam, W, H); },
+                  objcnt + (size_t)ci * 3u * n_objects + n_objects, n_objects, counters + 2u * n_cams + 8u + ci,
+                  counters + 3u * n_cams + 8u + ci);
 }
 
 /* Builds the record of one (camera, cluster pointer) whose cluster holds a
@@ -621,11 +681,28 @@ __global__ __launch_bounds__(1024) void vis_scan_local_k(const uint32_t* __restr
 /* Scans sums[0..nb) in place. *total gets the grand total; with stats,
  * thread 0 also accumulates the visibility frame statistics: stats[0] +=
  * records of the n_cams cameras, stats[1] += list entries, stats[2] = max
- * list entries. */
+ * list entries; host (the host's own memory, if not null) gets them too. */
+__device__ static inline void stats_add(uint32_t entries, const uint32_t* __restrict__ rec_count, uint32_t n_cams,
+                                        unsigned long long* __restrict__ stats, unsigned long long* __restrict__ host)
+{
+    unsigned long long recs = stats[0];
+    for (uint32_t c = 0; c < n_cams; c++) recs += rec_count[c];
+    const unsigned long long sum = stats[1] + entries, most = entries > stats[2] ? entries : stats[2];
+    stats[0] = recs;
+    stats[1] = sum;
+    stats[2] = most;
+    if (host) {
+        host[0] = recs;
+        host[1] = sum;
+        host[2] = most;
+    }
+}
+
 __global__ __launch_bounds__(1024) void vis_scan_top_k(uint32_t* __restrict__ sums, uint32_t nb,
                                                        uint32_t* __restrict__ total,
                                                        const uint32_t* __restrict__ rec_count, uint32_t n_cams,
-                                                       unsigned long long* __restrict__ stats)
+                                                       unsigned long long* __restrict__ stats,
+                                                       unsigned long long* __restrict__ host)
 {
     __shared__ uint32_t wsum[16];
     uint32_t carry = 0u;
@@ -648,13 +725,63 @@ __global__ __launch_bounds__(1024) void vis_scan_top_k(uint32_t* __restrict__ su
     }
     if (threadIdx.x == 0) {
         *total = carry;
-        if (stats) {
-            unsigned long long recs = 0;
-            for (uint32_t c = 0; c < n_cams; c++) recs += rec_count[c];
-            stats[0] += recs;
-            stats[1] += carry;
-            if (carry > stats[2]) stats[2] = carry;
+        if (stats) stats_add(carry, rec_count, n_cams, stats, host);
+    }
+}
+
+/* The three passes in one workgroup, eight values a lane: 4.6 us for the 8160
+ * tiles of a 1080p frame, where the three launches take 13. Two rounds, for
+ * up to VIS_SCAN_ONE values, are still ahead of them. */
+#define VIS_SCAN_ONE 16384u
+__global__ __launch_bounds__(1024) void vis_scan_one_k(const uint32_t* in, uint32_t* __restrict__ out, uint32_t n,
+                                                       uint32_t* copy, uint32_t* __restrict__ total,
+                                                       const uint32_t* __restrict__ rec_count, uint32_t n_cams,
+                                                       unsigned long long* __restrict__ stats,
+                                                       unsigned long long* __restrict__ host)
+{
+    __shared__ uint32_t wsum[16];
+    uint32_t carry = 0u;
+    for (uint32_t b0 = 0; b0 < n; b0 += 8192u) {
+        const uint32_t i0 = b0 + 8u * threadIdx.x;
+        const bool full = i0 + 8u <= n; /* without a test per element the accesses are 16 bytes */
+        uint32_t v[8], s = 0u;
+        if (full) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) v[k] = in[i0 + k];
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) v[k] = i0 + k < n ? in[i0 + k] : 0u;
         }
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; k++) s += v[k];
+        uint32_t tot;
+        uint32_t run = carry + block_excl_scan(s, wsum, tot);
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; k++) {
+            const uint32_t c = v[k];
+            v[k] = run;
+            run += c;
+        }
+        if (full) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) out[i0 + k] = v[k];
+            if (copy) {
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; k++) copy[i0 + k] = v[k];
+            }
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++)
+                if (i0 + k < n) {
+                    out[i0 + k] = v[k];
+                    if (copy) copy[i0 + k] = v[k];
+                }
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) {
+        *total = carry;
+        if (stats) stats_add(carry, rec_count, n_cams, stats, host);
     }
 }
 
@@ -681,6 +808,7 @@ __global__ __launch_bounds__(1024) void vis_scan_add_k(uint32_t* __restrict__ ou
  * object of its first index with a 64-way search (one load per lane and a
  * ballot per round), then each lane steps over the objects its own index
  * has passed (kept objects have at least one cluster pointer). */
+#define VIS_LANE_TILES 16u
 __global__ __launch_bounds__(256) void vis_setup(const tgx_object* __restrict__ objects,
                                                  const uint32_t* __restrict__ cptrs,
                                                  const uint32_t* __restrict__ occ_list,
@@ -744,6 +872,20 @@ __global__ __launch_bounds__(256) void vis_setup(const tgx_object* __restrict__ 
         if (!binned) rec_flags[cam.rec_base + k] = 0u;
     }
     const uint32_t tb = cam.tile_base;
+    /* A few tiles: each lane counts its own, all rectangles at once. Taking
+     * the wave's rectangles one after the other cost 64 turns. */
+    if (binned) {
+        const uint32_t x0 = (rec.rect_lo & 0xFFFFu) >> tshift, x1 = (rec.rect_hi & 0xFFFFu) >> tshift;
+        const uint32_t y1 = (rec.rect_hi >> 16) >> tshift;
+        uint32_t x = x0, y = (rec.rect_lo >> 16) >> tshift;
+        if ((x1 - x0 + 1u) * (y1 - y + 1u) <= VIS_LANE_TILES) {
+            binned = false;
+            while (y <= y1) {
+                atomicAdd(&tile_count[tb + y * tiles_x + x], 1u);
+                if (x++ == x1) { x = x0; y++; }
+            }
+        }
+    }
     for_each_rect_tile(binned, binned ? rec.rect_lo : 0u, binned ? rec.rect_hi : 0u, 0ull, tshift,
                        [&](uint64_t, uint32_t tx, uint32_t ty) { atomicAdd(&tile_count[tb + ty * tiles_x + tx], 1u); });
     }
@@ -757,19 +899,6 @@ __global__ void vis_fill_u32(uint32_t* __restrict__ p, uint32_t n, uint32_t valu
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = value;
-}
-
-/* Camera records passed by value (kernel arguments), so that a call can
- * place them in device memory without a copy from host memory. */
-#define VIS_ARG_CAMS 16u
-struct vis_cam_pack {
-    vis_cam c[VIS_ARG_CAMS];
-};
-
-__global__ void vis_cams_k(vis_cam_pack pack, uint32_t n, vis_cam* __restrict__ out)
-{
-    const uint32_t i = threadIdx.x;
-    if (i < n) out[i] = pack.c[i];
 }
 
 /* Each list entry is the sort key (depth_lb24 << 32) | record slot. Eight
@@ -978,11 +1107,17 @@ static uint32_t scan_groups(uint64_t n) { return (uint32_t)((n + VIS_SCAN_BLOCK 
  * statistics are accumulated as well (see vis_scan_top_k). */
 static int scan_launch(tgx_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* sums,
                        uint32_t* copy, uint32_t* total, const uint32_t* rec_count = nullptr, uint32_t n_cams = 0,
-                       unsigned long long* stats = nullptr)
+                       unsigned long long* stats = nullptr, unsigned long long* host = nullptr)
 {
+    if (n <= VIS_SCAN_ONE) {
+        hipLaunchKernelGGL(vis_scan_one_k, dim3(1), dim3(1024), 0, ctx->stream, in, out, n, copy, total, rec_count, n_cams,
+                           stats, host);
+        TGX_LAUNCH_CHECK(ctx, "vis_scan_one_k");
+        return TGX_OK;
+    }
     const uint32_t nb = scan_groups(n);
     if (nb) hipLaunchKernelGGL(vis_scan_local_k, dim3(nb), dim3(1024), 0, ctx->stream, in, out, n, sums);
-    hipLaunchKernelGGL(vis_scan_top_k, dim3(1), dim3(1024), 0, ctx->stream, sums, nb, total, rec_count, n_cams, stats);
+    hipLaunchKernelGGL(vis_scan_top_k, dim3(1), dim3(1024), 0, ctx->stream, sums, nb, total, rec_count, n_cams, stats, host);
     if (nb) hipLaunchKernelGGL(vis_scan_add_k, dim3(nb), dim3(1024), 0, ctx->stream, out, n, sums, copy);
     TGX_LAUNCH_CHECK(ctx, "vis_scan");
     return TGX_OK;
@@ -1063,7 +1198,10 @@ static uint32_t tiles_of(uint32_t n, uint32_t shift) { return (n + (1u << shift)
 
 /* Device buffers of one visibility batch. */
 struct vis_bufs {
-    const vis_cam*      cams;
+    vis_cam*            cams;
+    const vis_cam_pack* pack;       /* the cameras by value; null: cams holds them */
+    bool                clear_stats;
+    unsigned long long* host_stats; /* host memory for the statistics, or null */
     const uint32_t*     occ_list;   /* occupied cluster pointers            */
     const uint2*        obj_occ;    /* per object: first occupied entry, count */
     uint32_t            slots;      /* record slots per camera              */
@@ -1098,20 +1236,21 @@ static int visibility_launch(tgx_context* ctx, const vis_bufs& b, uint32_t n_cam
     uint32_t* d_kept = d_counters + 2 * n_cams + 8;
     uint32_t* d_nkept = d_counters + 3 * n_cams + 8;
     {
-        tgx_launch_scope s(ctx, "vis_fill_u32", b.timed);
-        hipLaunchKernelGGL(vis_fill_u32, dim3((n_tiles + 255) / 256), dim3(256), 0, ctx->stream, b.tile_count, n_tiles, 0u);
-        hipLaunchKernelGGL(vis_fill_u32, dim3((4 * n_cams + 8 + 255) / 256), dim3(256), 0, ctx->stream, d_counters,
-                           4 * n_cams + 8, 0u);
+        static const vis_cam_pack none = {};
+        const bool one = ctx->n_objects <= VIS_CULL_ONE;
+        tgx_launch_scope s(ctx, "vis_begin_k", b.timed);
+        hipLaunchKernelGGL(vis_begin_k, dim3(n_cams), dim3(1024), 0, ctx->stream, b.pack ? *b.pack : none, b.pack ? 1u : 0u,
+                           b.cams, (const tgx_object*)ctx->objects.ptr, ctx->n_objects, b.obj_occ, W, H, one ? 1u : 0u,
+                           b.objcnt, b.tile_count, tiles_per_cam, d_counters, n_cams,
+                           b.clear_stats ? (uint32_t*)b.stats : (uint32_t*)nullptr);
+        if (!one) {
+            hipLaunchKernelGGL(vis_objcull_k, dim3((ctx->n_objects + 255u) / 256u, n_cams), dim3(256), 0, ctx->stream,
+                               (const tgx_object*)ctx->objects.ptr, ctx->n_objects, b.obj_occ, b.cams, W, H, b.objcnt);
+            hipLaunchKernelGGL(vis_objscan_k, dim3(n_cams), dim3(1024), 0, ctx->stream, b.objcnt, ctx->n_objects, d_kept,
+                               d_nkept);
+        }
     }
-    TGX_LAUNCH_CHECK(ctx, "vis_fill_u32");
-    {
-        tgx_launch_scope s(ctx, "vis_objcull_k", b.timed);
-        hipLaunchKernelGGL(vis_objcull_k, dim3((ctx->n_objects + 255u) / 256u, n_cams), dim3(256), 0, ctx->stream,
-                           (const tgx_object*)ctx->objects.ptr, ctx->n_objects, b.obj_occ, b.cams, W, H, b.objcnt);
-        hipLaunchKernelGGL(vis_objscan_k, dim3(n_cams), dim3(1024), 0, ctx->stream, b.objcnt, ctx->n_objects, d_kept,
-                           d_nkept);
-    }
-    TGX_LAUNCH_CHECK(ctx, "vis_objcull_k");
+    TGX_LAUNCH_CHECK(ctx, "vis_begin_k");
     {
         tgx_launch_scope s(ctx, "vis_setup", b.timed);
         const uint32_t cap = ctx->tuning.vis_setup_blocks;
@@ -1129,7 +1268,7 @@ static int visibility_launch(tgx_context* ctx, const vis_bufs& b, uint32_t n_cam
         tgx_launch_scope s(ctx, "vis_scan", b.timed);
         int rc;
         if ((rc = scan_launch(ctx, b.tile_count, b.tile_off, n_tiles, b.scan_sums, b.tile_count, d_counters + n_cams,
-                              d_counters, n_cams, b.stats)))
+                              d_counters, n_cams, b.stats, b.host_stats)))
             return rc;
     }
     {
@@ -1179,7 +1318,7 @@ static bool batch_fits_grid(uint32_t n_cams, uint32_t W, uint32_t H, uint32_t sl
 }
 
 static int visibility_batch(tgx_context* ctx, const tgx_camera* cams, uint32_t n_cams, uint32_t W,
-                            uint32_t H, uint64_t* out_dev, const vis_cam* resident)
+                            uint32_t H, uint64_t* out_dev, const vis_cam* resident, bool first)
 {
     const uint32_t ts = vis_tile_shift(ctx);
     const uint32_t tiles_per_cam = tiles_of(W, ts) * tiles_of(H, ts);
@@ -1192,13 +1331,17 @@ static int visibility_batch(tgx_context* ctx, const tgx_camera* cams, uint32_t n
     const uint64_t n_slots = (uint64_t)slots * n_cams;
     const uint32_t n_tiles = tiles_per_cam * n_cams;
 
+    /* up to VIS_ARG_CAMS cameras travel as kernel arguments */
     std::vector<vis_cam> vc;
+    const bool by_value = !resident && n_cams <= VIS_ARG_CAMS;
+    vis_cam_pack pack;
     if (!resident) {
-        vc.resize(n_cams);
+        if (!by_value) vc.resize(n_cams);
+        vis_cam* v = by_value ? pack.c : vc.data();
         for (uint32_t i = 0; i < n_cams; i++) {
-            make_cam(cams[i], vc[i]);
-            vc[i].rec_base = i * slots;
-            vc[i].tile_base = i * tiles_per_cam;
+            make_cam(cams[i], v[i]);
+            v[i].rec_base = i * slots;
+            v[i].tile_base = i * tiles_per_cam;
         }
         if ((rc = tgx_buffer_reserve(ctx, &ctx->vis_cams, sizeof(vis_cam) * n_cams, "vis cams"))) return rc;
     }
@@ -1211,11 +1354,14 @@ static int visibility_batch(tgx_context* ctx, const tgx_camera* cams, uint32_t n
     if ((rc = tgx_buffer_reserve(ctx, &ctx->vis_objcnt, 12ull * ctx->n_objects * n_cams, "object cull lists")))
         return rc;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->vis_scan_sums, 4ull * (scan_groups(n_tiles) + 1u), "scan sums"))) return rc;
-    if (!resident)
+    if (!resident && !by_value)
         TGX_HIP_CHECK(ctx, hipMemcpyAsync(ctx->vis_cams.ptr, vc.data(), sizeof(vis_cam) * n_cams, hipMemcpyHostToDevice,
                                           ctx->stream));
     vis_bufs b;
-    b.cams = resident ? resident : (const vis_cam*)ctx->vis_cams.ptr;
+    b.cams = resident ? (vis_cam*)resident : (vis_cam*)ctx->vis_cams.ptr;
+    b.pack = by_value ? &pack : nullptr;
+    b.clear_stats = first;
+    b.host_stats = resident ? nullptr : (unsigned long long*)ctx->host_pinned;
     b.occ_list = (const uint32_t*)ctx->vis_occ.ptr + 2ull * n_cptr;
     b.obj_occ = (const uint2*)ctx->vis_obj_occ.ptr;
     b.slots = slots;
@@ -1251,11 +1397,10 @@ static int check_args(tgx_context* ctx, const tgx_camera* cams, uint32_t n_cams,
 
 /* Sizes the tile-list buffer. A frame whose lists exceed the capacity is
  * still exact (its overflowing tiles walk every record); the largest total
- * of the previous call, once its readback has landed, grows the buffer. */
+ * of the last call whose statistics have landed grows the buffer. */
 static int list_capacity_update(tgx_context* ctx, uint32_t w, uint32_t h)
 {
     int rc;
-    if (!ctx->vis_stats_event) TGX_HIP_CHECK(ctx, hipEventCreateWithFlags(&ctx->vis_stats_event, hipEventDisableTiming));
     if ((rc = tgx_buffer_reserve(ctx, &ctx->vis_stats_dev, 64, "vis stats"))) return rc;
     uint64_t want = ctx->vis_list_capacity;
     const uint32_t ts = vis_tile_shift(ctx);
@@ -1267,9 +1412,8 @@ static int list_capacity_update(tgx_context* ctx, uint32_t w, uint32_t h)
         if (2ull * ctx->n_cluster_pointers > want) want = 2ull * ctx->n_cluster_pointers;
     }
     if (ctx->vis_list_capacity_fixed) want = ctx->vis_list_capacity_fixed;
-    else if (ctx->vis_stats_pending && hipEventQuery(ctx->vis_stats_event) == hipSuccess) {
-        ctx->vis_stats_pending = false;
-        const uint64_t max_total = ((const unsigned long long*)ctx->host_pinned)[2];
+    else {
+        const uint64_t max_total = ((volatile const unsigned long long*)ctx->host_pinned)[2];
         if (max_total > want) want = max_total + max_total / 4u + 1024u;
     }
     if (want > 0xFFFFFFFFull) want = 0xFFFFFFFFull;
@@ -1323,14 +1467,13 @@ int tgx_visibility_record(tgx_context* ctx, const void* dev_cams, const tgx_came
     if (rc) return rc;
     if (!ctx->vis_tile_list.ptr || !ctx->vis_stats_dev.ptr)
         return tgx_fail(ctx, TGX_ERR_NOT_BUILT, "record a frame only after one tgx_visibility_device call");
-    hipLaunchKernelGGL(vis_fill_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)ctx->vis_stats_dev.ptr, 8u, 0u);
-    TGX_LAUNCH_CHECK(ctx, "vis_fill_u32");
     if ((rc = tgx_vis_solid_refresh(ctx))) return rc;
     const uint32_t per = batch_cams(ctx, n_cams);
     const vis_cam* rc_cams = (const vis_cam*)dev_cams;
     for (uint32_t c0 = 0; c0 < n_cams; c0 += per) {
         const uint32_t n = (n_cams - c0) < per ? (n_cams - c0) : per;
-        if ((rc = visibility_batch(ctx, cams + c0, n, w, h, out_dev + (size_t)c0 * w * h, rc_cams + c0))) return rc;
+        if ((rc = visibility_batch(ctx, cams + c0, n, w, h, out_dev + (size_t)c0 * w * h, rc_cams + c0, c0 == 0)))
+            return rc;
     }
     return TGX_OK;
 }
@@ -1346,23 +1489,18 @@ int tgx_visibility_device(tgx_context* ctx, const tgx_camera* cams, uint32_t n_c
     TGX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     memset(&ctx->vis_stats, 0, sizeof(ctx->vis_stats));
     if ((rc = list_capacity_update(ctx, w, h))) return rc;
-    {
-        tgx_launch_scope s(ctx, "vis_fill_u32");
-        hipLaunchKernelGGL(vis_fill_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)ctx->vis_stats_dev.ptr, 8u, 0u);
-    }
-    TGX_LAUNCH_CHECK(ctx, "vis_fill_u32");
     if ((rc = tgx_vis_solid_refresh(ctx))) return rc;
     const uint32_t per = batch_cams(ctx, n_cams);
     for (uint32_t c0 = 0; c0 < n_cams; c0 += per) {
         const uint32_t n = (n_cams - c0) < per ? (n_cams - c0) : per;
-        rc = visibility_batch(ctx, cams + c0, n, w, h, out_dev + (size_t)c0 * w * h, nullptr);
+        rc = visibility_batch(ctx, cams + c0, n, w, h, out_dev + (size_t)c0 * w * h, nullptr, c0 == 0);
         if (rc) return rc;
     }
-    /* Frame statistics travel back asynchronously; the next call (or
-     * tgx_visibility_last_stats) reads them. */
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync(ctx->host_pinned, ctx->vis_stats_dev.ptr, 32, hipMemcpyDeviceToHost, ctx->stream));
-    TGX_HIP_CHECK(ctx, hipEventRecord(ctx->vis_stats_event, ctx->stream));
-    ctx->vis_stats_pending = true;
+    if (ctx->n_cluster_pointers == 0) /* no batch ran a scan */
+        hipLaunchKernelGGL(vis_fill_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)ctx->host_pinned, 8u, 0u);
+    TGX_LAUNCH_CHECK(ctx, "vis_fill_u32");
+    /* The last batch's scan writes the frame statistics to host memory; the
+     * next call (or tgx_visibility_last_stats) reads them. */
     return TGX_OK;
 }
 
@@ -1515,13 +1653,15 @@ int tgx_visibility_device_noalloc(tgx_context* ctx, const tgx_camera* cams, uint
             pack.c[i].tile_base = i * tiles_per_cam;
         }
         vis_bufs b;
-        vis_cam* d_cams = (vis_cam*)carve(sizeof(vis_cam) * n);
+        b.cams = (vis_cam*)carve(sizeof(vis_cam) * n);
+        b.pack = &pack;
+        b.clear_stats = true;
+        b.host_stats = nullptr;
         uint8_t* d_solid = (uint8_t*)carve(ctx->n_clusters);
         uint32_t* d_occ = (uint32_t*)carve(12ull * n_cptr);
         uint2* d_obj_occ = (uint2*)carve(8ull * ctx->n_objects);
         uint32_t* d_sums = (uint32_t*)carve(4ull * noalloc_sums(ctx, n, tiles_per_cam));
         const vis_occ_bufs ob = {d_occ, d_occ + n_cptr, d_occ + 2ull * n_cptr, d_obj_occ, d_sums};
-        b.cams = d_cams;
         b.occ_list = d_occ + 2ull * n_cptr;
         b.obj_occ = d_obj_occ;
         b.slots = n_cptr;
@@ -1539,8 +1679,6 @@ int tgx_visibility_device_noalloc(tgx_context* ctx, const tgx_camera* cams, uint
         b.list = (uint64_t*)(base + off);
         b.capacity = entries > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)entries;
         b.timed = false;
-        hipLaunchKernelGGL(vis_cams_k, dim3(1), dim3(64), 0, ctx->stream, pack, n, d_cams);
-        TGX_LAUNCH_CHECK(ctx, "vis_cams_k");
         /* The solid flags and the occupied-pointer lists are derived from
          * the scene on every call: the array keeps whatever the last call on
          * this GPU left. */
@@ -1548,8 +1686,6 @@ int tgx_visibility_device_noalloc(tgx_context* ctx, const tgx_camera* cams, uint
                            (const uint4*)ctx->bits.ptr, ctx->n_clusters, d_solid);
         TGX_LAUNCH_CHECK(ctx, "vis_solid_k");
         if ((rc = occ_launch(ctx, d_solid, ob))) return rc;
-        hipLaunchKernelGGL(vis_fill_u32, dim3(1), dim3(64), 0, ctx->stream, (uint32_t*)b.stats, 16u, 0u);
-        TGX_LAUNCH_CHECK(ctx, "vis_fill_u32");
         if ((rc = visibility_launch(ctx, b, n, w, h, out))) return rc;
     }
     return TGX_OK;
