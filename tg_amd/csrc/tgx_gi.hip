@@ -1670,14 +1670,39 @@ __global__ void gi_gather_rays_k(const svo_ray* __restrict__ src, const uint32_t
     if (i < *n_ptr) dst[i] = src[idx[i]];
 }
 
-/* svo_res -> tgx_svo_hit for the C ABI */
-__global__ void svo_hits_k(const svo_gnode* __restrict__ nodes, const svo_res* __restrict__ res, uint32_t n,
-                           tgx_svo_hit* __restrict__ out)
+/* Ray queue of a host call, its counters cleared and the count set (cnt[6]).
+ * The arrays are the host's memory, which no cache holds: a block reads its
+ * 256 rays' floats once, in order, into LDS. */
+__global__ __launch_bounds__(256) void svo_rays_k(const float* __restrict__ origins, const float* __restrict__ dirs,
+                                                  uint32_t n, svo_ray* __restrict__ rays, uint32_t* __restrict__ cnt)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float s[2][768];
+    const uint32_t first = blockIdx.x * 256u, t = threadIdx.x;
+    const uint64_t base = 3ull * first, all = 3ull * n;
+    for (uint32_t k = t; k < 768u; k += 256u)
+        if (base + k < all) {
+            s[0][k] = origins[base + k];
+            s[1][k] = dirs[base + k];
+        }
+    if (blockIdx.x == 0u && t < GI_N_COUNTERS) cnt[t] = t == 6u ? n : 0u;
+    __syncthreads();
+    const uint32_t i = first + t;
     if (i >= n) return;
+    const svo_ray r = {s[0][3u * t], s[0][3u * t + 1u], s[0][3u * t + 2u], s[1][3u * t], s[1][3u * t + 1u], s[1][3u * t + 2u], i, 0u};
+    rays[i] = r;
+}
+
+/* svo_res -> tgx_svo_hit for the C ABI, through LDS: out may be the host's
+ * memory, to which 40-byte records of single lanes would go in pieces. */
+__global__ __launch_bounds__(256) void svo_hits_k(const svo_gnode* __restrict__ nodes, const svo_res* __restrict__ res,
+                                                  uint32_t n, tgx_svo_hit* __restrict__ out)
+{
+    __shared__ tgx_svo_hit s[256];
+    const uint32_t first = blockIdx.x * 256u, i = first + threadIdx.x;
+    constexpr uint32_t kWords = sizeof(tgx_svo_hit) / 4u;
+    tgx_svo_hit& h = s[threadIdx.x];
+    if (i < n) {
     const svo_res r = res[i];
-    tgx_svo_hit h;
     h.hit = r.flags & 1u;
     h.distance = r.distance;
     h.block[0] = h.block[1] = h.block[2] = 0u;
@@ -1689,7 +1714,11 @@ __global__ void svo_hits_k(const svo_gnode* __restrict__ nodes, const svo_res* _
         h.normal[(r.flags >> 2) & 3u] = (r.flags & 16u) ? 1 : -1;
     }
     h.steps = r.steps;
-    out[i] = h;
+    }
+    __syncthreads();
+    const uint32_t words = (n - first < 256u ? n - first : 256u) * kWords;
+    uint32_t* o = (uint32_t*)(out + first);
+    for (uint32_t k = threadIdx.x; k < words; k += 256u) o[k] = ((const uint32_t*)s)[k];
 }
 
 /* SVO primary visibility (debug_visibility_svo.frag:27-70): one ray per
@@ -2067,23 +2096,29 @@ int tgx_svo_trace(tgx_context* ctx, const float* origins, const float* direction
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_hits, (sizeof(svo_res) + sizeof(tgx_svo_hit)) * (size_t)n, "svo hits")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->gi_counts, 4ull * GI_CNT_TOTAL, "gi counters")))
         return rc;
-    std::vector<svo_ray> h(n);
-    for (uint32_t i = 0; i < n; i++)
-        h[i] = {origins[3 * i], origins[3 * i + 1], origins[3 * i + 2], directions[3 * i], directions[3 * i + 1],
-                directions[3 * i + 2], i, 0u};
+    /* Host arrays pass through pinned memory that the kernels read and write
+     * themselves: no copies on the stream, no records built on the host. */
+    const size_t in_bytes = 12ull * n, out_bytes = sizeof(tgx_svo_hit) * (size_t)n;
+    const void *in_o = nullptr, *in_d = nullptr;
+    if ((rc = tgx_stage_in(ctx, origins, in_bytes, 0, 2u * in_bytes + out_bytes, &in_o)) ||
+        (rc = tgx_stage_in(ctx, directions, in_bytes, in_bytes, 2u * in_bytes + out_bytes, &in_d)))
+        return rc;
     svo_ray* d_rays = (svo_ray*)ctx->svo_rays.ptr;
     svo_res* d_res = (svo_res*)ctx->svo_hits.ptr;
-    tgx_svo_hit* d_hits = (tgx_svo_hit*)(d_res + n);
+    tgx_svo_hit* staged = (tgx_svo_hit*)tgx_stage(ctx, 2u * in_bytes + out_bytes);
+    if (staged) staged = (tgx_svo_hit*)((char*)staged + 2u * in_bytes);
+    tgx_svo_hit* d_hits = staged ? staged : (tgx_svo_hit*)(d_res + n);
     uint32_t* cnt = (uint32_t*)ctx->gi_counts.ptr + GI_CNT_SVO;
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync(d_rays, h.data(), sizeof(svo_ray) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(gi_fill_k, dim3(1), dim3(64), 0, ctx->stream, cnt, (uint64_t)GI_N_COUNTERS, 0u);
-    hipLaunchKernelGGL(gi_fill_k, dim3(1), dim3(64), 0, ctx->stream, cnt + 6, 1ull, n);
+    hipLaunchKernelGGL(svo_rays_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, (const float*)in_o, (const float*)in_d, n,
+                       d_rays, cnt);
+    TGX_LAUNCH_CHECK(ctx, "svo_rays_k");
     if ((rc = launch_trace(ctx, d_rays, cnt + 6, n, max_distance, d_res, nullptr))) return rc;
     hipLaunchKernelGGL(svo_hits_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, (const svo_gnode*)ctx->svo_nodes.ptr,
                        d_res, n, d_hits);
     TGX_LAUNCH_CHECK(ctx, "svo_hits_k");
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync(out_host, d_hits, sizeof(tgx_svo_hit) * (size_t)n, hipMemcpyDeviceToHost, ctx->stream));
+    if (!staged) TGX_HIP_CHECK(ctx, hipMemcpyAsync(out_host, d_hits, out_bytes, hipMemcpyDeviceToHost, ctx->stream));
     TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    if (staged) memcpy(out_host, staged, out_bytes);
     return TGX_OK;
 }
 

@@ -63,6 +63,9 @@ struct tgx_context {
     uint32_t     vis_list_capacity = 0;   /* tile-list entries allocated    */
     uint32_t     vis_list_capacity_fixed = 0; /* caller override, 0 = auto */
     void*        host_pinned = nullptr; /* small pinned readback area       */
+    void*        stage = nullptr;       /* pinned, see tgx_stage             */
+    size_t       stage_bytes = 0;
+    tgx_buffer   stage_dev;             /* host arrays beyond TGX_STAGE_MAX  */
     tgx_visibility_stats vis_stats = {};
 
     /* Sparse voxel octree (built by tgx_svo_build). */
@@ -160,6 +163,16 @@ int  tgx_fail(tgx_context* ctx, int code, const char* fmt, ...);
 int  tgx_prim_exclusive_scan_u32(tgx_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n);
 int  tgx_prim_sort_pairs_u32(tgx_context* ctx, const uint32_t* keys_in, uint32_t* keys_out,
                              const uint32_t* vals_in, uint32_t* vals_out, uint32_t n, unsigned end_bit);
+/* Pinned memory of at least `bytes` for host arrays that a call takes or gives
+ * back, held until the context is destroyed; null beyond TGX_STAGE_MAX or when
+ * there is none (callers then copy through device memory). A call that uses it
+ * ends with the stream synchronised. */
+#define TGX_STAGE_MAX (32ull << 20)
+void* tgx_stage(tgx_context* ctx, size_t bytes);
+/* The host array src of `bytes`, where a kernel can read it until the call's
+ * synchronisation: in the stage at offset `at` of the `all` bytes that the
+ * call needs there, or else in device memory. */
+int  tgx_stage_in(tgx_context* ctx, const void* src, size_t bytes, size_t at, size_t all, const void** out);
 int  tgx_prim_sort_keys_u64(tgx_context* ctx, const uint64_t* keys_in, uint64_t* keys_out, uint32_t n, unsigned end_bit);
 void tgx_svo_release(tgx_context* ctx);
 void tgx_nrc_release(tgx_context* ctx);

@@ -46,6 +46,40 @@ int tgx_buffer_reserve(tgx_context* ctx, tgx_buffer* b, size_t bytes, const char
     return TGX_OK;
 }
 
+void* tgx_stage(tgx_context* ctx, size_t bytes)
+{
+    if (bytes <= ctx->stage_bytes) return ctx->stage;
+    if (bytes > TGX_STAGE_MAX) return nullptr;
+    if (ctx->stage) {
+        (void)hipStreamSynchronize(ctx->stream); /* a call that failed may not have */
+        (void)hipHostFree(ctx->stage);
+    }
+    ctx->stage = nullptr;
+    ctx->stage_bytes = 0;
+    const size_t want = bytes + bytes / 4u < TGX_STAGE_MAX ? bytes + bytes / 4u : TGX_STAGE_MAX;
+    if (hipHostMalloc(&ctx->stage, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->stage = nullptr;
+        return nullptr;
+    }
+    ctx->stage_bytes = want;
+    return ctx->stage;
+}
+
+int tgx_stage_in(tgx_context* ctx, const void* src, size_t bytes, size_t at, size_t all, const void** out)
+{
+    if (char* p = (char*)tgx_stage(ctx, all)) {
+        memcpy(p + at, src, bytes);
+        *out = p + at;
+        return TGX_OK;
+    }
+    int rc;
+    if ((rc = tgx_buffer_reserve(ctx, &ctx->stage_dev, all, "host arrays"))) return rc;
+    *out = (char*)ctx->stage_dev.ptr + at;
+    TGX_HIP_CHECK(ctx, hipMemcpyAsync((void*)*out, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    return TGX_OK;
+}
+
 void tgx_buffer_release(tgx_buffer* b)
 {
     if (b->ptr) (void)hipFree(b->ptr);
@@ -149,11 +183,12 @@ int tgx_destroy(tgx_context* ctx)
                           &ctx->vis_rec_flags, &ctx->vis_global_keys,
                           &ctx->vis_counters, &ctx->vis_tile_count, &ctx->vis_tile_off,
                           &ctx->vis_tile_list, &ctx->vis_cams, &ctx->vis_out, &ctx->vis_stats_dev,
-                          &ctx->frame_acc, &ctx->pick_buf, &ctx->dyn_stage, &ctx->dyn_tmp, &ctx->cl_dirty};
+                          &ctx->frame_acc, &ctx->pick_buf, &ctx->stage_dev, &ctx->dyn_stage, &ctx->dyn_tmp, &ctx->cl_dirty};
     for (tgx_buffer* b : bufs) tgx_buffer_release(b);
     tgx_svo_release(ctx);
     tgx_nrc_release(ctx);
     if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return TGX_OK;
