@@ -554,17 +554,17 @@ typedef struct tgx_tuning {
     uint32_t vis_setup_blocks;    /* visibility: workgroups per camera of the grid-stride cull
                                      and tile-list scatter passes, 64..16384 (2048) */
     uint32_t trace_dda;           /* lane-machine launch: 1 runs a wave's leaf DDA without the
-                                     iteration count (two steps per exit test) when every DDA lane's
+                                     iteration count (six voxels at a time) when every DDA lane's
                                      direction has components of 0 or 2^-100 to 2^26 only, one of
                                      them not 0 (1) */
     uint32_t vis_tile;            /* visibility: tile edge in pixels, 8, 16 or 32 (16); one
                                      workgroup of vis_tile^2 lanes walks each tile's list */
     uint32_t trace_cross;         /* uncounted DDA: 0 walks every voxel; k in 1..64 makes a
                                      wave cross 8^3 bricks without solid voxels in one exact
-                                     step once >= k/64 of its walking lanes are in one (32) */
+                                     step once >= k/64 of its walking lanes are in one (40) */
     uint32_t trace_node;          /* lane-machine launch: moves between child slots a lane outside
                                      the leaves may take per step before the DDA burst, 1..4 (2) */
-    uint32_t trace_burst;         /* uncounted DDA: iterations per burst, even, 2..32 (12) */
+    uint32_t trace_burst;         /* uncounted DDA: voxels per burst, even, 2..32, taken in sixes (18) */
     uint32_t trace_chunk;         /* lane-machine launch: rays a wave takes from the queue per
                                      cursor atomic, kept for its next refills, 0..256 (32); 0
                                      takes only the idle lanes' rays. A wave takes only what it

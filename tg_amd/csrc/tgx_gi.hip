@@ -73,6 +73,14 @@
 
 #define TRACE_BLOCK 1024
 #define DDA_BURST 8u
+/* Voxels that the uncounted DDA takes at a time. Where the walk goes does not
+ * depend on what is solid, so their places come first, then their words are
+ * loaded together, then the first that ends the walk is picked: one wait for
+ * memory instead of one per voxel, 24 slots a voxel instead of 35 with a branch
+ * for the load. What is computed beyond a hit is lost, 2.5 voxels on average.
+ * 1080p frame's trace 2.80 ms with 1 voxel, 2.62 with 2, 2.50 with 4, 2.40 with
+ * 6 and with 8; 100003 rays, where few waves are in flight, 0.36 -> 0.32. */
+#define DDA_AHEAD 6u
 #define TRACE_LDS_LEAVES_MAX 8000u  /* leaf brick masks in LDS (64000 B) */
 
 /* ------------------------------------------------------------------------ */
@@ -175,7 +183,6 @@ struct trace_lane {
     uint32_t vox;          /* x | y << 5 | z << 10 | it << 15 */
     float    tmx, tmy, tmz, tdx, tdy, tdz;
     unsigned long long bm; /* brick mask of the leaf */
-    uint32_t wi, wv;       /* last bit word index and value */
 };
 
 #define ND_X(n)   ((n) & 255u)
@@ -614,7 +621,6 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_br
                 L.tmy = L.dy == 0.0f ? SVO_F32_MAX : ty;
                 L.tmz = L.dz == 0.0f ? SVO_F32_MAX : tz;
                 L.vox = (uint32_t)x0 | ((uint32_t)y0 << 5) | ((uint32_t)z0 << 10);
-                L.wi = 0xFFFFFFFFu;
                 L.node &= ~ND_SETUP;
             }
         }
@@ -636,7 +642,7 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_br
         float tmx = L.tmx, tmy = L.tmy, tmz = L.tmz;
         const float tdx = L.tdx, tdy = L.tdy, tdz = L.tdz;
         const unsigned long long bm = L.bm;
-        uint32_t wi_last = L.wi, wv = L.wv;
+        uint32_t wi_last = 0xFFFFFFFFu, wv = 0u; /* the bit word in hand */
         /* brick skips need every moving axis' t_delta below 2^100 */
         const uint32_t skip_ok = (!kSkip || ((sx == 0 || tdx < 0x1p100f) && (sy == 0 || tdy < 0x1p100f) &&
                                              (sz == 0 || tdz < 0x1p100f))) ? 1u : 0u;
@@ -644,64 +650,75 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_br
          * one axis moves, so no t_max overflows, each step moves a
          * coordinate and the walk leaves the 32^3 block within 94 steps: the
          * iteration cap cannot bind, and a wave whose DDA lanes all have such
-         * rays runs the walk without counting iterations, two per exit test.
+         * rays runs the walk without counting iterations, DDA_AHEAD at a time.
          * A lane's count is then left behind, which only lanes that never
          * take this path read. */
         const bool regular = !(L.node & ND_ODD);
         if (kDda != 0u && !kSkip && __all(regular || !in_dda)) {
             /* the count is not kept on this path (see above) */
             it = 0u;
+            /* voxel in bytes: leaving 0..31 sets a bit of 0xE0E0E0 or above */
+            uint32_t pos = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)z << 16);
+            /* few leaves: 32-bit offsets from a uniform base */
+            const uint32_t leaf_off = 4u * TGX_SVO_BLOCK_WORDS * L.leaf;
+            const uint32_t ix = L.dx > 0.0f ? 1u : ~0u, iy = L.dy > 0.0f ? 0x100u : 0u - 0x100u,
+                           iz = L.dz > 0.0f ? 0x10000u : 0u - 0x10000u;
 #pragma unroll 1
-            for (uint32_t k = 0; k < burst; k += 2) {
+            for (uint32_t k = 0; k < burst; k += DDA_AHEAD) {
                 if constexpr (kDda == 2u) {
                     /* once at least cross/64 of the wave's walking lanes
                      * are in bricks without solid voxels, those lanes cross
-                     * their bricks (brick_cross) before the two steps */
-                    const uint32_t b = ((uint32_t)x >> 3) | (((uint32_t)y >> 3) << 2) | (((uint32_t)z >> 3) << 4);
+                     * their bricks (brick_cross) before the next steps */
+                    const uint32_t b = ((pos >> 3) & 3u) | ((pos >> 9) & 12u) | ((pos >> 15) & 48u);
                     const uint32_t emp = live & ((uint32_t)(bm >> b) ^ 1u) & 1u;
                     const uint32_t n_emp = (uint32_t)__popcll(__ballot(emp != 0u));
                     const uint32_t n_live = (uint32_t)__popcll(__ballot(live != 0u));
                     if (64u * n_emp >= cross * n_live && n_emp != 0u) {
-                        if (emp && brick_cross(x, y, z, tmx, tmy, tmz, tdx, tdy, tdz, sx, sy, sz)) {
-                            const uint32_t outside =
-                                (((uint32_t)x | (uint32_t)y | (uint32_t)z) >> 5) != 0u ? 1u : 0u;
-                            leave_i |= outside;
-                            live &= outside ^ 1u;
+                        if (emp) {
+                            int cx = (int)(pos & 31u), cy = (int)((pos >> 8) & 31u), cz = (int)(pos >> 16);
+                            (void)brick_cross(cx, cy, cz, tmx, tmy, tmz, tdx, tdy, tdz, sx, sy, sz);
+                            /* a coordinate that left is -1 or 32 */
+                            pos = ((uint32_t)cx & 255u) | (((uint32_t)cy & 255u) << 8) | (((uint32_t)cz & 255u) << 16);
                         }
                     }
                 }
+                if (live) {
+                    /* The next DDA_AHEAD voxels, as if none were solid, and
+                     * their words; the walk then ends at the first that is
+                     * solid or outside. */
+                    uint32_t v[DDA_AHEAD], w[DDA_AHEAD];
 #pragma unroll
-                for (uint32_t u = 0; u < 2u; u++) {
-                    const uint32_t b = ((uint32_t)x >> 3) | (((uint32_t)y >> 3) << 2) | (((uint32_t)z >> 3) << 4);
-                    const uint32_t inb = live & (uint32_t)(bm >> b);
-                    const uint32_t wi = 32u * (uint32_t)z + (uint32_t)y;
-                    if ((inb & 1u) && wi != wi_last) { wi_last = wi; wv = grid[wi]; }
-                    const uint32_t h = inb & (wv >> (uint32_t)x) & 1u;
-                    const float m = fminf(fminf(tmx, tmy), tmz);
-                    const uint32_t sz_ = tmz == m ? 1u : 0u;
-                    const uint32_t sy_ = (tmy == m ? 1u : 0u) & (sz_ ^ 1u);
-                    const uint32_t sx_ = (sz_ | sy_) ^ 1u;
-                    const uint32_t move = live & (h ^ 1u);
-                    const uint32_t mx = move & sx_, my = move & sy_, mz = move & sz_;
-                    /* t_max += t_delta on the stepping axis as fma(1, td, t)
-                     * (the same rounded sum) and fma(0, td, t) elsewhere (t
-                     * itself, or +0 for a t of -0, which compares and adds
-                     * alike) */
-                    tmx = fmaf((float)mx, tdx, tmx);
-                    tmy = fmaf((float)my, tdy, tmy);
-                    tmz = fmaf((float)mz, tdz, tmz);
-                    /* 24-bit multiply-adds (mx..mz are 0 or 1) */
-                    x = x + __mul24((int)mx, sx);
-                    y = y + __mul24((int)my, sy);
-                    z = z + __mul24((int)mz, sz);
-                    const uint32_t outside = (((uint32_t)x | (uint32_t)y | (uint32_t)z) >> 5) != 0u ? 1u : 0u;
-                    const uint32_t lv = move & outside;
-                    hit_i |= h;
-                    leave_i |= lv;
-                    live &= (h | lv) ^ 1u;
+                    for (uint32_t u = 0; u < DDA_AHEAD; u++) {
+                        v[u] = pos;
+                        const uint32_t row = 32u * ((pos >> 16) & 31u) + ((pos >> 8) & 31u);
+                        if constexpr (kLds)
+                            w[u] = *(const uint32_t*)((const char*)P.leaf_bits + (uint32_t)(leaf_off + 4u * row));
+                        else
+                            w[u] = grid[row];
+                        const float m = fminf(fminf(tmx, tmy), tmz);
+                        const bool ez = tmz == m, ey = tmy == m;
+                        pos += ez ? iz : (ey ? iy : ix);
+                        tmx = ez || ey ? tmx : tmx + tdx;
+                        tmy = ey && !ez ? tmy + tdy : tmy;
+                        tmz = ez ? tmz + tdz : tmz;
+                    }
+                    if (pos & 0xFFE0E0E0u) live = 0u;
+#pragma unroll
+                    for (uint32_t u = DDA_AHEAD; u-- > 0u;) {
+                        const bool out = (v[u] & 0xFFE0E0E0u) != 0u, solid = (w[u] >> (v[u] & 31u)) & 1u;
+                        if (out || solid) {
+                            pos = v[u];
+                            live = 0u;
+                        }
+                    }
                 }
                 if (!__any(live != 0u)) break;
             }
+            const uint32_t out = (pos & 0xFFE0E0E0u) != 0u ? 1u : 0u;
+            const uint32_t ended = in_dda && !live ? 1u : 0u;
+            hit_i = ended & (out ^ 1u);
+            leave_i = ended & out;
+            x = (int)(pos & 31u); y = (int)((pos >> 8) & 31u); z = (int)((pos >> 16) & 31u);
         } else
 #pragma unroll 1
         for (uint32_t k = 0; k < DDA_BURST; k++) {
@@ -746,7 +763,6 @@ __device__ static inline bool lane_step(const trace_params& P, const uint2* s_br
             if (!__any(live != 0u)) break;
         }
         L.tmx = tmx; L.tmy = tmy; L.tmz = tmz;
-        L.wi = wi_last; L.wv = wv;
         hit = hit_i != 0u;
         leave = leave_i != 0u;
         if (in_dda && !hit && !leave) L.vox = (uint32_t)x | ((uint32_t)y << 5) | ((uint32_t)z << 10) | (it << 15);
@@ -1185,9 +1201,8 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
             active = (flags & 1u) != 0u;
             pending = (flags & 2u) != 0u;
             ox = f.x; oy = f.y; oz = f.z; sid = __float_as_uint(f.w);
-            /* the leaf's brick mask and an empty bit-word cache */
+            /* the leaf's brick mask */
             if (active && (L.node & ND_DDA)) L.bm = bricks_at<kLds>(P.bricks, s_bricks, L.leaf);
-            L.wi = 0xFFFFFFFFu;
         } else {
             active = false;
             pending = false;
