@@ -110,37 +110,35 @@ __device__ static inline float feat_tail(const gi_surf_rec& r, uint32_t f)
          : f == 76u ? r.albedo[1] : f == 77u ? r.albedo[2] : f == 78u ? 1.0f : 0.0f;
 }
 
-/* B fragment of the input features for K step s (features 32 s + 8 g + j).
- * sin(2^k pi x) = sin(2 pi frac(2^(k-1) x)); v_sin / v_cos take turns. */
-__device__ static inline bf16x8 input_frag(const gi_surf_rec& r, float px, float py, float pz, uint32_t s, uint32_t g)
-{
-    bf16x8 v;
-#pragma unroll
-    for (uint32_t jj = 0; jj < 8u; jj += 2u) {
-        const uint32_t f = 32u * s + 8u * g + jj;
-        float a, b;
-        if (f < 72u) {
-            const uint32_t ax = f / 24u, k = (f % 24u) / 2u;
-            const float ph = ax == 0u ? px : (ax == 1u ? py : pz);
-            const float x = ldexpf(ph, (int)k - 1);
-            const float t = x - floorf(x);
-            a = __builtin_amdgcn_sinf(t);
-            b = __builtin_amdgcn_cosf(t);
-        } else {
-            a = feat_tail(r, f);
-            b = feat_tail(r, f + 1u);
-        }
-        v[jj] = (__bf16)a;
-        v[jj + 1] = (__bf16)b;
-    }
-    return v;
-}
-
+/* B fragments of the input features, feature 32 s + 8 g + j in element j of
+ * K step s: features 24 axis + 2 k and the next are sine and cosine of 2^k pi
+ * x, as v_sin / v_cos of frac(2^(k-1) x) turns; 72 on see feat_tail. A lane's
+ * eight features of a K step are of one axis and have four consecutive k, from
+ * 4 ((4 s + g) mod 3), so one coordinate times one power of two gives them by
+ * doubling (all exact). Features and exponents per pair, by divisions of a
+ * lane's f, took half of the encoding. */
 __device__ static inline void encode(const gi_surf_rec& r, const nrc_enc& e, uint32_t g, bf16x8 x[3])
 {
     const float px = (r.p[0] - e.ox) * e.scale, py = (r.p[1] - e.oy) * e.scale, pz = (r.p[2] - e.oz) * e.scale;
 #pragma unroll
-    for (uint32_t s = 0; s < 3u; s++) x[s] = input_frag(r, px, py, pz, s, g);
+    for (uint32_t s = 0; s < 3u; s++) {
+        const uint32_t o = 4u * s + g;                     /* feature octet, 0..11; 9 on are no sines */
+        const float ph = o < 3u ? px : (o < 6u ? py : pz); /* octets 0..2, 3..5, 6..8 */
+        const uint32_t q = o % 3u;
+        const float y = ph * (q == 0u ? 0.5f : (q == 1u ? 8.0f : 128.0f));
+#pragma unroll
+        for (uint32_t jj = 0; jj < 8u; jj += 2u) {
+            const float v = y * (float)(1u << (jj / 2u));
+            const float t = v - floorf(v);
+            float a = __builtin_amdgcn_sinf(t), b = __builtin_amdgcn_cosf(t);
+            if (s == 2u) {
+                a = o < 9u ? a : (o == 9u ? feat_tail(r, 72u + jj) : 0.0f);
+                b = o < 9u ? b : (o == 9u ? feat_tail(r, 73u + jj) : 0.0f);
+            }
+            x[s][jj] = (__bf16)a;
+            x[s][jj + 1u] = (__bf16)b;
+        }
+    }
 }
 
 __device__ static inline void relu_pack(const f32x4 acc[4], bf16x8 out[2])
@@ -149,8 +147,9 @@ __device__ static inline void relu_pack(const f32x4 acc[4], bf16x8 out[2])
     for (uint32_t s = 0; s < 2u; s++)
 #pragma unroll
         for (uint32_t j = 0; j < 8u; j++) {
-            const float v = acc[2u * s + j / 4u][j & 3u];
-            out[s][j] = (__bf16)(v > 0.0f ? v : 0.0f);
+            /* v > 0 ? v : 0 in one operation, 0 for NaN as well; beyond the
+             * largest float only infinity, which both round to */
+            out[s][j] = (__bf16)__builtin_amdgcn_fmed3f(acc[2u * s + j / 4u][j & 3u], 0.0f, 3.402823466e+38f);
         }
 }
 
@@ -363,6 +362,8 @@ __global__ __launch_bounds__(NRC_BLOCK) __attribute__((amdgpu_waves_per_eu(1, 2)
 /* One 16 x 16 tile of dW_L = A_L^T dZ_(L+1) over `per` consecutive
  * chunks of NRC_CHUNK samples per wave (in sample order); partial[group]
  * [param] for the n_chunks groups. */
+#define WGRAD_AHEAD 8u
+static_assert(NRC_CHUNK % (32u * WGRAD_AHEAD) == 0u, "K steps per group of loads");
 __global__ __launch_bounds__(NRC_BLOCK) void nrc_wgrad_k(const __bf16* __restrict__ train, uint32_t Bc,
                                                          uint32_t n_chunks, uint32_t per, float* __restrict__ partial)
 {
@@ -378,15 +379,26 @@ __global__ __launch_bounds__(NRC_BLOCK) void nrc_wgrad_k(const __bf16* __restric
     const uint32_t brow = (L == 4u ? R_DZ5 : R_DZ1 + 64u * L) + 16u * to + n;
     const bool bvalid = L != 4u || n < 3u;
     const __bf16* ap = train + (size_t)arow * Bc + (size_t)chunk * per * NRC_CHUNK + 8u * g;
-    const __bf16* bp = train + (size_t)brow * Bc + (size_t)chunk * per * NRC_CHUNK + 8u * g;
+    /* rows past the outputs read the inputs' and count as zero: no branch
+     * around a load */
+    const __bf16* bp = bvalid ? train + (size_t)brow * Bc + (size_t)chunk * per * NRC_CHUNK + 8u * g : ap;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     bf16x8 zero;
 #pragma unroll
     for (uint32_t j = 0; j < 8u; j++) zero[j] = (__bf16)0.0f;
-    for (uint32_t k = 0; k < per * NRC_CHUNK; k += 32u) {
-        const bf16x8 a = *(const bf16x8*)(ap + k);
-        const bf16x8 bq = bvalid ? *(const bf16x8*)(bp + k) : zero;
-        acc = mfma16(a, bq, acc);
+    /* WGRAD_AHEAD K steps' operands are loaded together (NRC_CHUNK is a
+     * multiple of 32 WGRAD_AHEAD): the products stay one chain, the waits for
+     * memory do not. 10000 samples 13.5 -> 11.7 us a step; larger batches, 18 us
+     * at 16384, stay as they were. */
+    for (uint32_t k = 0; k < per * NRC_CHUNK; k += 32u * WGRAD_AHEAD) {
+        bf16x8 a[WGRAD_AHEAD], bq[WGRAD_AHEAD];
+#pragma unroll
+        for (uint32_t u = 0; u < WGRAD_AHEAD; u++) {
+            a[u] = *(const bf16x8*)(ap + k + 32u * u);
+            bq[u] = *(const bf16x8*)(bp + k + 32u * u);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < WGRAD_AHEAD; u++) acc = mfma16(a[u], bvalid ? bq[u] : zero, acc);
     }
     const uint32_t out_dim = L == 4u ? 3u : 64u;
     const uint32_t off = L == 0u ? P_W0 : (L == 4u ? P_W4 : P_W1 + 4096u * (L - 1u));
@@ -436,6 +448,7 @@ __global__ void nrc_pack_k(const float* __restrict__ master, __bf16* __restrict_
     if (b >= 0 && bwd) bwd[b] = v;
 }
 
+#define NRC_ADAM_THREADS (256u + 2u * 64u)
 struct nrc_adam_args {
     float lr, beta1, beta2, eps;
 };
@@ -492,7 +505,7 @@ __global__ void nrc_tick_k(uint32_t* counter) { *counter += 1u; }
  * with loss_out, adds the batch's per-sample squared errors to *loss_out in
  * a fixed order. dev[NRC_DEV_DONE] counts finished blocks; it is 0 between
  * launches. */
-__global__ __launch_bounds__(256) void nrc_adam_k(const float* __restrict__ partial, uint32_t n_chunks, nrc_adam_args a,
+__global__ __launch_bounds__(NRC_ADAM_THREADS) void nrc_adam_k(const float* __restrict__ partial, uint32_t n_chunks, nrc_adam_args a,
                                                   uint32_t* __restrict__ dev, float* __restrict__ master,
                                                   float* __restrict__ m, float* __restrict__ v, float* __restrict__ grad,
                                                   __bf16* __restrict__ fwd, __bf16* __restrict__ bwd,
@@ -503,19 +516,31 @@ __global__ __launch_bounds__(256) void nrc_adam_k(const float* __restrict__ part
     __shared__ float s[256];
     __shared__ uint32_t last;
     __shared__ float bc[2];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     const uint32_t t_u = dev[NRC_DEV_STEP] + 1u;
-    if (threadIdx.x == 0) {
-        /* bias corrections, once per block */
-        const double t = (double)t_u;
-        bc[0] = (float)(1.0 / (1.0 - pow((double)a.beta1, t)));
-        bc[1] = (float)(1.0 / (1.0 - pow((double)a.beta2, t)));
+    /* Bias corrections, once per block, each by a wave of its own behind the
+     * 256 parameters' while those load; the partial sums' loads are issued
+     * sixteen together and added in order. One wave's two powers first and then
+     * a load at a time took 14.7 us a step, this 10.7. */
+    float gsum = 0.0f;
+    if (threadIdx.x >= 256u) {
+        if ((threadIdx.x & 63u) == 0u) {
+            const uint32_t w = (threadIdx.x - 256u) >> 6;
+            bc[w] = (float)(1.0 / (1.0 - pow((double)(w ? a.beta2 : a.beta1), (double)t_u)));
+        }
+    } else if (i < NRC_N) {
+        for (uint32_t c0 = 0; c0 < n_chunks; c0 += 16u) {
+            float p[16];
+#pragma unroll
+            for (uint32_t c = 0; c < 16u; c++) p[c] = c0 + c < n_chunks ? partial[(size_t)(c0 + c) * NRC_N + i] : 0.0f;
+#pragma unroll
+            for (uint32_t c = 0; c < 16u; c++)
+                if (c0 + c < n_chunks) gsum += p[c];
+        }
     }
     __syncthreads();
-    if (i < NRC_N) {
+    if (threadIdx.x < 256u && i < NRC_N) {
         const float inv_bc1 = bc[0], inv_bc2 = bc[1];
-        float gsum = 0.0f;
-        for (uint32_t c = 0; c < n_chunks; c++) gsum += partial[(size_t)c * NRC_N + i];
         grad[i] = gsum;
         const float mi = a.beta1 * m[i] + (1.0f - a.beta1) * gsum;
         const float vi = a.beta2 * v[i] + (1.0f - a.beta2) * gsum * gsum;
@@ -538,9 +563,11 @@ __global__ __launch_bounds__(256) void nrc_adam_k(const float* __restrict__ part
     /* the batch's loss: every block sums a strided slice in a fixed order,
      * the last block adds the block sums in block order */
     if (loss_out) {
-        float acc = 0.0f;
-        for (uint32_t k = i; k < n_loss; k += gridDim.x * blockDim.x) acc += loss[k];
-        s[threadIdx.x] = acc;
+        if (threadIdx.x < 256u) {
+            float acc = 0.0f;
+            for (uint32_t k = i; k < n_loss; k += gridDim.x * 256u) acc += loss[k];
+            s[threadIdx.x] = acc;
+        }
         __syncthreads();
         for (uint32_t w = 128u; w > 0u; w >>= 1) {
             if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
@@ -558,7 +585,8 @@ __global__ __launch_bounds__(256) void nrc_adam_k(const float* __restrict__ part
     if (loss_out) {
         /* the block sums (gridDim.x <= 256) in a fixed tree */
         __threadfence();
-        s[threadIdx.x] = threadIdx.x < gridDim.x ? ((volatile const float*)loss_part)[threadIdx.x] : 0.0f;
+        if (threadIdx.x < 256u)
+            s[threadIdx.x] = threadIdx.x < gridDim.x ? ((volatile const float*)loss_part)[threadIdx.x] : 0.0f;
         __syncthreads();
         for (uint32_t w = 128u; w > 0u; w >>= 1) {
             if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
@@ -573,9 +601,11 @@ __global__ __launch_bounds__(256) void nrc_adam_k(const float* __restrict__ part
 }
 
 /* Inference over list entries b < *count (persistent waves, 16 samples a
- * tile, each wave's forward fragments in its registers, two waves per SIMD;
- * the next tile's surface record is loaded while the current one is
- * evaluated). With cells, an entry whose cell is
+ * tile, each wave's forward fragments in its registers, two waves per SIMD).
+ * With two waves a SIMD hides no load, so none is waited for where it is issued:
+ * list entries come two tiles ahead, surface records one, the cell before its
+ * tile is evaluated. 1080p (72 k tiles) 101 us with the entry, its record and
+ * the cell one after the other, 75 us so (with the shorter encoding and relu). With cells, an entry whose cell is
  * unreliable gets fallback flag 1 instead of an output: fewer than min_n
  * samples, or a bias^2 sum above w_ref times the targets' t^2 sum plus
  * w_var times their variance sum. */
@@ -593,20 +623,24 @@ __global__ __launch_bounds__(NRC_BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2)
     const uint32_t n_tiles = (count + 15u) / 16u;
     const uint32_t waves = gridDim.x * (NRC_BLOCK / 64u);
     uint32_t tile = (blockIdx.x * NRC_BLOCK + threadIdx.x) >> 6;
+    const uint32_t step = waves * 16u;
+    /* the entry of this tile, the next one and, loaded while the tile is
+     * evaluated, the one after it; n_entry past the end */
+    auto entry = [&](uint32_t b) { return b < count ? (list ? list[b] : b) : 0xFFFFFFFFu; };
+    uint32_t b = tile * 16u + n;
+    uint32_t e_now = entry(b), e_next = entry(b + step);
     gi_surf_rec rn = {};
-    {
-        const uint32_t b = tile * 16u + n;
-        if (tile < n_tiles && b < count) rn = surf[list ? list[b] : b];
-    }
-    for (; tile < n_tiles; tile += waves) {
-        const uint32_t b = tile * 16u + n;
+    if (e_now != 0xFFFFFFFFu) rn = surf[e_now];
+    for (; tile < n_tiles; tile += waves, b += step) {
         const bool valid = b < count;
         const gi_surf_rec r = rn;
-        {
-            const uint32_t t2 = tile + waves, b2 = t2 * 16u + n;
-            rn = gi_surf_rec{};
-            if (t2 < n_tiles && b2 < count) rn = surf[list ? list[b2] : b2];
-        }
+        const uint32_t pix = e_now;
+        e_now = e_next;
+        e_next = entry(b + 2u * step);
+        rn = gi_surf_rec{};
+        if (e_now != 0xFFFFFFFFu) rn = surf[e_now];
+        nrc_cell c = {};
+        if (cells && valid && g == 0u) c = cells[cell_of(r, cell_shift)];
         bf16x8 x[3];
         encode(r, enc, g, x);
         const f32x4 y = infer_tile(w, x);
@@ -615,12 +649,10 @@ __global__ __launch_bounds__(NRC_BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2)
         if (out_entry) { out_entry[3ull * b] = e0; out_entry[3ull * b + 1] = e1; out_entry[3ull * b + 2] = e2; }
         bool fb = false;
         if (cells) {
-            const nrc_cell c = cells[cell_of(r, cell_shift)];
             fb = c.n < min_n || (float)c.err > w_ref * (float)c.ref + w_var * (float)c.var;
             fb_flag[b] = fb ? 1u : 0u;
         }
         if (fb) continue;
-        const uint32_t pix = list ? list[b] : b;
         if (irradiance) { irradiance[3ull * pix] = e0; irradiance[3ull * pix + 1] = e1; irradiance[3ull * pix + 2] = e2; }
         if (radiance) {
             radiance[3ull * pix] = r.albedo[0] * e0;
@@ -794,7 +826,7 @@ int train_step(tgx_context* ctx, const gi_surf_rec* surf, const uint32_t* list, 
     uint32_t* dev = (uint32_t*)ctx->nrc_dev.ptr;
     {
         tgx_launch_scope s(ctx, "nrc_adam_k");
-        hipLaunchKernelGGL(nrc_adam_k, dim3(nrc_blocks(NRC_N, 256)), dim3(256), 0, ctx->stream,
+        hipLaunchKernelGGL(nrc_adam_k, dim3(nrc_blocks(NRC_N, 256)), dim3(NRC_ADAM_THREADS), 0, ctx->stream,
                            (const float*)ctx->nrc_partials.ptr, n_chunks, a, dev, (float*)ctx->nrc_master.ptr,
                            (float*)ctx->nrc_m.ptr, (float*)ctx->nrc_v.ptr, (float*)ctx->nrc_grad.ptr,
                            (__bf16*)ctx->nrc_fwd.ptr, (__bf16*)ctx->nrc_bwd.ptr, (const float*)ctx->nrc_loss.ptr, Bc,
