@@ -842,34 +842,46 @@ struct trace_fuse {
  * (flag bit 0) are added to *hit_counter when it is not null. Fused GI
  * (kFused true): see trace_fuse; out and hit_counter are not used. `cursor`
  * holds TRACE_SEGS segment cursors 16 words apart, 0 at launch. */
+struct trace_args {
+    trace_params    P;
+    const svo_ray*  rays;
+    const uint32_t* n_rays;
+    uint32_t*       cursor;
+    svo_res*        out;
+    uint32_t*       hit_counter;
+    float           maxd;
+    uint32_t        refill, vote, cross, node_iters, burst, chunk, small_rays, small_blocks;
+    trace_fuse      F;
+};
+
+/* The arguments are read from their segment anew in every step (the empty asm
+ * keeps loads from being moved out of the loop): held in scalar registers they
+ * and the lane masks did not fit, and the spilled ones came back by v_readlane,
+ * 40 of the 200 vector slots of a move. SPILLS */
 template <bool kLds, bool kFused, uint32_t kDda>
-__global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void gi_trace_k(trace_params P, const svo_ray* __restrict__ rays,
-                                                          const uint32_t* __restrict__ n_rays_ptr, float maxd,
-                                                          uint32_t* __restrict__ cursor, svo_res* __restrict__ out,
-                                                          uint32_t* __restrict__ hit_counter, uint32_t refill,
-                                                          uint32_t vote, uint32_t cross, uint32_t node_iters,
-                                                          uint32_t burst, uint32_t chunk, uint32_t small_rays,
-                                                          uint32_t small_blocks, const trace_fuse F)
+__global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void gi_trace_k(const trace_args)
 {
+    typedef __attribute__((address_space(4))) const trace_args* arg_ptr;
+    arg_ptr A = (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
     extern __shared__ uint2 s_bricks[];
     /* a queue of fewer than small_rays rays is traced by the first
      * small_blocks workgroups (one per CU) alone: with few rays per lane the
      * launch is as long as its slowest rays, which run faster with fewer
      * waves per SIMD */
-    const uint32_t n_rays = __builtin_amdgcn_readfirstlane(*n_rays_ptr);
-    const bool small = n_rays < small_rays;
-    if (small && blockIdx.x >= small_blocks) return;
+    const uint32_t n_rays = __builtin_amdgcn_readfirstlane(*A->n_rays);
+    const bool small = n_rays < A->small_rays;
+    if (small && blockIdx.x >= A->small_blocks) return;
     if constexpr (kLds) {
-        const uint2* gb = (const uint2*)P.bricks;
-        for (uint32_t i = threadIdx.x; i < P.n_leaves; i += blockDim.x) s_bricks[i] = gb[i];
+        const uint2* gb = (const uint2*)A->P.bricks;
+        const uint32_t n_leaves = A->P.n_leaves;
+        for (uint32_t i = threadIdx.x; i < n_leaves; i += blockDim.x) s_bricks[i] = gb[i];
         __syncthreads();
     }
     const uint32_t lane = threadIdx.x & 63u;
     /* fused GI: each lane's bounce ray origin and id, behind the nodes; the
      * wave's part of the stash is a uniform base indexed by lane */
-    float4* s_ray = (float4*)(s_bricks + (kLds ? ((P.n_leaves + 1u) & ~1u) : 0u)) +
+    float4* s_ray = (float4*)(s_bricks + (kLds ? ((A->P.n_leaves + 1u) & ~1u) : 0u)) +
                     __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
-    const float half = P.half;
     trace_lane L = {};
     uint32_t slot = 0;
     /* the wave's bounce hits (plain trace) */
@@ -884,7 +896,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
      * atomic) a wave takes only what it hands out, so no wave holds back
      * rays that idle waves could trace. */
     uint32_t q_next = 0, q_end = 0, seen = 0;
-    const uint32_t n_waves = (small && small_blocks < gridDim.x ? small_blocks : gridDim.x) * (TRACE_BLOCK / 64u);
+    const uint32_t n_waves = (small && A->small_blocks < gridDim.x ? A->small_blocks : gridDim.x) * (TRACE_BLOCK / 64u);
     /* The queue is split into TRACE_SEGS segments with a cursor each (16
      * words apart). A wave starts in segment blockIdx.x mod TRACE_SEGS
      * (workgroups are dealt to the XCDs in turn, so an XCD's waves share a
@@ -896,6 +908,10 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
     seen = seg_start(seg);
     const uint32_t seg_waves = (n_waves + TRACE_SEGS - 1u) / TRACE_SEGS;
     do {
+        asm volatile("" : "+s"(A));
+        const trace_params& P = *(const trace_params*)&A->P;
+        const float half = P.half, maxd = A->maxd;
+        const uint32_t refill = A->refill;
         /* the queue state is the wave's: kept in scalar registers */
         q_next = __builtin_amdgcn_readfirstlane(q_next);
         q_end = __builtin_amdgcn_readfirstlane(q_end);
@@ -912,12 +928,12 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
             uint32_t nb = 0, nend = 0;
             if (avail < want && !drained) {
                 const uint32_t seg_lo = seg_start(seg), seg_hi = seg_start(seg + 1u);
-                const uint32_t need = want - avail;
+                const uint32_t need = want - avail, chunk = A->chunk;
                 const bool tail = (uint64_t)(seg_hi - (seen < seg_hi ? seen : seg_hi)) <
                                   2ull * seg_waves * chunk;
                 const uint32_t take = tail || chunk < need ? need : chunk;
                 uint32_t base = 0;
-                if (lane == 0) base = atomicAdd(cursor + 16u * seg, take);
+                if (lane == 0) base = atomicAdd(A->cursor + 16u * seg, take);
                 /* the whole wave runs this block, so lane 0 is the first active */
                 base = __builtin_amdgcn_readfirstlane(base) + seg_lo;
                 seen = base;
@@ -938,7 +954,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
                 const uint32_t r = rk < avail ? q_next + rk : nb + (rk - avail);
                 if (rk < avail || rk - avail < nend - nb) {
                     slot = r;
-                    const svo_ray q = rays[r];
+                    const svo_ray q = A->rays[r];
                     L.px = q.ox; L.py = q.oy; L.pz = q.oz;
                     L.dx = q.dx; L.dy = q.dy; L.dz = q.dz;
                     if constexpr (kFused) s_ray[lane] = make_float4(q.ox, q.oy, q.oz, __uint_as_float(q.id));
@@ -957,12 +973,13 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
             pending = false;
             /* a shadow ray's step lengths are the sun's, set with its ray */
             active = lane_init_self(P, half, L, kFused && (slot & TRACE_SHADOW));
-            if (!kFused && !active) out[slot] = res_miss(0u);
+            if (!kFused && !active) A->out[slot] = res_miss(0u);
         }
         /* phase vote (tuning): a wave runs only DDA bursts in an iteration
          * once at least vote/64 of its active lanes are in a leaf DDA, and
          * only node steps otherwise */
         bool allow_node = true, allow_dda = true;
+        const uint32_t vote = A->vote;
         if (vote) {
             const uint32_t n_dda = (uint32_t)__popcll(__ballot(active && (L.node & ND_DDA)));
             const uint32_t n_all = (uint32_t)__popcll(__ballot(active));
@@ -974,19 +991,19 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
          * 1 bounce hit, 2 shadow ray started, 4 shadow hit; << 3 for the
          * second list */
         uint32_t ev = 0u;
-        if (lane_step<kLds, false, kDda>(P, s_bricks, half, maxd, L, res, active, allow_node, allow_dda, cross,
-                                         node_iters, burst) &&
+        if (lane_step<kLds, false, kDda>(P, s_bricks, half, maxd, L, res, active, allow_node, allow_dda, A->cross,
+                                         A->node_iters, A->burst) &&
             active) {
             active = false;
             if constexpr (!kFused) {
-                out[slot] = res;
+                A->out[slot] = res;
                 ev = res.flags & 1u;
             } else if (slot & TRACE_SHADOW) {
                 const uint32_t id = slot & ~TRACE_SHADOW;
                 if (res.flags & 1u) {
                     /* occluded: the sample contributes nothing (weight 0) */
-                    F.contrib[3ull * id] = 0.0f;
-                    F.contrib[3ull * id + 2] = __uint_as_float(SAMPLE_HIT | SAMPLE_LIT | SAMPLE_OCC);
+                    A->F.contrib[3ull * id] = 0.0f;
+                    A->F.contrib[3ull * id + 2] = __uint_as_float(SAMPLE_HIT | SAMPLE_LIT | SAMPLE_OCC);
                 }
             } else {
                 /* the ray's origin and id from LDS; its direction is L.dx..dz */
@@ -995,7 +1012,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
                 /* cosine of the hit face with the sun (gi_shade_k) */
                 const uint32_t ax = (res.flags >> 2) & 3u;
                 const float sign = (res.flags & 16u) ? 1.0f : -1.0f;
-                const float sc = ax == 0u ? F.sun0 : (ax == 1u ? F.sun1 : F.sun2);
+                const float sc = ax == 0u ? A->F.sun0 : (ax == 1u ? A->F.sun1 : A->F.sun2);
                 const float cosv = ((res.flags & 1u) && !(res.distance < 0.0f)) ? sign * sc : 0.0f;
                 if (cosv > 0.0f) {
                     /* the shadow ray goes into the lane's own (dead) ray
@@ -1006,17 +1023,17 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
                     L.pz = o.z + L.dz * res.distance;
                     const float off = sign * GI_SHADOW_OFFSET;
                     if (ax == 0u) L.px = L.px + off; else if (ax == 1u) L.py = L.py + off; else L.pz = L.pz + off;
-                    L.dx = F.sun0; L.dy = F.sun1; L.dz = F.sun2;
-                    L.tdx = F.sun_td0; L.tdy = F.sun_td1; L.tdz = F.sun_td2;
+                    L.dx = A->F.sun0; L.dy = A->F.sun1; L.dz = A->F.sun2;
+                    L.tdx = A->F.sun_td0; L.tdy = A->F.sun_td1; L.tdz = A->F.sun_td2;
                     /* the sample record: weight, hit node and voxel (the
                      * albedo is applied when the samples are resolved) */
-                    const float wgt = cosv * F.sun_radiance * GI_INV_PI;
-                    float* c = F.contrib + 3ull * id;
+                    const float wgt = cosv * A->F.sun_radiance * GI_INV_PI;
+                    float* c = A->F.contrib + 3ull * id;
                     c[0] = wgt; c[1] = __uint_as_float(res.node); c[2] = __uint_as_float(res.voxel | SAMPLE_HIT | SAMPLE_LIT);
                     slot = id | TRACE_SHADOW;
                     pending = true;
                 } else if (res.flags & 1u) {
-                    F.contrib[3ull * id + 2] = __uint_as_float(SAMPLE_HIT);
+                    A->F.contrib[3ull * id + 2] = __uint_as_float(SAMPLE_HIT);
                 }
             }
         }
@@ -1027,7 +1044,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
          * divergent and keeps the queue state in vector registers */
     } while ((__ballot(active || pending) | (seg_left == 0u && q_next == q_end ? 0ull : 1ull)) != 0ull);
     if constexpr (!kFused) {
-        if (lane == 0 && hit_counter && n_hit0) atomicAdd(hit_counter, n_hit0);
+        if (lane == 0 && A->hit_counter && n_hit0) atomicAdd(A->hit_counter, n_hit0);
     }
 }
 
@@ -1834,9 +1851,10 @@ static int launch_trace(tgx_context* ctx, const svo_ray* rays, const uint32_t* n
          * frame clears them on every replay) */
         uint32_t* seg_cursors = (uint32_t*)ctx->gi_counts.ptr + GI_CNT_SEG;
         hipLaunchKernelGGL(gi_fill_k, dim3(1), dim3(128), 0, ctx->stream, seg_cursors, 16ull * TRACE_SEGS, 0u);
-        hipLaunchKernelGGL(kernel, grid, dim3(TRACE_BLOCK), shmem, ctx->stream, P, rays, n_dev, maxd, seg_cursors, out,
-                           hit_counter, refill, vote, ctx->tuning.trace_cross, ctx->tuning.trace_node,
-                           ctx->tuning.trace_burst, ctx->tuning.trace_chunk, small_rays, (uint32_t)cus, F);
+        const trace_args args = {P, rays, n_dev, seg_cursors, out, hit_counter, maxd, refill, vote, ctx->tuning.trace_cross,
+                                 ctx->tuning.trace_node, ctx->tuning.trace_burst, ctx->tuning.trace_chunk, small_rays,
+                                 (uint32_t)cus, F};
+        hipLaunchKernelGGL(kernel, grid, dim3(TRACE_BLOCK), shmem, ctx->stream, args);
     }
     TGX_LAUNCH_CHECK(ctx, "gi_trace_k");
     return TGX_OK;
