@@ -857,7 +857,7 @@ struct trace_args {
 /* The arguments are read from their segment anew in every step (the empty asm
  * keeps loads from being moved out of the loop): held in scalar registers they
  * and the lane masks did not fit, and the spilled ones came back by v_readlane,
- * 40 of the 200 vector slots of a move. SPILLS */
+ * 40 of the 200 vector slots of a move. */
 template <bool kLds, bool kFused, uint32_t kDda>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void gi_trace_k(const trace_args)
 {

@@ -964,6 +964,26 @@ __device__ static inline void lds_bitonic_sort(uint64_t* keys, uint32_t n2)
     }
 }
 
+/* Sorts keys[0..n), all different, by counting for each how many are smaller:
+ * two barriers and n broadcast reads, where the bitonic network of 64 keys has
+ * 21 barriers. n <= blockDim.x. Traversal at 256x256 16.8 -> 14.5 us, at 1080p
+ * 73 -> 71; up to 32 keys only 72, up to 256 the same as up to 128, where the
+ * reads come near the network's time. */
+#define VIS_RANK_MAX 128u
+__device__ static inline void lds_rank_sort(uint64_t* keys, uint32_t n)
+{
+    const uint32_t t = threadIdx.x;
+    uint64_t mine = 0ull;
+    uint32_t rank = 0u;
+    if (t < n) {
+        mine = keys[t];
+        for (uint32_t j = 0; j < n; j++) rank += keys[j] < mine ? 1u : 0u;
+    }
+    __syncthreads();
+    if (t < n) keys[rank] = mine;
+    __syncthreads();
+}
+
 /* One workgroup of T x T lanes (T = 1 << kShift) per tile, each wave an
  * 8 x 8 pixel block. The sorted entries are staged VIS_STAGE at a time:
  * the workgroup loads their records, then their clusters' bit words, into
@@ -1034,7 +1054,8 @@ __global__ __launch_bounds__(1u << (2u * kShift)) void vis_traverse(const vis_ca
             keys[j] = kv;
         }
         __syncthreads();
-        lds_bitonic_sort(keys, n2);
+        if (n <= VIS_RANK_MAX && n <= blockDim.x) lds_rank_sort(keys, n);
+        else lds_bitonic_sort(keys, n2);
         for (uint32_t sb = 0; sb < n; sb += VIS_STAGE) {
             const uint32_t ns = min(VIS_STAGE, n - sb);
             for (uint32_t q = threadIdx.x; q < ns * 20u; q += blockDim.x) {
