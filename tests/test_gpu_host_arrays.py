@@ -1,7 +1,7 @@
 """Calls on host arrays pass them through pinned memory that the kernels read,
-256 records a block, and beyond 32 MiB through device memory: odd counts about
-a block's edge, a call after a larger one, and one beyond the bound, whose
-results are those of the same records in small calls, bit for bit."""
+256 records a block, in pieces of 4 MiB: odd counts about a block's edge, a call
+after a larger one, and one of many pieces, whose results are those of the same
+records in small calls, bit for bit."""
 from __future__ import annotations
 
 import numpy as np
@@ -26,12 +26,12 @@ def test_trace_counts(ctx):
         print(f"{n} rays", flush=True)
         o, d = rays_from(rng, max(n, 8), -10, 140, centre=(64.0, 64.0, 64.0))
         assert_same_hits(ctx.svo_trace(o[:n], d[:n], 300.0), ref.trace(o[:n], d[:n], 300.0), f"{n} rays")
-    n = 600_001  # 24 + 40 bytes a ray
+    n = 600_001
     print(f"{n} rays", flush=True)
     o, d = rays_from(rng, n, -10, 140)
     big = ctx.svo_trace(o, d, 300.0)
     for a in (0, 299_999, n - 1000):
-        assert_same_hits(big[a:a + 1000], ctx.svo_trace(o[a:a + 1000], d[a:a + 1000], 300.0), "beyond the bound")
+        assert_same_hits(big[a:a + 1000], ctx.svo_trace(o[a:a + 1000], d[a:a + 1000], 300.0), "in many pieces")
 
 
 def test_cache_counts(ctx):
@@ -54,8 +54,8 @@ def test_cache_counts(ctx):
     first = infer(0, 1)
     before = [step(n) for n in counts]
     ctx.nrc_create(T.nrc_config())
-    print("inference beyond the bound", flush=True)
-    big = infer(0, len(s))  # 36 + 12 bytes a sample
+    print("inference in many pieces", flush=True)
+    big = infer(0, len(s))
     assert np.array_equal(big[:1], first)
     for a, n in ((16, 255), (0, 256), (777, 257), (797_000, 3001)):
         print(f"inference of {n}", flush=True)

@@ -1702,11 +1702,12 @@ __global__ void gi_gather_rays_k(const svo_ray* __restrict__ src, const uint32_t
     if (i < *n_ptr) dst[i] = src[idx[i]];
 }
 
-/* Ray queue of a host call, its counters cleared and the count set (cnt[6]).
- * The arrays are the host's memory, which no cache holds: a block reads its
- * 256 rays' floats once, in order, into LDS. */
+/* Rays id0 .. id0 + n of a host call, its counters cleared and the count of all
+ * set (cnt[6]). The arrays are the host's memory, which no cache holds: a block
+ * reads its 256 rays' floats once, in order, into LDS. */
 __global__ __launch_bounds__(256) void svo_rays_k(const float* __restrict__ origins, const float* __restrict__ dirs,
-                                                  uint32_t n, svo_ray* __restrict__ rays, uint32_t* __restrict__ cnt)
+                                                  uint32_t n, uint32_t id0, uint32_t n_all, svo_ray* __restrict__ rays,
+                                                  uint32_t* __restrict__ cnt)
 {
     __shared__ float s[2][768];
     const uint32_t first = blockIdx.x * 256u, t = threadIdx.x;
@@ -1716,15 +1717,16 @@ __global__ __launch_bounds__(256) void svo_rays_k(const float* __restrict__ orig
             s[0][k] = origins[base + k];
             s[1][k] = dirs[base + k];
         }
-    if (blockIdx.x == 0u && t < GI_N_COUNTERS) cnt[t] = t == 6u ? n : 0u;
+    if (blockIdx.x == 0u && t < GI_N_COUNTERS) cnt[t] = t == 6u ? n_all : 0u;
     __syncthreads();
     const uint32_t i = first + t;
     if (i >= n) return;
-    const svo_ray r = {s[0][3u * t], s[0][3u * t + 1u], s[0][3u * t + 2u], s[1][3u * t], s[1][3u * t + 1u], s[1][3u * t + 2u], i, 0u};
-    rays[i] = r;
+    const svo_ray r = {s[0][3u * t], s[0][3u * t + 1u], s[0][3u * t + 2u], s[1][3u * t], s[1][3u * t + 1u], s[1][3u * t + 2u],
+                       id0 + i, 0u};
+    rays[id0 + i] = r;
 }
 
-/* svo_res -> tgx_svo_hit for the C ABI, through LDS: out may be the host's
+/* svo_res -> tgx_svo_hit for the C ABI, through LDS: out is the host's
  * memory, to which 40-byte records of single lanes would go in pieces. */
 __global__ __launch_bounds__(256) void svo_hits_k(const svo_gnode* __restrict__ nodes, const svo_res* __restrict__ res,
                                                   uint32_t n, tgx_svo_hit* __restrict__ out)
@@ -2126,32 +2128,29 @@ int tgx_svo_trace(tgx_context* ctx, const float* origins, const float* direction
     if (n == 0) return TGX_OK;
     int rc;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_rays, sizeof(svo_ray) * (size_t)n, "svo rays")) ||
-        (rc = tgx_buffer_reserve(ctx, &ctx->svo_hits, (sizeof(svo_res) + sizeof(tgx_svo_hit)) * (size_t)n, "svo hits")) ||
+        (rc = tgx_buffer_reserve(ctx, &ctx->svo_hits, sizeof(svo_res) * (size_t)n, "svo hits")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->gi_counts, 4ull * GI_CNT_TOTAL, "gi counters")))
-        return rc;
-    /* Host arrays pass through pinned memory that the kernels read and write
-     * themselves: no copies on the stream, no records built on the host. */
-    const size_t in_bytes = 12ull * n, out_bytes = sizeof(tgx_svo_hit) * (size_t)n;
-    const void *in_o = nullptr, *in_d = nullptr;
-    if ((rc = tgx_stage_in(ctx, origins, in_bytes, 0, 2u * in_bytes + out_bytes, &in_o)) ||
-        (rc = tgx_stage_in(ctx, directions, in_bytes, in_bytes, 2u * in_bytes + out_bytes, &in_d)))
         return rc;
     svo_ray* d_rays = (svo_ray*)ctx->svo_rays.ptr;
     svo_res* d_res = (svo_res*)ctx->svo_hits.ptr;
-    tgx_svo_hit* staged = (tgx_svo_hit*)tgx_stage(ctx, 2u * in_bytes + out_bytes);
-    if (staged) staged = (tgx_svo_hit*)((char*)staged + 2u * in_bytes);
-    tgx_svo_hit* d_hits = staged ? staged : (tgx_svo_hit*)(d_res + n);
     uint32_t* cnt = (uint32_t*)ctx->gi_counts.ptr + GI_CNT_SVO;
-    hipLaunchKernelGGL(svo_rays_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, (const float*)in_o, (const float*)in_d, n,
-                       d_rays, cnt);
-    TGX_LAUNCH_CHECK(ctx, "svo_rays_k");
+    if ((rc = tgx_stage_in(ctx, n, 24u, [&](char* p, uint64_t first, uint64_t m) -> int {
+            memcpy(p, origins + 3u * first, 12u * m);
+            memcpy(p + 12u * m, directions + 3u * first, 12u * m);
+            hipLaunchKernelGGL(svo_rays_k, dim3(blocks_for(m)), dim3(256), 0, ctx->stream, (const float*)p,
+                               (const float*)(p + 12u * m), (uint32_t)m, (uint32_t)first, n, d_rays, cnt);
+            TGX_LAUNCH_CHECK(ctx, "svo_rays_k");
+            return TGX_OK;
+        })))
+        return rc;
     if ((rc = launch_trace(ctx, d_rays, cnt + 6, n, max_distance, d_res, nullptr))) return rc;
-    hipLaunchKernelGGL(svo_hits_k, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, (const svo_gnode*)ctx->svo_nodes.ptr,
-                       d_res, n, d_hits);
-    TGX_LAUNCH_CHECK(ctx, "svo_hits_k");
-    if (!staged) TGX_HIP_CHECK(ctx, hipMemcpyAsync(out_host, d_hits, out_bytes, hipMemcpyDeviceToHost, ctx->stream));
-    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    if (staged) memcpy(out_host, staged, out_bytes);
+    if ((rc = tgx_stage_out(ctx, n, sizeof(tgx_svo_hit), out_host, [&](char* p, uint64_t first, uint64_t m) -> int {
+            hipLaunchKernelGGL(svo_hits_k, dim3(blocks_for(m)), dim3(256), 0, ctx->stream,
+                               (const svo_gnode*)ctx->svo_nodes.ptr, d_res + first, (uint32_t)m, (tgx_svo_hit*)p);
+            TGX_LAUNCH_CHECK(ctx, "svo_hits_k");
+            return TGX_OK;
+        })))
+        return rc;
     return TGX_OK;
 }
 

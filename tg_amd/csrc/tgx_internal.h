@@ -62,10 +62,8 @@ struct tgx_context {
     tgx_buffer   vis_stats_dev;  /* frame statistics (records, entries, max)*/
     uint32_t     vis_list_capacity = 0;   /* tile-list entries allocated    */
     uint32_t     vis_list_capacity_fixed = 0; /* caller override, 0 = auto */
-    void*        host_pinned = nullptr; /* small pinned readback area       */
-    void*        stage = nullptr;       /* pinned, see tgx_stage             */
-    size_t       stage_bytes = 0;
-    tgx_buffer   stage_dev;             /* host arrays beyond TGX_STAGE_MAX  */
+    void*        host_pinned = nullptr; /* pinned: TGX_PINNED_SMALL bytes of readback area, then the stage */
+    size_t       stage_at = 0;          /* bytes of the stage in use, see tgx_stage_take */
     tgx_visibility_stats vis_stats = {};
 
     /* Sparse voxel octree (built by tgx_svo_build). */
@@ -163,16 +161,15 @@ int  tgx_fail(tgx_context* ctx, int code, const char* fmt, ...);
 int  tgx_prim_exclusive_scan_u32(tgx_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n);
 int  tgx_prim_sort_pairs_u32(tgx_context* ctx, const uint32_t* keys_in, uint32_t* keys_out,
                              const uint32_t* vals_in, uint32_t* vals_out, uint32_t n, unsigned end_bit);
-/* Pinned memory of at least `bytes` for host arrays that a call takes or gives
- * back, held until the context is destroyed; null beyond TGX_STAGE_MAX or when
- * there is none (callers then copy through device memory). A call that uses it
- * ends with the stream synchronised. */
-#define TGX_STAGE_MAX (32ull << 20)
-void* tgx_stage(tgx_context* ctx, size_t bytes);
-/* The host array src of `bytes`, where a kernel can read it until the call's
- * synchronisation: in the stage at offset `at` of the `all` bytes that the
- * call needs there, or else in device memory. */
-int  tgx_stage_in(tgx_context* ctx, const void* src, size_t bytes, size_t at, size_t all, const void** out);
+/* Host arrays of a call go through the context's stage, pinned memory which
+ * kernels read and write themselves, in pieces of up to TGX_STAGE_PIECE bytes.
+ * A call that uses it ends with tgx_stage_done. Beyond the stage a piece waits
+ * for the earlier ones, so that a larger call needs no more memory. */
+#define TGX_PINNED_SMALL 4096ull
+#define TGX_STAGE_BYTES  (8ull << 20)
+#define TGX_STAGE_PIECE  (4ull << 20)
+int tgx_stage_take(tgx_context* ctx, size_t bytes, char** p);
+int tgx_stage_done(tgx_context* ctx);
 int  tgx_prim_sort_keys_u64(tgx_context* ctx, const uint64_t* keys_in, uint64_t* keys_out, uint32_t n, unsigned end_bit);
 void tgx_svo_release(tgx_context* ctx);
 void tgx_nrc_release(tgx_context* ctx);
@@ -246,5 +243,33 @@ struct tgx_launch_scope {
             return tgx_fail((ctx), TGX_ERR_HIP, "launch of %s failed: %s", (name),        \
                             hipGetErrorString(_e));                                       \
     } while (0)
+
+/* f(piece, first, count): copies the records' bytes there and launches. */
+template <typename F> int tgx_stage_in(tgx_context* ctx, uint64_t n, size_t bytes, F f)
+{
+    const uint64_t per = TGX_STAGE_PIECE / bytes / 256u * 256u;
+    for (uint64_t first = 0; first < n; first += per) {
+        const uint64_t m = n - first < per ? n - first : per;
+        char* p = nullptr;
+        int   rc;
+        if ((rc = tgx_stage_take(ctx, m * bytes, &p)) || (rc = f(p, first, m))) return rc;
+    }
+    return TGX_OK;
+}
+
+/* f(piece, first, count): launches what writes the records; they are then
+ * copied to dst. Ends the call's use of the stage. */
+template <typename F> int tgx_stage_out(tgx_context* ctx, uint64_t n, size_t bytes, void* dst, F f)
+{
+    const uint64_t per = TGX_STAGE_PIECE / bytes / 256u * 256u;
+    for (uint64_t first = 0; first < n; first += per) {
+        const uint64_t m = n - first < per ? n - first : per;
+        char* p = nullptr;
+        int   rc;
+        if ((rc = tgx_stage_take(ctx, m * bytes, &p)) || (rc = f(p, first, m)) || (rc = tgx_stage_done(ctx))) return rc;
+        memcpy((char*)dst + first * bytes, p, m * bytes);
+    }
+    return TGX_OK;
+}
 
 #endif

@@ -458,16 +458,17 @@ struct nrc_adam_args {
 #define NRC_DEV_STEP  1
 #define NRC_DEV_DONE  2   /* blocks of the running Adam step that are done */
 
-/* Records of host samples, zero beyond n, and n itself. The samples are the
+/* Records of n host samples, zero from n to padded, and the count of all. The samples are the
  * host's memory: a block reads its 256 samples' floats once, in order. */
 __global__ __launch_bounds__(256) void nrc_samples_k(const float* __restrict__ samples, uint32_t n, uint32_t padded,
-                                                     gi_surf_rec* __restrict__ out, uint32_t* __restrict__ count)
+                                                     uint32_t n_all, gi_surf_rec* __restrict__ out,
+                                                     uint32_t* __restrict__ count)
 {
     __shared__ float s[9u * 256u];
     const uint32_t first = blockIdx.x * 256u, t = threadIdx.x, i = first + t;
     for (uint32_t k = t; k < 9u * 256u; k += 256u)
         if (9ull * first + k < 9ull * n) s[k] = samples[9ull * first + k];
-    if (i == 0u) *count = n;
+    if (i == 0u) *count = n_all;
     __syncthreads();
     if (i >= padded) return;
     gi_surf_rec r = {};
@@ -837,23 +838,24 @@ int train_step(tgx_context* ctx, const gi_surf_rec* surf, const uint32_t* list, 
     return TGX_OK;
 }
 
-/* Host samples (9 floats) -> surface records in ctx->nrc_samples, with n at
- * the end of the buffer. The kernels read the samples, and write what goes
- * back, in pinned memory themselves (tgx_stage); `all` is what the call needs
- * there, the samples come first. */
-int upload_samples(tgx_context* ctx, const float* samples, uint32_t n, uint32_t padded, size_t all, uint32_t** count_dev)
+/* Host samples (9 floats) -> surface records in ctx->nrc_samples, zero from n
+ * to padded, with n at the end of the buffer. */
+int upload_samples(tgx_context* ctx, const float* samples, uint32_t n, uint32_t padded, uint32_t** count_dev)
 {
     int rc;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->nrc_samples, sizeof(gi_surf_rec) * (size_t)padded + 256, "nrc samples")))
         return rc;
-    const void* src = nullptr;
-    if ((rc = tgx_stage_in(ctx, samples, 36ull * n, 0, all, &src))) return rc;
     char* base = (char*)ctx->nrc_samples.ptr;
     *count_dev = (uint32_t*)(base + sizeof(gi_surf_rec) * (size_t)padded);
-    hipLaunchKernelGGL(nrc_samples_k, dim3(nrc_blocks(padded, 256)), dim3(256), 0, ctx->stream, (const float*)src, n, padded,
-                       (gi_surf_rec*)base, *count_dev);
-    TGX_LAUNCH_CHECK(ctx, "nrc_samples_k");
-    return TGX_OK;
+    return tgx_stage_in(ctx, n, 36u, [&](char* p, uint64_t first, uint64_t m) -> int {
+        memcpy(p, samples + 9u * first, 36u * m);
+        /* the last piece pads */
+        const uint32_t room = first + m == n ? padded - (uint32_t)first : (uint32_t)m;
+        hipLaunchKernelGGL(nrc_samples_k, dim3(nrc_blocks(room, 256)), dim3(256), 0, ctx->stream, (const float*)p,
+                           (uint32_t)m, room, n, (gi_surf_rec*)base + first, *count_dev);
+        TGX_LAUNCH_CHECK(ctx, "nrc_samples_k");
+        return TGX_OK;
+    });
 }
 
 int launch_infer(tgx_context* ctx, const gi_surf_rec* surf, const uint32_t* list, const uint32_t* count_dev,
@@ -974,22 +976,18 @@ int tgx_nrc_infer(tgx_context* ctx, const float* samples, uint32_t n, float* out
     if (n == 0) return TGX_OK;
     if (n > (1u << 26)) return tgx_fail(ctx, TGX_ERR_INVALID_ARG, "at most 2^26 samples per call");
     uint32_t* count_dev = nullptr;
-    const size_t all = (36ull + 12ull) * n;
-    if ((rc = upload_samples(ctx, samples, n, n, all, &count_dev))) return rc;
+    if ((rc = upload_samples(ctx, samples, n, n, &count_dev))) return rc;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->nrc_out, 12ull * n, "nrc outputs"))) return rc;
     if ((rc = launch_infer(ctx, (const gi_surf_rec*)ctx->nrc_samples.ptr, nullptr, count_dev, n,
                            (float*)ctx->nrc_out.ptr, nullptr, nullptr, nullptr, nullptr)))
         return rc;
-    char* staged = (char*)tgx_stage(ctx, all);
-    if (staged) {
-        hipLaunchKernelGGL(nrc_copy_k, dim3(nrc_blocks(3ull * n, 256)), dim3(256), 0, ctx->stream,
-                           (const float*)ctx->nrc_out.ptr, 3ull * n, (float*)(staged + 36ull * n));
-        TGX_LAUNCH_CHECK(ctx, "nrc_copy_k");
-    } else {
-        TGX_HIP_CHECK(ctx, hipMemcpyAsync(out, ctx->nrc_out.ptr, 12ull * n, hipMemcpyDeviceToHost, ctx->stream));
-    }
-    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    if (staged) memcpy(out, staged + 36ull * n, 12ull * n);
+    if ((rc = tgx_stage_out(ctx, 3ull * n, 4u, out, [&](char* p, uint64_t first, uint64_t m) -> int {
+            hipLaunchKernelGGL(nrc_copy_k, dim3(nrc_blocks(m, 256)), dim3(256), 0, ctx->stream,
+                               (const float*)ctx->nrc_out.ptr + first, m, (float*)p);
+            TGX_LAUNCH_CHECK(ctx, "nrc_copy_k");
+            return TGX_OK;
+        })))
+        return rc;
     return TGX_OK;
 }
 
@@ -1003,38 +1001,33 @@ int tgx_nrc_train_batch(tgx_context* ctx, const float* samples, const float* tar
     if (n > (1u << 22)) return tgx_fail(ctx, TGX_ERR_INVALID_ARG, "at most 2^22 samples per batch");
     const uint32_t Bc = (n + NRC_CHUNK - 1) / NRC_CHUNK * NRC_CHUNK;
     uint32_t* count_dev = nullptr;
-    const size_t all = (36ull + 12ull) * n + 4ull * NRC_N + 4ull;
-    if ((rc = upload_samples(ctx, samples, n, Bc, all, &count_dev))) return rc;
+    if ((rc = upload_samples(ctx, samples, n, Bc, &count_dev))) return rc;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->nrc_targets, 12ull * Bc + 16, "nrc targets"))) return rc;
     float* loss_acc = (float*)((char*)ctx->nrc_targets.ptr + 12ull * Bc);
-    const void* t_in = nullptr;
-    if ((rc = tgx_stage_in(ctx, targets, 12ull * n, 36ull * n, all, &t_in))) return rc;
-    /* the targets, and the loss cleared behind them */
-    hipLaunchKernelGGL(nrc_targets_k, dim3(nrc_blocks(3ull * n + 1u, 256)), dim3(256), 0, ctx->stream, (const float*)t_in,
-                       3ull * n, (float*)ctx->nrc_targets.ptr, loss_acc);
-    TGX_LAUNCH_CHECK(ctx, "nrc_targets_k");
+    /* the targets, and the loss cleared behind the last */
+    if ((rc = tgx_stage_in(ctx, 3ull * n, 4u, [&](char* p, uint64_t first, uint64_t m) -> int {
+            memcpy(p, targets + first, 4u * m);
+            hipLaunchKernelGGL(nrc_targets_k, dim3(nrc_blocks(m + 1u, 256)), dim3(256), 0, ctx->stream, (const float*)p, m,
+                               (float*)ctx->nrc_targets.ptr + first, loss_acc);
+            TGX_LAUNCH_CHECK(ctx, "nrc_targets_k");
+            return TGX_OK;
+        })))
+        return rc;
     if ((rc = train_step(ctx, (const gi_surf_rec*)ctx->nrc_samples.ptr, nullptr, count_dev, 0, Bc, n,
                          (const float*)ctx->nrc_targets.ptr, nullptr, nullptr, loss_acc)))
         return rc;
     float l = 0.0f;
-    char* staged = (char*)tgx_stage(ctx, all);
-    float* s_loss = staged ? (float*)(staged + 48ull * n) : nullptr;
-    if (staged) {
-        hipLaunchKernelGGL(nrc_copy_k, dim3(1), dim3(256), 0, ctx->stream, (const float*)loss_acc, 1ull, s_loss);
-        if (grad)
-            hipLaunchKernelGGL(nrc_copy_k, dim3(nrc_blocks(NRC_N, 256)), dim3(256), 0, ctx->stream,
-                               (const float*)ctx->nrc_grad.ptr, (uint64_t)NRC_N, s_loss + 1);
-        TGX_LAUNCH_CHECK(ctx, "nrc_copy_k");
-    } else {
-        TGX_HIP_CHECK(ctx, hipMemcpyAsync(&l, loss_acc, 4, hipMemcpyDeviceToHost, ctx->stream));
-        if (grad)
-            TGX_HIP_CHECK(ctx, hipMemcpyAsync(grad, ctx->nrc_grad.ptr, 4ull * NRC_N, hipMemcpyDeviceToHost, ctx->stream));
-    }
-    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    if (staged) {
-        l = *s_loss;
-        if (grad) memcpy(grad, s_loss + 1, 4ull * NRC_N);
-    }
+    static_assert(4ull * (NRC_N + 1u) <= TGX_STAGE_PIECE, "loss and gradient in one piece");
+    char* p = nullptr;
+    if ((rc = tgx_stage_take(ctx, 4ull * (NRC_N + 1u), &p))) return rc;
+    hipLaunchKernelGGL(nrc_copy_k, dim3(1), dim3(256), 0, ctx->stream, (const float*)loss_acc, 1ull, (float*)p);
+    if (grad)
+        hipLaunchKernelGGL(nrc_copy_k, dim3(nrc_blocks(NRC_N, 256)), dim3(256), 0, ctx->stream,
+                           (const float*)ctx->nrc_grad.ptr, (uint64_t)NRC_N, (float*)p + 1);
+    TGX_LAUNCH_CHECK(ctx, "nrc_copy_k");
+    if ((rc = tgx_stage_done(ctx))) return rc;
+    l = *(const float*)p;
+    if (grad) memcpy(grad, (const float*)p + 1, 4ull * NRC_N);
     if (loss) *loss = l / (3.0f * (float)n);
     return TGX_OK;
 }

@@ -46,37 +46,19 @@ int tgx_buffer_reserve(tgx_context* ctx, tgx_buffer* b, size_t bytes, const char
     return TGX_OK;
 }
 
-void* tgx_stage(tgx_context* ctx, size_t bytes)
+int tgx_stage_take(tgx_context* ctx, size_t bytes, char** p)
 {
-    if (bytes <= ctx->stage_bytes) return ctx->stage;
-    if (bytes > TGX_STAGE_MAX) return nullptr;
-    if (ctx->stage) {
-        (void)hipStreamSynchronize(ctx->stream); /* a call that failed may not have */
-        (void)hipHostFree(ctx->stage);
-    }
-    ctx->stage = nullptr;
-    ctx->stage_bytes = 0;
-    const size_t want = bytes + bytes / 4u < TGX_STAGE_MAX ? bytes + bytes / 4u : TGX_STAGE_MAX;
-    if (hipHostMalloc(&ctx->stage, want, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->stage = nullptr;
-        return nullptr;
-    }
-    ctx->stage_bytes = want;
-    return ctx->stage;
+    int rc;
+    if (ctx->stage_at + bytes > TGX_STAGE_BYTES && (rc = tgx_stage_done(ctx))) return rc;
+    *p = (char*)ctx->host_pinned + TGX_PINNED_SMALL + ctx->stage_at;
+    ctx->stage_at += (bytes + 255u) & ~(size_t)255u;
+    return TGX_OK;
 }
 
-int tgx_stage_in(tgx_context* ctx, const void* src, size_t bytes, size_t at, size_t all, const void** out)
+int tgx_stage_done(tgx_context* ctx)
 {
-    if (char* p = (char*)tgx_stage(ctx, all)) {
-        memcpy(p + at, src, bytes);
-        *out = p + at;
-        return TGX_OK;
-    }
-    int rc;
-    if ((rc = tgx_buffer_reserve(ctx, &ctx->stage_dev, all, "host arrays"))) return rc;
-    *out = (char*)ctx->stage_dev.ptr + at;
-    TGX_HIP_CHECK(ctx, hipMemcpyAsync((void*)*out, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->stage_at = 0;
     return TGX_OK;
 }
 
@@ -152,12 +134,12 @@ int tgx_create(int device, tgx_context** out_ctx)
         delete ctx;
         return TGX_ERR_HIP;
     }
-    if (hipHostMalloc(&ctx->host_pinned, 4096, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&ctx->host_pinned, TGX_PINNED_SMALL + TGX_STAGE_BYTES, hipHostMallocDefault) != hipSuccess) {
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return TGX_ERR_HIP;
     }
-    memset(ctx->host_pinned, 0, 4096);
+    memset(ctx->host_pinned, 0, TGX_PINNED_SMALL);
     if (tgx_vis_scratch_init(ctx) != TGX_OK) {
         (void)hipHostFree(ctx->host_pinned);
         (void)hipStreamDestroy(ctx->stream);
@@ -183,12 +165,11 @@ int tgx_destroy(tgx_context* ctx)
                           &ctx->vis_rec_flags, &ctx->vis_global_keys,
                           &ctx->vis_counters, &ctx->vis_tile_count, &ctx->vis_tile_off,
                           &ctx->vis_tile_list, &ctx->vis_cams, &ctx->vis_out, &ctx->vis_stats_dev,
-                          &ctx->frame_acc, &ctx->pick_buf, &ctx->stage_dev, &ctx->dyn_stage, &ctx->dyn_tmp, &ctx->cl_dirty};
+                          &ctx->frame_acc, &ctx->pick_buf, &ctx->dyn_stage, &ctx->dyn_tmp, &ctx->cl_dirty};
     for (tgx_buffer* b : bufs) tgx_buffer_release(b);
     tgx_svo_release(ctx);
     tgx_nrc_release(ctx);
     if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
-    if (ctx->stage) (void)hipHostFree(ctx->stage);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return TGX_OK;
