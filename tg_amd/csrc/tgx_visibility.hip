@@ -2,15 +2,16 @@
  * tgx_visibility.hip — primary visibility on gfx950.
  *
  * Replaces tg's instanced raster of cluster boxes (visibility.vert:19-26)
- * and the per-fragment DDA (visibility.frag:22-208) with three compute
- * passes per frame:
+ * and the per-fragment DDA (visibility.frag:22-208) with five launches per
+ * call (more where its sizes need a cull or a scan of several launches):
  *
- *   1. vis_setup     one thread per (camera, cluster pointer): drops empty
+ *   0. vis_begin_k   cameras, clears and the cull of whole objects per camera.
+ *   1. vis_setup     one thread per (camera, kept cluster pointer): drops empty
  *                    clusters and clusters no pixel ray can reach, builds
  *                    the cluster's world->cluster frame (exact fp32 order of
  *                    visibility.frag:57-66), a conservative pixel rectangle
  *                    and a lower bound of its depth; counts 16x16 tiles.
- *   2. vis_scan +    tile lists: exclusive scan of the tile counts and a
+ *   2. vis_scan_*_k  tile lists: exclusive scan of the tile counts and a
  *      vis_scatter   scatter of record indices into each covered tile.
  *   3. vis_traverse  one 256-thread workgroup per tile, one pixel per lane,
  *                    each wave an 8x8 pixel block. For each listed cluster
