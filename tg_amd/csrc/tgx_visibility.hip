@@ -1427,7 +1427,8 @@ static int check_args(tgx_context* ctx, const tgx_camera* cams, uint32_t n_cams,
 
 /* Sizes the tile-list buffer. A frame whose lists exceed the capacity is
  * still exact (its overflowing tiles walk every record); the largest total
- * of the last call whose statistics have landed grows the buffer. */
+ * of the last call whose statistics have landed grows the buffer, unless a
+ * frame graph holds it: growth may wait, the call may not fail for it. */
 static int list_capacity_update(tgx_context* ctx, uint32_t w, uint32_t h)
 {
     int rc;
@@ -1444,7 +1445,8 @@ static int list_capacity_update(tgx_context* ctx, uint32_t w, uint32_t h)
     if (ctx->vis_list_capacity_fixed) want = ctx->vis_list_capacity_fixed;
     else {
         const uint64_t max_total = ((volatile const unsigned long long*)ctx->host_pinned)[2];
-        if (max_total > want) want = max_total + max_total / 4u + 1024u;
+        const uint64_t grown = max_total + max_total / 4u + 1024u;
+        if (max_total > want && (ctx->n_graphs == 0 || 8ull * grown <= ctx->vis_tile_list.bytes)) want = grown;
     }
     if (want > 0xFFFFFFFFull) want = 0xFFFFFFFFull;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->vis_tile_list, 8ull * want, "tile list"))) return rc;
