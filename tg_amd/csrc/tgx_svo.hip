@@ -479,6 +479,9 @@ __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict
  * average) no longer makes the launch. 512 objects, depth 11: bits 0.69 -> 0.16
  * ms, materials 0.73 -> 0.29 ms. 512 lanes against 256: 0.16 and 0.20 ms. */
 #define LEAF_BLOCK 512u
+/* A launch holds less than 2^32 lanes along a dimension, and takes more modulo
+ * 2^32 without an error: the leaves' workgroups lie in rows of LEAF_ROW leaves. */
+#define LEAF_ROW (1u << 20)
 #define LEAF_STAGE (LEAF_BLOCK / 8u)
 
 struct leaf_stage {
@@ -600,7 +603,8 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __rest
                                                          const uint32_t* __restrict__ old_list_off,
                                                          const uint32_t* __restrict__ old_list)
 {
-    const uint32_t leaf = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t leaf = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (leaf >= n_leaves) return;
     if (reuse && reuse[leaf] != SVO_NONE) {
         /* an update: same candidate clusters in the same order, none of
          * them new, so the previous build's leaf is this leaf */
@@ -721,8 +725,9 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_mats_k(const svo_gnode* _
                                                               const uint32_t* __restrict__ old_off,
                                                               const uint16_t* __restrict__ old_pool)
 {
-    const uint32_t leaf = blockIdx.x / LEAF_PARTS, part = blockIdx.x % LEAF_PARTS;
+    const uint32_t leaf = blockIdx.y * (gridDim.x / LEAF_PARTS) + blockIdx.x / LEAF_PARTS, part = blockIdx.x % LEAF_PARTS;
     const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    if (leaf >= n_leaves) return;
     if (reuse && reuse[leaf] != SVO_NONE) {
         const uint32_t j = reuse[leaf];
         const uint32_t o = old_off[j], n = old_off[j + 1] - o, d = mat_off[leaf];
@@ -1170,9 +1175,14 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
      * solid voxels only. */
     const uint32_t quirk = (flags & TGX_SVO_FLAG_REFERENCE_CORNER_QUIRK) ? 1u : 0u;
     const uint32_t* rz = update ? reuse.as<uint32_t>() : nullptr;
+    auto leaf_grid = [&](uint32_t per_leaf) {
+        const uint32_t row = n_leaves < LEAF_ROW ? n_leaves : LEAF_ROW;
+        return dim3(per_leaf * row, (n_leaves + row - 1u) / row);
+    };
+    static_assert((uint64_t)LEAF_PARTS * LEAF_ROW * LEAF_BLOCK < 1ull << 32, "lanes of a row");
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_k");
-        hipLaunchKernelGGL(svo_leaf_k, dim3(n_leaves), dim3(LEAF_BLOCK), 0, ctx->stream, nodes, leaf_base,
+        hipLaunchKernelGGL(svo_leaf_k, leaf_grid(1u), dim3(LEAF_BLOCK), 0, ctx->stream, nodes, leaf_base,
                            pair_cptr.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs,
                            n_leaves, frames, (const uint32_t*)ctx->bits.ptr, mn[0], mn[1], mn[2], quirk,
                            (uint32_t*)ctx->svo_leaf_bits.ptr, solid.as<uint32_t>(), (uint16_t*)ctx->svo_leaf_wpre.ptr,
@@ -1207,7 +1217,7 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
     ctx->svo_n_solid = n_solid;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_mats_k");
-        hipLaunchKernelGGL(svo_leaf_mats_k, dim3(n_leaves * LEAF_PARTS), dim3(LEAF_BLOCK), 0, ctx->stream, nodes,
+        hipLaunchKernelGGL(svo_leaf_mats_k, leaf_grid(LEAF_PARTS), dim3(LEAF_BLOCK), 0, ctx->stream, nodes,
                            leaf_base, pair_cptr.as<uint32_t>(),
                            first.as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
                            (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx), mn[0], mn[1], mn[2], quirk,
