@@ -187,9 +187,11 @@ __host__ __device__ static inline uint32_t node_word(uint32_t l)
 
 /* Counters of a build (u32): pairs of level l at l, then the summary the host
  * reads: first node of level l at SVO_CNT_BASE + l, all nodes after the last;
- * leaves that an update took over at SVO_CNT_REUSED. */
+ * leaves that an update took over at SVO_CNT_REUSED; at SVO_CNT_MANY whether a
+ * leaf is svo_leaf_mats_k's (leaf_few). */
 #define SVO_CNT_BASE 16u
 #define SVO_CNT_REUSED 31u
+#define SVO_CNT_MANY 30u
 #define SVO_CNT_N    32u
 
 /* Children of the level's (node, cluster pointer) pairs: eight lanes per pair,
@@ -432,12 +434,14 @@ __global__ __launch_bounds__(256) void svo_pair_split_k(const uint64_t* __restri
 }
 
 /* Totals of two exclusive scans over n counts, written behind the offsets
- * and to the host's out[0..1]; out[2] takes *extra (null: 0). */
+ * and to the host's out[0..1]; out[2] and out[3] take the counters
+ * SVO_CNT_REUSED and SVO_CNT_MANY. */
 __global__ void svo_totals_k(const uint32_t* __restrict__ count0, uint32_t* __restrict__ off0,
                              const uint32_t* __restrict__ count1, uint32_t* __restrict__ off1, uint32_t n,
-                             const uint32_t* __restrict__ extra, uint32_t* __restrict__ out)
+                             const uint32_t* __restrict__ cnt, uint32_t* __restrict__ out)
 {
-    if (threadIdx.x == 2u) out[2] = extra ? *extra : 0u;
+    if (threadIdx.x == 2u) out[2] = cnt[SVO_CNT_REUSED];
+    if (threadIdx.x == 3u) out[3] = cnt[SVO_CNT_MANY];
     if (threadIdx.x > 1u) return;
     const uint32_t* c = threadIdx.x ? count1 : count0;
     uint32_t* o = threadIdx.x ? off1 : off0;
@@ -450,7 +454,7 @@ __global__ void svo_totals_k(const uint32_t* __restrict__ count0, uint32_t* __re
  * leaves, against 14 in three launches, which are what longer counts take. */
 __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict__ count0, uint32_t* __restrict__ off0,
                                                       const uint32_t* __restrict__ count1, uint32_t* __restrict__ off1,
-                                                      uint32_t n, const uint32_t* __restrict__ extra,
+                                                      uint32_t n, const uint32_t* __restrict__ cnt,
                                                       uint32_t* __restrict__ out)
 {
     const uint32_t* c = blockIdx.x ? count1 : count0;
@@ -459,7 +463,7 @@ __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict
     if (threadIdx.x == 0u) {
         o[n] = t;
         out[blockIdx.x] = t;
-        if (blockIdx.x) out[2] = extra ? *extra : 0u;
+        out[2u + blockIdx.x] = cnt[blockIdx.x ? SVO_CNT_MANY : SVO_CNT_REUSED];
     }
 }
 
@@ -482,18 +486,48 @@ __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict
 /* A launch holds less than 2^32 lanes along a dimension, and takes more modulo
  * 2^32 without an error: the leaves' workgroups lie in rows of LEAF_ROW leaves. */
 #define LEAF_ROW (1u << 20)
-#define LEAF_STAGE (LEAF_BLOCK / 8u)
+/* Bits: a leaf of few candidates leaves most of 512 lanes idle and is one chain
+ * of dependent loads, so where the leaves have up to LEAF_SPARSE candidates on
+ * average their workgroups are of LEAF_SPARSE_BLOCK lanes, four times as many at
+ * once. 200 thousand single clusters in 267 thousand leaves: 512 lanes 3.29 ms,
+ * 256 1.19, 128 0.81; 5000 objects of up to 27 clusters 0.23, 0.13, 0.14. From
+ * five to eight on average the two are equal (0.31 ms), below two 128 lanes are
+ * needed (0.46 against 0.17). */
+#define LEAF_SPARSE 4u
+#define LEAF_SPARSE_BLOCK 128u
+/* Materials: leaves of up to LEAF_FEW candidates and LEAF_FEW_SOLID solid
+ * voxels are svo_leaf_mats_few_k's, a workgroup each; the others are
+ * svo_leaf_mats_k's, whose four workgroups clear and read 32768 keys whatever
+ * the leaf holds. 267 thousand leaves of one or two clusters: 10.8 ms there, 1.01
+ * here (2.50 with a limit of 512 voxels); 14 thousand of seven 0.79 and 0.47. The
+ * limits of 8, 16 and 32 candidates measure the same; beyond 2048 voxels 256
+ * lanes take longer than 2048 (646 leaves, limit 4096: 113 us against 71), and
+ * fewer than LEAF_FEW_LEAVES leaves do not fill the chip with one workgroup each
+ * (86 against 71). */
+#define LEAF_FEW 16u
+#define LEAF_FEW_SOLID 2048u
+#define LEAF_FEW_LEAVES 1024u
 
+__device__ static inline bool leaf_few(uint32_t candidates, uint32_t solid, uint32_t few)
+{
+    return candidates <= few && solid <= LEAF_FEW_SOLID;
+}
+
+/* Candidate clusters of a workgroup of kBlock lanes. */
+template <uint32_t kBlock>
 struct leaf_stage {
-    float    c[LEAF_STAGE][24];      /* block corners in cluster space, x y z each */
-    uint32_t lo[LEAF_STAGE];         /* trimmed range: x | y << 8 | z << 16 ... */
-    uint32_t hi[LEAF_STAGE];         /* ... one past it; equal where empty */
-    uint32_t cidx[LEAF_STAGE];
-    uint32_t bits[LEAF_STAGE][16];
+    static constexpr uint32_t kCount = kBlock / 8u;
+    float    c[kCount][24];          /* block corners in cluster space, x y z each */
+    uint32_t lo[kCount];             /* trimmed range: x | y << 8 | z << 16 ... */
+    uint32_t hi[kCount];             /* ... one past it; equal where empty */
+    uint32_t cidx[kCount];
+    uint32_t lut[kCount];
+    uint32_t bits[kCount][16];
 };
 
 /* Stages n clusters from pair_cptr; slices z0 .. z1 of the leaf only. */
-__device__ static inline void leaf_stage_load(leaf_stage& st, const uint32_t* __restrict__ pair_cptr, uint32_t n,
+template <uint32_t kBlock>
+__device__ static inline void leaf_stage_load(leaf_stage<kBlock>& st, const uint32_t* __restrict__ pair_cptr, uint32_t n,
                                               const svo_frame* __restrict__ frames, const uint32_t* __restrict__ bits,
                                               float pminx, float pminy, float pminz, uint32_t quirk, uint32_t z0,
                                               uint32_t z1)
@@ -535,17 +569,44 @@ __device__ static inline void leaf_stage_load(leaf_stage& st, const uint32_t* __
             st.lo[k] = lo[0] | (lo[1] << 8) | (lo[2] << 16);
             st.hi[k] = empty ? st.lo[k] : hi[0] | (hi[1] << 8) | (hi[2] << 16);
             st.cidx[k] = f.cidx;
+            st.lut[k] = f.lut;
         }
     }
-    for (uint32_t j = threadIdx.x; j < 16u * n; j += LEAF_BLOCK)
+    for (uint32_t j = threadIdx.x; j < 16u * n; j += kBlock)
         st.bits[j >> 4][j & 15u] = bits[(size_t)frames[pair_cptr[j >> 4]].cidx * 16u + (j & 15u)];
+}
+
+/* Ends of row (y, z) in cluster space, interpolated over z, then y. */
+__device__ static inline void leaf_row_ends(const float* c, uint32_t y, uint32_t z, float p0[3], float p1[3])
+{
+    const float tz = ((float)z + 0.5f) / 32.0f, omtz = 1.0f - tz;
+    const float ty = ((float)y + 0.5f) / 32.0f, omty = 1.0f - ty;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float pz0 = omtz * c[a] + tz * c[12 + a], pz1 = omtz * c[3 + a] + tz * c[15 + a];
+        const float pz2 = omtz * c[6 + a] + tz * c[18 + a], pz3 = omtz * c[9 + a] + tz * c[21 + a];
+        p0[a] = omty * pz0 + ty * pz2;
+        p1[a] = omty * pz1 + ty * pz3;
+    }
+}
+
+/* The cluster voxel v that the row's sample x falls on; false for none. */
+__device__ static inline bool leaf_voxel(const float p0[3], const float p1[3], uint32_t x, uint32_t& v)
+{
+    const float tx = ((float)x + 0.5f) / 32.0f, omtx = 1.0f - tx;
+    /* 0 <= centre < 8 on each axis as its floor in 0 .. 7 */
+    const uint32_t ix = (uint32_t)(int)floorf(omtx * p0[0] + tx * p1[0]);
+    const uint32_t iy = (uint32_t)(int)floorf(omtx * p0[1] + tx * p1[1]);
+    const uint32_t iz = (uint32_t)(int)floorf(omtx * p0[2] + tx * p1[2]);
+    v = 64u * iz + 8u * iy + ix;
+    return (ix | iy | iz) < 8u;
 }
 
 /* Calls f(row word 32 z + y of the leaf, voxel x, cluster voxel v) for every
  * sample of staged cluster k that falls on a solid voxel, a lane per row;
  * row_done(row word) after each row. Called by whole waves. */
-template <typename F, typename R>
-__device__ static inline void leaf_rows(const leaf_stage& st, uint32_t k, F&& f, R&& row_done)
+template <uint32_t kBlock, typename F, typename R>
+__device__ static inline void leaf_rows(const leaf_stage<kBlock>& st, uint32_t k, F&& f, R&& row_done)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t lo = __builtin_amdgcn_readfirstlane(st.lo[k]), hi = __builtin_amdgcn_readfirstlane(st.hi[k]);
@@ -557,26 +618,11 @@ __device__ static inline void leaf_rows(const leaf_stage& st, uint32_t k, F&& f,
     for (uint32_t r = lane; r < n_rows; r += 64u) {
         const uint32_t q = (r * inv) >> 16;
         const uint32_t y = y0 + r - q * ny, z = z0 + q;
-        const float tz = ((float)z + 0.5f) / 32.0f, omtz = 1.0f - tz;
-        const float ty = ((float)y + 0.5f) / 32.0f, omty = 1.0f - ty;
         float p0[3], p1[3];
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            const float pz0 = omtz * c[a] + tz * c[12 + a], pz1 = omtz * c[3 + a] + tz * c[15 + a];
-            const float pz2 = omtz * c[6 + a] + tz * c[18 + a], pz3 = omtz * c[9 + a] + tz * c[21 + a];
-            p0[a] = omty * pz0 + ty * pz2;
-            p1[a] = omty * pz1 + ty * pz3;
-        }
+        leaf_row_ends(c, y, z, p0, p1);
         for (uint32_t x = x0; x < x1; x++) {
-            const float tx = ((float)x + 0.5f) / 32.0f, omtx = 1.0f - tx;
-            /* 0 <= centre < 8 on each axis as its floor in 0 .. 7 */
-            const uint32_t ix = (uint32_t)(int)floorf(omtx * p0[0] + tx * p1[0]);
-            const uint32_t iy = (uint32_t)(int)floorf(omtx * p0[1] + tx * p1[1]);
-            const uint32_t iz = (uint32_t)(int)floorf(omtx * p0[2] + tx * p1[2]);
-            if ((ix | iy | iz) < 8u) {
-                const uint32_t v = 64u * iz + 8u * iy + ix;
-                if ((st.bits[k][v >> 5] >> (v & 31u)) & 1u) f(x, v, 32u * z + y);
-            }
+            uint32_t v;
+            if (leaf_voxel(p0, p1, x, v) && ((st.bits[k][v >> 5] >> (v & 31u)) & 1u)) f(x, v, 32u * z + y);
         }
         row_done(32u * z + y);
     }
@@ -586,7 +632,8 @@ __device__ static inline void leaf_rows(const leaf_stage& st, uint32_t k, F&& f,
  * index its materials (wpre[w] = solid voxels in the leaf's words before w),
  * its solid voxel count and its list: the clusters with a sample on a solid
  * voxel, in candidate order. */
-__global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __restrict__ nodes, uint32_t leaf_base,
+template <uint32_t kBlock>
+__global__ __launch_bounds__(kBlock) void svo_leaf_k(const svo_gnode* __restrict__ nodes, uint32_t leaf_base,
                                                          const uint32_t* __restrict__ pair_cptr,
                                                          const uint32_t* __restrict__ leaf_first_pair, uint32_t n_pairs,
                                                          uint32_t n_leaves, const svo_frame* __restrict__ frames,
@@ -601,10 +648,14 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __rest
                                                          const uint16_t* __restrict__ old_wpre,
                                                          const uint32_t* __restrict__ old_n,
                                                          const uint32_t* __restrict__ old_list_off,
-                                                         const uint32_t* __restrict__ old_list)
+                                                         const uint32_t* __restrict__ old_list,
+                                                         uint32_t few, uint32_t* __restrict__ n_many)
 {
+    constexpr uint32_t kStage = leaf_stage<kBlock>::kCount;
     const uint32_t leaf = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     if (leaf >= n_leaves) return;
+    const uint32_t b = leaf_first_pair[leaf];
+    const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
     if (reuse && reuse[leaf] != SVO_NONE) {
         /* an update: same candidate clusters in the same order, none of
          * them new, so the previous build's leaf is this leaf */
@@ -613,35 +664,35 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __rest
         uint4* db = (uint4*)(leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS);
         const uint2* sw = (const uint2*)(old_wpre + (size_t)j * TGX_SVO_BLOCK_WORDS);
         uint2* dw = (uint2*)(wpre + (size_t)leaf * TGX_SVO_BLOCK_WORDS);
-        for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS / 4u; w += LEAF_BLOCK) {
+        for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS / 4u; w += kBlock) {
             db[w] = sb[w];
             dw[w] = sw[w];
         }
-        const uint32_t n = old_n[j], b = leaf_first_pair[leaf], o = old_list_off[j];
-        for (uint32_t i = tid; i < n; i += LEAF_BLOCK) list_tmp[b + i] = old_list[o + i];
+        const uint32_t n = old_n[j], o = old_list_off[j];
+        for (uint32_t i = tid; i < n; i += kBlock) list_tmp[b + i] = old_list[o + i];
         if (tid == 0) {
             leaf_n[leaf] = n;
             nodes_rw[leaf_base + leaf].leaf_n = n;
-            leaf_solid[leaf] = old_off[j + 1] - old_off[j];
+            const uint32_t solid = old_off[j + 1] - old_off[j];
+            leaf_solid[leaf] = solid;
+            if (!leaf_few(e - b, solid, few)) *n_many = 1u;
         }
         return;
     }
-    __shared__ leaf_stage st;
+    __shared__ leaf_stage<kBlock> st;
     __shared__ uint32_t lbits[TGX_SVO_BLOCK_WORDS];
-    __shared__ uint32_t s_any[LEAF_STAGE];
-    __shared__ uint32_t wsum[LEAF_BLOCK / 64u];
+    __shared__ uint32_t s_any[kStage];
+    __shared__ uint32_t wsum[kBlock / 64u];
     const svo_gnode nd = nodes[leaf_base + leaf];
     const float pminx = mnx + (float)nd.cx * 32.0f, pminy = mny + (float)nd.cy * 32.0f, pminz = mnz + (float)nd.cz * 32.0f;
-    for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS; w += LEAF_BLOCK) lbits[w] = 0u;
-    const uint32_t b = leaf_first_pair[leaf];
-    const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
+    for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS; w += kBlock) lbits[w] = 0u;
     /* wave 0: list entries so far, and the last flagged cluster */
     uint32_t n_contrib = 0u, last_cidx = SVO_NONE;
-    for (uint32_t s0 = b; s0 < e; s0 += LEAF_STAGE) {
-        const uint32_t n = e - s0 < LEAF_STAGE ? e - s0 : LEAF_STAGE;
+    for (uint32_t s0 = b; s0 < e; s0 += kStage) {
+        const uint32_t n = e - s0 < kStage ? e - s0 : kStage;
         leaf_stage_load(st, pair_cptr + s0, n, frames, bits, pminx, pminy, pminz, quirk, 0u, 32u);
         __syncthreads();
-        for (uint32_t k = wave; k < n; k += LEAF_BLOCK / 64u) {
+        for (uint32_t k = wave; k < n; k += kBlock / 64u) {
             uint32_t mask = 0u, any = 0u;
             leaf_rows(st, k, [&](uint32_t x, uint32_t, uint32_t) { mask |= 1u << x; },
                       [&](uint32_t w) {
@@ -671,10 +722,16 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __rest
         __syncthreads();
     }
     __syncthreads();
-    /* bits, prefix counts and total: two words per thread */
-    const uint32_t w0 = lbits[2u * tid], w1 = lbits[2u * tid + 1u];
-    const uint32_t c0 = (uint32_t)__popc(w0), c1 = (uint32_t)__popc(w1);
-    uint32_t incl = c0 + c1;
+    /* bits, prefix counts and total: kWords words per thread */
+    constexpr uint32_t kWords = TGX_SVO_BLOCK_WORDS / kBlock;
+    uint32_t w[kWords], pre[kWords], cnt = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kWords; k++) {
+        w[k] = lbits[kWords * tid + k];
+        pre[k] = cnt;
+        cnt += (uint32_t)__popc(w[k]);
+    }
+    uint32_t incl = cnt;
 #pragma unroll
     for (uint32_t d = 1; d < 64u; d <<= 1) {
         const uint32_t u = __shfl_up(incl, d);
@@ -682,23 +739,29 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_k(const svo_gnode* __rest
     }
     if (lane == 63u) wsum[wave] = incl;
     __syncthreads();
-    uint32_t run = incl - c0 - c1, total = 0u;
-    for (uint32_t k = 0; k < LEAF_BLOCK / 64u; k++) {
+    uint32_t run = incl - cnt, total = 0u;
+    for (uint32_t k = 0; k < kBlock / 64u; k++) {
         run += k < wave ? wsum[k] : 0u;
         total += wsum[k];
     }
-    ((uint2*)(leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS))[tid] = make_uint2(w0, w1);
-    ((uint32_t*)(wpre + (size_t)leaf * TGX_SVO_BLOCK_WORDS))[tid] = run | ((run + c0) << 16);
+    uint32_t* gb = leaf_bits + (size_t)leaf * TGX_SVO_BLOCK_WORDS + kWords * tid;
+    uint32_t* gp = (uint32_t*)(wpre + (size_t)leaf * TGX_SVO_BLOCK_WORDS) + kWords / 2u * tid;
+#pragma unroll
+    for (uint32_t k = 0; k < kWords; k++) gb[k] = w[k];
+#pragma unroll
+    for (uint32_t k = 0; k < kWords / 2u; k++) gp[k] = (run + pre[2u * k]) | ((run + pre[2u * k + 1u]) << 16);
     if (tid == 0) {
         leaf_n[leaf] = n_contrib;
         nodes_rw[leaf_base + leaf].leaf_n = n_contrib;
         leaf_solid[leaf] = total;
+        if (!leaf_few(e - b, total, few)) *n_many = 1u;
     }
 }
 
-/* Second pass (after the counts are scanned into mat_off), LEAF_PARTS
- * workgroups per leaf, eight z slices each: the materials of the leaf's solid
- * voxels, in bit order, at mat_off[leaf] in the pool. A voxel's material is
+/* Second pass (after the counts are scanned into mat_off) for all leaves but
+ * those of few candidates (leaf_few), LEAF_PARTS workgroups per leaf, eight z
+ * slices each: the materials of the leaf's solid voxels, in bit order, at
+ * mat_off[leaf] in the pool. A voxel's material is
  * that of the first candidate that samples it solid: the samples of a
  * candidate k on cluster voxel v lower the voxel's key to k << 9 | v, so waves
  * run different candidates in any order (a wave's lanes are on rows of the
@@ -723,18 +786,22 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_mats_k(const svo_gnode* _
                                                               uint16_t* __restrict__ pool,
                                                               const uint32_t* __restrict__ reuse,
                                                               const uint32_t* __restrict__ old_off,
-                                                              const uint16_t* __restrict__ old_pool)
+                                                              const uint16_t* __restrict__ old_pool, uint32_t few)
 {
     const uint32_t leaf = blockIdx.y * (gridDim.x / LEAF_PARTS) + blockIdx.x / LEAF_PARTS, part = blockIdx.x % LEAF_PARTS;
     const uint32_t tid = threadIdx.x, wave = tid >> 6;
     if (leaf >= n_leaves) return;
+    const uint32_t b = leaf_first_pair[leaf];
+    const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
+    if (leaf_few(e - b, mat_off[leaf + 1] - mat_off[leaf], few)) return;
     if (reuse && reuse[leaf] != SVO_NONE) {
         const uint32_t j = reuse[leaf];
         const uint32_t o = old_off[j], n = old_off[j + 1] - o, d = mat_off[leaf];
         for (uint32_t i = part * LEAF_BLOCK + tid; i < n; i += LEAF_PARTS * LEAF_BLOCK) pool[d + i] = old_pool[o + i];
         return;
     }
-    __shared__ leaf_stage st;
+    constexpr uint32_t kStage = leaf_stage<LEAF_BLOCK>::kCount;
+    __shared__ leaf_stage<LEAF_BLOCK> st;
     __shared__ uint32_t key[LEAF_SLICES * 1024u];
     __shared__ uint32_t s_bits[LEAF_SLICES * 32u], s_done[LEAF_SLICES * 32u];
     const svo_gnode nd = nodes[leaf_base + leaf];
@@ -745,14 +812,12 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_mats_k(const svo_gnode* _
         s_bits[w] = leaf_bits[word0 + w];
         s_done[w] = 0u;
     }
-    const uint32_t b = leaf_first_pair[leaf];
-    const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
     uint16_t* mats = pool + mat_off[leaf];
     for (uint32_t t0 = b; t0 < e; t0 += 1u << LEAF_SPAN) {
         const uint32_t t1 = e - t0 < (1u << LEAF_SPAN) ? e : t0 + (1u << LEAF_SPAN);
         for (uint32_t v = tid; v < LEAF_SLICES * 1024u; v += LEAF_BLOCK) key[v] = SVO_NONE;
-        for (uint32_t s0 = t0; s0 < t1; s0 += LEAF_STAGE) {
-            const uint32_t n = t1 - s0 < LEAF_STAGE ? t1 - s0 : LEAF_STAGE;
+        for (uint32_t s0 = t0; s0 < t1; s0 += kStage) {
+            const uint32_t n = t1 - s0 < kStage ? t1 - s0 : kStage;
             leaf_stage_load(st, pair_cptr + s0, n, frames, bits, pminx, pminy, pminz, quirk, z0, z0 + LEAF_SLICES);
             __syncthreads();
             for (uint32_t k = wave; k < n; k += LEAF_BLOCK / 64u)
@@ -778,6 +843,76 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_mats_k(const svo_gnode* _
             if ((i & 31u) == 0u) s_done[w] |= (uint32_t)(got >> (tid & 32u));
         }
         __syncthreads();
+    }
+}
+
+/* The same for the leaves of leaf_few, a workgroup per leaf and a lane per solid
+ * voxel in the pool's order: it looks its voxel up in the leaf's prefix counts
+ * and samples it for the candidates in turn until one has it solid (the first
+ * pass found one). Bound by its chain of loads, eight workgroups a CU. */
+#define LEAF_FEW_BLOCK 256u
+__global__ __launch_bounds__(LEAF_FEW_BLOCK) void svo_leaf_mats_few_k(
+    const svo_gnode* __restrict__ nodes, uint32_t leaf_base, const uint32_t* __restrict__ pair_cptr,
+    const uint32_t* __restrict__ leaf_first_pair, uint32_t n_pairs, uint32_t n_leaves,
+    const svo_frame* __restrict__ frames, const uint32_t* __restrict__ bits, const uint8_t* __restrict__ materials,
+    float mnx, float mny, float mnz, uint32_t quirk, const uint32_t* __restrict__ leaf_bits,
+    const uint16_t* __restrict__ wpre, const uint32_t* __restrict__ mat_off, uint16_t* __restrict__ pool,
+    const uint32_t* __restrict__ reuse, const uint32_t* __restrict__ old_off, const uint16_t* __restrict__ old_pool,
+    uint32_t few)
+{
+    const uint32_t leaf = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x;
+    if (leaf >= n_leaves) return;
+    const uint32_t b = leaf_first_pair[leaf];
+    const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
+    const uint32_t n = e - b, off = mat_off[leaf], n_solid = mat_off[leaf + 1] - off;
+    if (!leaf_few(n, n_solid, few)) return;
+    uint16_t* mats = pool + off;
+    if (reuse && reuse[leaf] != SVO_NONE) {
+        const uint16_t* old = old_pool + old_off[reuse[leaf]];
+        for (uint32_t i = tid; i < n_solid; i += LEAF_FEW_BLOCK) mats[i] = old[i];
+        return;
+    }
+    static_assert(LEAF_FEW <= leaf_stage<LEAF_FEW_BLOCK>::kCount, "one stage holds the candidates");
+    __shared__ leaf_stage<LEAF_FEW_BLOCK> st;
+    __shared__ uint32_t s_bits[TGX_SVO_BLOCK_WORDS];
+    __shared__ uint16_t s_pre[TGX_SVO_BLOCK_WORDS];
+    const svo_gnode nd = nodes[leaf_base + leaf];
+    const float pminx = mnx + (float)nd.cx * 32.0f, pminy = mny + (float)nd.cy * 32.0f, pminz = mnz + (float)nd.cz * 32.0f;
+    const size_t word0 = (size_t)leaf * TGX_SVO_BLOCK_WORDS;
+    for (uint32_t w = tid; w < TGX_SVO_BLOCK_WORDS; w += LEAF_FEW_BLOCK) {
+        s_bits[w] = leaf_bits[word0 + w];
+        s_pre[w] = wpre[word0 + w];
+    }
+    leaf_stage_load(st, pair_cptr + b, n, frames, bits, pminx, pminy, pminz, quirk, 0u, 32u);
+    __syncthreads();
+    for (uint32_t i = tid; i < n_solid; i += LEAF_FEW_BLOCK) {
+        /* the last word with a prefix count of up to i, and its bit */
+        uint32_t w = 0u;
+        for (uint32_t s = TGX_SVO_BLOCK_WORDS / 2u; s; s >>= 1)
+            if (s_pre[w + s] <= i) w += s;
+        uint32_t m = s_bits[w], r = i - s_pre[w], x = 0u;
+#pragma unroll
+        for (uint32_t s = 16u; s; s >>= 1) {
+            const uint32_t c = (uint32_t)__popc(m & ((1u << s) - 1u));
+            const bool up = r >= c;
+            r -= up ? c : 0u;
+            x += up ? s : 0u;
+            m = up ? m >> s : m;
+        }
+        const uint32_t y = w & 31u, z = w >> 5;
+        for (uint32_t k = 0; k < n; k++) {
+            const uint32_t lo = st.lo[k], hi = st.hi[k];
+            if (lo == hi || x < (lo & 255u) || x >= (hi & 255u) || y < ((lo >> 8) & 255u) || y >= ((hi >> 8) & 255u) ||
+                z < lo >> 16 || z >= hi >> 16)
+                continue;
+            float p0[3], p1[3];
+            leaf_row_ends(st.c[k], y, z, p0, p1);
+            uint32_t v;
+            if (!leaf_voxel(p0, p1, x, v) || !((st.bits[k][v >> 5] >> (v & 31u)) & 1u)) continue;
+            mats[i] = (uint16_t)(st.lut[k] |
+                                 (materials ? (uint32_t)materials[(size_t)st.cidx[k] * TGX_VOXELS_PER_CLUSTER + v] : 0u));
+            break;
+        }
     }
 }
 
@@ -1175,6 +1310,7 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
      * solid voxels only. */
     const uint32_t quirk = (flags & TGX_SVO_FLAG_REFERENCE_CORNER_QUIRK) ? 1u : 0u;
     const uint32_t* rz = update ? reuse.as<uint32_t>() : nullptr;
+    const uint32_t few = n_leaves >= LEAF_FEW_LEAVES ? LEAF_FEW : 0u;
     auto leaf_grid = [&](uint32_t per_leaf) {
         const uint32_t row = n_leaves < LEAF_ROW ? n_leaves : LEAF_ROW;
         return dim3(per_leaf * row, (n_leaves + row - 1u) / row);
@@ -1182,48 +1318,54 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
     static_assert((uint64_t)LEAF_PARTS * LEAF_ROW * LEAF_BLOCK < 1ull << 32, "lanes of a row");
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_k");
-        hipLaunchKernelGGL(svo_leaf_k, leaf_grid(1u), dim3(LEAF_BLOCK), 0, ctx->stream, nodes, leaf_base,
+        const bool sparse = n_leaf_pairs <= (uint64_t)LEAF_SPARSE * n_leaves;
+        hipLaunchKernelGGL(sparse ? svo_leaf_k<LEAF_SPARSE_BLOCK> : svo_leaf_k<LEAF_BLOCK>, leaf_grid(1u),
+                           dim3(sparse ? LEAF_SPARSE_BLOCK : LEAF_BLOCK), 0, ctx->stream, nodes, leaf_base,
                            pair_cptr.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs,
                            n_leaves, frames, (const uint32_t*)ctx->bits.ptr, mn[0], mn[1], mn[2], quirk,
                            (uint32_t*)ctx->svo_leaf_bits.ptr, solid.as<uint32_t>(), (uint16_t*)ctx->svo_leaf_wpre.ptr,
                            (uint32_t*)ctx->svo_leaf_n.ptr, list_tmp.as<uint32_t>(), nodes, rz,
                            (const uint32_t*)ctx->svo_old_bits.ptr, (const uint32_t*)ctx->svo_old_moff.ptr,
                            (const uint16_t*)ctx->svo_old_wpre.ptr, (const uint32_t*)ctx->svo_old_n.ptr,
-                           (const uint32_t*)ctx->svo_old_list_off.ptr, (const uint32_t*)ctx->svo_old_list.ptr);
+                           (const uint32_t*)ctx->svo_old_list_off.ptr, (const uint32_t*)ctx->svo_old_list.ptr,
+                           few, cnt + SVO_CNT_MANY);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_k");
     /* material offsets and list offsets, their totals read back together */
-    const uint32_t* n_reused = update && n_leaves ? cnt + SVO_CNT_REUSED : (const uint32_t*)nullptr;
     uint32_t* moff = (uint32_t*)ctx->svo_leaf_moff.ptr;
     uint32_t* list_off = (uint32_t*)ctx->svo_list_off.ptr;
     const uint32_t* leaf_n = (const uint32_t*)ctx->svo_leaf_n.ptr;
     if (n_leaves <= SVO_ONE_BLOCK_MAX) {
         hipLaunchKernelGGL(svo_offsets_k, dim3(2), dim3(1024), 0, ctx->stream, solid.as<uint32_t>(), moff, leaf_n, list_off,
-                           n_leaves, n_reused, h);
+                           n_leaves, cnt, h);
     } else {
         if ((rc = tgx_prim_exclusive_scan_u32(ctx, solid.as<uint32_t>(), moff, n_leaves)) ||
             (rc = tgx_prim_exclusive_scan_u32(ctx, leaf_n, list_off, n_leaves)))
             return rc;
         hipLaunchKernelGGL(svo_totals_k, dim3(1), dim3(64), 0, ctx->stream, solid.as<uint32_t>(), moff, leaf_n, list_off,
-                           n_leaves, n_reused, h);
+                           n_leaves, cnt, h);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_offsets_k");
     TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     const uint32_t n_solid = h[0], n_list = h[1];
     ctx->svo_reused = h[2];
+    const bool many = h[3] != 0u;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_mats, 2ull * (n_solid ? n_solid : 1), "svo leaf materials")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_list, 4ull * (n_list ? n_list : 1), "svo list")))
         return rc;
     ctx->svo_n_solid = n_solid;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_mats_k");
-        hipLaunchKernelGGL(svo_leaf_mats_k, leaf_grid(LEAF_PARTS), dim3(LEAF_BLOCK), 0, ctx->stream, nodes,
-                           leaf_base, pair_cptr.as<uint32_t>(),
-                           first.as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
-                           (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx), mn[0], mn[1], mn[2], quirk,
-                           (const uint32_t*)ctx->svo_leaf_bits.ptr, (const uint16_t*)ctx->svo_leaf_wpre.ptr,
-                           (const uint32_t*)ctx->svo_leaf_moff.ptr, (uint16_t*)ctx->svo_leaf_mats.ptr, rz,
-                           (const uint32_t*)ctx->svo_old_moff.ptr, (const uint16_t*)ctx->svo_old_mats.ptr);
+        auto mats = [&](auto kernel, dim3 blocks, uint32_t lanes) {
+            hipLaunchKernelGGL(kernel, blocks, dim3(lanes), 0, ctx->stream, nodes, leaf_base,
+                               pair_cptr.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
+                               (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx), mn[0], mn[1], mn[2], quirk,
+                               (const uint32_t*)ctx->svo_leaf_bits.ptr, (const uint16_t*)ctx->svo_leaf_wpre.ptr,
+                               (const uint32_t*)ctx->svo_leaf_moff.ptr, (uint16_t*)ctx->svo_leaf_mats.ptr, rz,
+                               (const uint32_t*)ctx->svo_old_moff.ptr, (const uint16_t*)ctx->svo_old_mats.ptr, few);
+        };
+        if (few) mats(svo_leaf_mats_few_k, leaf_grid(1u), LEAF_FEW_BLOCK);
+        if (many) mats(svo_leaf_mats_k, leaf_grid(LEAF_PARTS), LEAF_BLOCK);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_mats_k");
     /* Lists; and the traversal layout: leaf brick masks and the leaf grid. */
