@@ -34,3 +34,19 @@ def ctx():
     c = tg_amd.Context(int(os.environ.get("TGX_DEVICE", "0")))
     yield c
     c.close()
+
+
+@pytest.fixture(scope="session")
+def shipped_tuning(ctx):
+    """The tuning a context is created with."""
+    return ctx.tuning().copy()
+
+
+@pytest.fixture(autouse=True)
+def start_from_the_shipped_tuning(request):
+    """A test on the session's context starts from the tuning that users get,
+    whatever the tests before it have set."""
+    if "ctx" in request.fixturenames:
+        t = request.getfixturevalue("shipped_tuning")
+        request.getfixturevalue("ctx").set_tuning(**{k: int(t[k][0]) for k in t.dtype.names})
+    yield
