@@ -15,7 +15,9 @@
  *   exact_root   fl(sqrt(x)), 2^-100 <= x <= 2^100: v_rsq_f32 and one
  *                correction by the remainder; compared likewise.
  *   exact_quot   fl(a / b) from y = fl(1 / b): a y is within 1.5 ulp, and one
- *                correction by the remainder rounds right. The corrected
+ *                correction by the remainder rounds right (P. Markstein,
+ *                "Computation of elementary functions on the IBM RISC
+ *                System/6000 processor", 1990). The corrected
  *                value's distance from a / b is below 2^-22 ulp, so only
  *                quotients that close to the middle of two floats could go
  *                wrong; all 9.3e7 pairs of 24-bit significands with

@@ -335,11 +335,11 @@ int tgx_autotune(tgx_context* ctx, const tgx_camera* cams, uint32_t n_cams, uint
         uint32_t values[6];
     };
     const knob knobs[] = {
-        {&tgx_tuning::trace_regroup, 4u, {0u, 1u, 2u, 4u}},          /* trace launch form, node steps per round */
+        {&tgx_tuning::trace_regroup, 4u, {0u, 1u, 2u, 4u}},          /* trace launch form, moves per round */
         {&tgx_tuning::trace_skip, 2u, {0u, 1u}},                      /* exact empty-brick skip (regrouped form) */
         {&tgx_tuning::trace_blocks_per_cu, 2u, {1u, 2u}},             /* lane-machine workgroups per CU */
         {&tgx_tuning::trace_dda, 2u, {0u, 1u}},                       /* lane-machine DDA without iteration count */
-        {&tgx_tuning::trace_node, 4u, {1u, 2u, 3u, 4u}},              /* node iterations per lane step */
+        {&tgx_tuning::trace_node, 4u, {1u, 2u, 3u, 4u}},              /* moves per lane step */
         {&tgx_tuning::trace_cross, 5u, {0u, 24u, 32u, 40u, 48u}},     /* empty-brick crossing threshold */
         {&tgx_tuning::trace_refill, 6u, {4u, 5u, 6u, 8u, 12u, 16u}}, /* idle lanes that trigger a queue refill */
         {&tgx_tuning::trace_chunk, 3u, {0u, 32u, 64u}},               /* rays per queue cursor atomic */

@@ -19,10 +19,12 @@
  *   grid[8^leaf_level] u32 per 32^3 cell of the root: its leaf, or the size of
  *                    the empty child slot it lies in (SVO_GRID_EMPTY).
  *   bricks[n_leaves] u64 per leaf: one bit per 8^3 brick holding a solid
- *                    voxel, held in LDS when they fit. The 32^3 DDA tests the
- *                    brick bit before it loads a bit word, so most DDA
- *                    iterations read no memory. Voxels tested and their order
- *                    are the reference's; only loads are skipped.
+ *                    voxel, held in LDS when they fit. They say which leaves
+ *                    a ray leaves without a hit (leaf_clear) and which bricks
+ *                    a walk crosses in one step (brick_cross); the counted DDA
+ *                    tests a voxel's brick before it loads the bit word.
+ *                    Results and step counts are those of the reference's
+ *                    voxel-by-voxel walk.
  * Leaves follow the inner nodes in node order, so a leaf's node is n_inner +
  * leaf.
  *
@@ -41,11 +43,12 @@
  * 125 instructions per node of a descent and 35 per pop, both in loops as long
  * as the slowest lane's; a move takes about 165 in all. 512 noise objects at
  * 1080p, 4 samples a pixel: 3.99 -> 2.97 ms, the 4096-object 16-camera frame
- * 92.5 -> 58.3 ms (2 moves and a 12-iteration burst a step, brick crossing from
- * half of the walking lanes; 1, 3 moves 3.16, 3.04 ms, bursts of 8 and 16 3.06
- * and 2.95 ms against 2.93). With the exact short quotients, six voxels at a
- * time, an 18-iteration burst and the arguments read from their segment the
- * first takes 2.28 ms and the second 47.2 ms.
+ * 92.5 -> 58.3 ms. With the exact short quotients, six voxels at a time and the
+ * arguments read from their segment the first takes 2.28 ms and the second 47.2.
+ * A step is 2 moves and an 18-voxel burst, bricks are crossed from 40 of 64
+ * walking lanes on. The 1080p frame, 3.04 ms in all: 1 and 4 moves 3.29 and 3.21,
+ * bursts of 2, 8 and 32 voxels 3.80, 3.13 and 3.33, crossing from 24 lanes 3.08
+ * and never 4.66, a phase vote at 16 and 32 of 64 lanes 3.31 and 3.24.
  *
  * GI frame (estimator documented at tgx_gi_params in tgx.h):
  *   gi_gen_k     surface of each visible pixel, spp bounce rays at
@@ -96,7 +99,6 @@ struct trace_params {
     uint32_t                  n_inner;       /* index of the first leaf node */
     uint32_t                  n_leaves;
     uint32_t                  leaf_level;    /* 2^leaf_level cells per axis */
-    float                     mnx, mny, mnz;
     float                     half;          /* 2^depth / 2 */
     float                     cx, cy, cz;    /* root centre, min + half */
 };
@@ -809,7 +811,8 @@ struct trace_args {
 /* The arguments are read from their segment anew in every step (the empty asm
  * keeps loads from being moved out of the loop): held in scalar registers they
  * and the lane masks did not fit, and the spilled ones came back by v_readlane,
- * 40 of the 200 vector slots of a move. */
+ * 40 of the 200 vector slots of a move. They are the kernel's one parameter, at
+ * offset 0 of the segment: another one before it would move them. */
 template <bool kLds, bool kFused, uint32_t kDda>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void gi_trace_k(const trace_args)
 {
@@ -819,7 +822,8 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
     /* a queue of fewer than small_rays rays is traced by the first
      * small_blocks workgroups (one per CU) alone: with few rays per lane the
      * launch is as long as its slowest rays, which run faster with fewer
-     * waves per SIMD */
+     * waves per SIMD. Below 4 to 64 rays a lane of one workgroup per CU: 960x540
+     * at 2 samples 0.80 ms, 1280x720 at 1 0.77, without it 0.86 and 0.85. */
     const uint32_t n_rays = __builtin_amdgcn_readfirstlane(*A->n_rays);
     const bool small = n_rays < A->small_rays;
     if (small && blockIdx.x >= A->small_blocks) return;
@@ -830,7 +834,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
         __syncthreads();
     }
     const uint32_t lane = threadIdx.x & 63u;
-    /* fused GI: each lane's bounce ray origin and id, behind the nodes; the
+    /* fused GI: each lane's bounce ray origin and id, behind the brick masks; the
      * wave's part of the stash is a uniform base indexed by lane */
     float4* s_ray = (float4*)(s_bricks + (kLds ? ((A->P.n_leaves + 1u) & ~1u) : 0u)) +
                     __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
@@ -929,7 +933,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
         }
         /* phase vote (tuning): a wave runs only DDA bursts in an iteration
          * once at least vote/64 of its active lanes are in a leaf DDA, and
-         * only node steps otherwise */
+         * only moves otherwise */
         bool allow_node = true, allow_dda = true;
         const uint32_t vote = A->vote;
         if (vote) {
@@ -939,9 +943,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
             allow_node = !allow_dda;
         }
         svo_res res;
-        /* per-lane events of this iteration, counted below at a uniform point:
-         * 1 bounce hit, 2 shadow ray started, 4 shadow hit; << 3 for the
-         * second list */
+        /* 1 for a ray that ended with a hit, counted below at a uniform point */
         uint32_t ev = 0u;
         if (lane_step<kLds, false, kDda>(P, s_bricks, half, maxd, L, res, active, allow_node, allow_dda, A->cross,
                                          A->node_iters, A->burst) &&
@@ -1007,19 +1009,20 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8, 
 /* gi_trace_rg_k runs the fused GI launch of gi_trace_k<*, true> with the
  * same per-ray arithmetic, but keeps the waves of a workgroup in one phase:
  * after every step the workgroup sorts its rays by phase (leaf DDA first,
- * then node walk, then idle lanes) through LDS, so a wave runs DDA bursts
- * for (nearly) all of its lanes or node steps and advances for (nearly) all
- * of them, instead of both at partial width. A lane leaving its leaf leaves
- * the advance to the node phase (ND_ADV). Idle lanes collect in the last
- * waves, which refill from the queue 64 rays per atomic. One 1024-lane
- * workgroup per CU; LDS holds the traversal layout (when it fits) and six
- * float4 planes of lane state. */
+ * then moves, then idle lanes) through LDS, so a wave runs DDA bursts for
+ * (nearly) all of its lanes or moves for (nearly) all of them, instead of both
+ * at partial width. A lane leaving its leaf leaves the advance to its next move
+ * (ND_ADV). Idle lanes collect in the last waves, which refill from the queue 64
+ * rays per atomic. One 1024-lane workgroup per CU; LDS holds the brick masks
+ * (when they fit) and six float4 planes of lane state. It walks leaves by the
+ * counted DDA, a voxel at a time: the 1080p frame takes 6.8 ms in this form, 4.9
+ * in gi_trace_k's with the counted DDA and 3.0 in its own. */
 #define RG_BLOCK 1024u
 #define RG_WAVES (RG_BLOCK / 64u)
 #define RG_PLANES 6u
 
 struct rg_ctl {
-    uint32_t cnt[RG_WAVES][2];   /* per wave: DDA lanes, node-walk lanes */
+    uint32_t cnt[RG_WAVES][2];   /* per wave: DDA lanes, moving lanes */
     uint32_t exhausted;
     uint32_t pad[3];
 };
@@ -1068,8 +1071,8 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
                                                              uint32_t node_iters, const trace_fuse F)
 {
     extern __shared__ uint2 s_bricks[];
-    const uint32_t lds_nodes = kLds ? ((P.n_leaves + 1u) & ~1u) : 0u;
-    float4* planes = (float4*)(s_bricks + lds_nodes);
+    const uint32_t n_bricks = kLds ? ((P.n_leaves + 1u) & ~1u) : 0u;
+    float4* planes = (float4*)(s_bricks + n_bricks);
     rg_ctl* ctl = (rg_ctl*)(planes + RG_PLANES * RG_BLOCK);
     if constexpr (kLds) {
         const uint2* gb = (const uint2*)P.bricks;
@@ -1109,8 +1112,8 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
             pending = false;
             active = lane_init_self(P, half, L);
         }
-        /* one step of each lane's phase; node-walk lanes take up to
-         * node_iters steps while the wave has node work */
+        /* one step of each lane's phase; moving lanes take up to node_iters
+         * moves while the wave has some to make */
         const bool was_dda = active && (L.node & ND_DDA);
         for (uint32_t k = 0; k < node_iters; k++) {
             const bool step_dda = k == 0 && was_dda;
@@ -1124,7 +1127,7 @@ __global__ __launch_bounds__(RG_BLOCK, 1) void gi_trace_rg_k(trace_params P, con
                 fused_result(P, F, L, res, slot, ox, oy, oz, sid, pending);
             }
         }
-        /* regroup: DDA lanes first, then node-walk lanes (pending shadow
+        /* regroup: DDA lanes first, then moving lanes (pending shadow
          * rays included), then idle lanes */
         const bool key_d = active && (L.node & ND_DDA);
         const bool key_n = (active || pending) && !key_d;
@@ -1757,16 +1760,15 @@ static trace_params params_of(tgx_context* ctx)
     P.n_inner = ctx->svo_n_inner;
     P.n_leaves = ctx->svo_info.n_leaves;
     P.leaf_level = ctx->svo_info.depth - 5u;
-    P.mnx = ctx->svo_info.min[0]; P.mny = ctx->svo_info.min[1]; P.mnz = ctx->svo_info.min[2];
     /* the kernels' former in-kernel expressions, in the same fp32 order */
     P.half = (float)(1u << ctx->svo_info.depth) * 0.5f;
-    P.cx = P.mnx + P.half; P.cy = P.mny + P.half; P.cz = P.mnz + P.half;
+    P.cx = ctx->svo_info.min[0] + P.half; P.cy = ctx->svo_info.min[1] + P.half; P.cz = ctx->svo_info.min[2] + P.half;
     return P;
 }
 
 /* Persistent trace of the queue rays[0 .. *n_dev) (n_max bounds it):
- * 1024-lane workgroups (tuning: per CU), the traversal layout in LDS when it
- * fits; the queue-segment cursors live in ctx->gi_counts. */
+ * 1024-lane workgroups (tuning: per CU), the brick masks in LDS when they fit;
+ * the queue-segment cursors live in ctx->gi_counts. */
 static int launch_trace(tgx_context* ctx, const svo_ray* rays, const uint32_t* n_dev, uint32_t n_max, float maxd,
                         svo_res* out, uint32_t* hit_counter, const trace_fuse* fuse = nullptr)
 {
@@ -1786,8 +1788,8 @@ static int launch_trace(tgx_context* ctx, const svo_ray* rays, const uint32_t* n
     const uint32_t small_rays = small64 < 0xFFFFFFFFull ? (uint32_t)small64 : 0xFFFFFFFFu;
     {
         tgx_launch_scope s(ctx, "gi_trace_k");
-        /* dynamic LDS: nodes and brick masks (when they fit), then for the
-         * fused GI trace one 16-B ray stash per lane */
+        /* dynamic LDS: brick masks (when they fit), then for the fused GI
+         * trace one 16-B ray stash per lane */
         const bool fused = F.contrib != nullptr;
         const uint32_t stash = fused ? 16u * TRACE_BLOCK : 0u;
         const bool lds = P.n_leaves <= TRACE_LDS_LEAVES_MAX;
@@ -1821,7 +1823,7 @@ static leaf_mat_view leaf_mats_of(const tgx_context* ctx)
 }
 
 /* The fused GI launch as regrouped waves (gi_trace_rg_k): one 1024-lane
- * workgroup per CU, node_iters node steps per round. */
+ * workgroup per CU, node_iters moves per round. */
 static int launch_trace_rg(tgx_context* ctx, const svo_ray* rays, const uint32_t* n_dev, uint32_t n_max, float maxd,
                            uint32_t* cursor, const trace_fuse& F, uint32_t node_iters)
 {
@@ -1833,12 +1835,12 @@ static int launch_trace_rg(tgx_context* ctx, const svo_ray* rays, const uint32_t
     const dim3 grid(want < (uint32_t)cus ? want : (uint32_t)cus);
     const trace_params P = params_of(ctx);
     const size_t state = sizeof(float4) * RG_PLANES * RG_BLOCK + sizeof(rg_ctl);
-    const size_t nodes = 8u * (size_t)((P.n_leaves + 1u) & ~1u);
-    const bool lds = P.n_leaves <= TRACE_LDS_LEAVES_MAX && nodes + state <= (size_t)max_lds;
+    const size_t masks = 8u * (size_t)((P.n_leaves + 1u) & ~1u);
+    const bool lds = P.n_leaves <= TRACE_LDS_LEAVES_MAX && masks + state <= (size_t)max_lds;
     if (state > (size_t)max_lds)
         return tgx_fail(ctx, TGX_ERR_CAPACITY, "regrouped trace needs %zu B of LDS per workgroup, the device has %d",
                         state, max_lds);
-    const size_t shmem = (lds ? nodes : 0u) + state;
+    const size_t shmem = (lds ? masks : 0u) + state;
     const bool skip = ctx->tuning.trace_skip != 0u;
     auto kernel = lds ? (skip ? gi_trace_rg_k<true, true> : gi_trace_rg_k<true, false>)
                       : (skip ? gi_trace_rg_k<false, true> : gi_trace_rg_k<false, false>);

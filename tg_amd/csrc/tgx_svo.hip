@@ -19,7 +19,7 @@
  *                        order (the reference's list order).
  *   4. svo_leaf_k        one workgroup per 32^3 leaf: the trimmed block box of
  *      svo_leaf_mats_k   each candidate cluster is point sampled in the
- *                        reference's exact fp32 order (:242-315); solid bits
+ *      svo_leaf_mats_few_k reference's exact fp32 order (:242-315); solid bits
  *                        collect in LDS, then the material of the first
  *                        candidate that sampled a voxel solid.
  * Traversal and GI live in tgx_gi.hip.

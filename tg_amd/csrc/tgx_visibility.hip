@@ -1254,7 +1254,7 @@ struct vis_bufs {
     uint32_t*           tile_off;
     uint64_t*           list;
     uint32_t            capacity;   /* tile-list entries                   */
-    unsigned long long* stats;      /* 8 u32, cleared by the caller        */
+    unsigned long long* stats;      /* 8 u32, cleared where clear_stats    */
     bool                timed;      /* profiling scopes allowed            */
 };
 
