@@ -484,11 +484,10 @@ struct vis_cam_pack {
  * to its place in cams), cleared tile counts and counters, the call's cleared
  * statistics, and with `cull` the object lists (objects culled and scanned by
  * the one workgroup). One launch of 6 us in place of three fills, a copy and two
- * passes: a call over one object at 256x256 is bound by its launches (66 us with
- * those, a scan in three and statistics copied back; 37 without). Above VIS_CULL_ONE
- * objects (three culled per lane) the cull takes its own grid: with 1024 objects
- * one workgroup takes 8.3 us and the grid 12.3, with 3072 14.6 and 14.9, with
- * 4096 17.9 and 16.9, with 16384 57 and 35. */
+ * passes: a call over one object at 256x256 is bound by its launches. Above
+ * VIS_CULL_ONE objects (three culled per lane) the cull takes its own grid: with
+ * 1024 objects one workgroup takes 8.3 us and the grid 12.3, with 3072 14.6 and
+ * 14.9, with 4096 17.9 and 16.9, with 16384 57 and 35. */
 #define VIS_CULL_ONE 3072u
 __global__ __launch_bounds__(1024) void vis_begin_k(vis_cam_pack pack, uint32_t from_args, vis_cam* __restrict__ cams,
                                                     const tgx_object* __restrict__ objects, uint32_t n_objects,
