@@ -340,7 +340,8 @@ typedef struct tgx_svo_hit {
  * their clusters (tg_sparse_voxel_octree.c:102-317). Each leaf also
  * stores, per solid voxel, (lut_idx << 8 | material) of the first cluster
  * in its list that sampled it. min must be integral; depth in
- * [TGX_SVO_MIN_DEPTH, TGX_SVO_MAX_DEPTH]. */
+ * [TGX_SVO_MIN_DEPTH, TGX_SVO_MAX_DEPTH]. An SVO holds at most 2^24 - 2 nodes
+ * and 2^32 - 1 solid voxels (TGX_ERR_CAPACITY). */
 int tgx_svo_build(tgx_context* ctx, const float min[3], uint32_t depth, uint32_t flags);
 
 /* Rebuilds the SVO after object creates and destroys, with the last

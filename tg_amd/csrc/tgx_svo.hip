@@ -188,10 +188,12 @@ __host__ __device__ static inline uint32_t node_word(uint32_t l)
 /* Counters of a build (u32): pairs of level l at l, then the summary the host
  * reads: first node of level l at SVO_CNT_BASE + l, all nodes after the last;
  * leaves that an update took over at SVO_CNT_REUSED; at SVO_CNT_MANY whether a
- * leaf is svo_leaf_mats_k's (leaf_few). */
+ * leaf is svo_leaf_mats_k's (leaf_few); at SVO_CNT_WRAP whether the leaves'
+ * solid voxels are more than the 32-bit material offsets hold. */
 #define SVO_CNT_BASE 16u
 #define SVO_CNT_REUSED 31u
 #define SVO_CNT_MANY 30u
+#define SVO_CNT_WRAP 29u
 #define SVO_CNT_N    32u
 
 /* Children of the level's (node, cluster pointer) pairs: eight lanes per pair,
@@ -438,15 +440,24 @@ __global__ __launch_bounds__(256) void svo_pair_split_k(const uint64_t* __restri
     if (i == 0u || (uint32_t)(key[i - 1u] >> cptr_bits) != leaf) first_pair[leaf] = i;
 }
 
+/* Notes an exclusive scan whose sums went past 2^32. */
+__global__ __launch_bounds__(256) void svo_wrap_k(const uint32_t* __restrict__ count, const uint32_t* __restrict__ off,
+                                                  uint32_t n, uint32_t* __restrict__ wrapped)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && off[i] + count[i] < off[i]) *wrapped = 1u;
+}
+
 /* Totals of two exclusive scans over n counts, written behind the offsets
- * and to the host's out[0..1]; out[2] and out[3] take the counters
- * SVO_CNT_REUSED and SVO_CNT_MANY. */
+ * and to the host's out[0..1]; out[2] to out[4] take the counters
+ * SVO_CNT_REUSED, SVO_CNT_MANY and SVO_CNT_WRAP. */
 __global__ void svo_totals_k(const uint32_t* __restrict__ count0, uint32_t* __restrict__ off0,
                              const uint32_t* __restrict__ count1, uint32_t* __restrict__ off1, uint32_t n,
                              const uint32_t* __restrict__ cnt, uint32_t* __restrict__ out)
 {
     if (threadIdx.x == 2u) out[2] = cnt[SVO_CNT_REUSED];
     if (threadIdx.x == 3u) out[3] = cnt[SVO_CNT_MANY];
+    if (threadIdx.x == 4u) out[4] = cnt[SVO_CNT_WRAP];
     if (threadIdx.x > 1u) return;
     const uint32_t* c = threadIdx.x ? count1 : count0;
     uint32_t* o = threadIdx.x ? off1 : off0;
@@ -456,7 +467,8 @@ __global__ void svo_totals_k(const uint32_t* __restrict__ count0, uint32_t* __re
 }
 
 /* Both scans with their totals in one launch, a block each: 5 us at 3.4 k
- * leaves, against 14 in three launches, which are what longer counts take. */
+ * leaves, against 14 in three launches, which are what longer counts take. Its
+ * 2^14 leaves of 2^15 voxels cannot pass 2^32. */
 __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict__ count0, uint32_t* __restrict__ off0,
                                                       const uint32_t* __restrict__ count1, uint32_t* __restrict__ off1,
                                                       uint32_t n, const uint32_t* __restrict__ cnt,
@@ -469,6 +481,7 @@ __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict
         o[n] = t;
         out[blockIdx.x] = t;
         out[2u + blockIdx.x] = cnt[blockIdx.x ? SVO_CNT_MANY : SVO_CNT_REUSED];
+        if (blockIdx.x) out[4] = 0u;
     }
 }
 
@@ -1361,11 +1374,15 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
         if ((rc = tgx_prim_exclusive_scan_u32(ctx, solid.as<uint32_t>(), moff, n_leaves)) ||
             (rc = tgx_prim_exclusive_scan_u32(ctx, leaf_n, list_off, n_leaves)))
             return rc;
+        hipLaunchKernelGGL(svo_wrap_k, dim3(blocks_for(n_leaves)), dim3(256), 0, ctx->stream, solid.as<uint32_t>(), moff,
+                           n_leaves, cnt + SVO_CNT_WRAP);
         hipLaunchKernelGGL(svo_totals_k, dim3(1), dim3(64), 0, ctx->stream, solid.as<uint32_t>(), moff, leaf_n, list_off,
                            n_leaves, cnt, h);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_offsets_k");
     TGX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    if (h[4])
+        return tgx_fail(ctx, TGX_ERR_CAPACITY, "the SVO's leaves hold 2^32 solid voxels or more; the limit is 2^32 - 1");
     const uint32_t n_solid = h[0], n_list = h[1];
     ctx->svo_reused = h[2];
     const bool many = h[3] != 0u;
@@ -1627,7 +1644,7 @@ int tgx_svo_load(tgx_context* ctx, const char* path)
                    !(fabsf(in.min[a]) + (float)(1u << (in.depth & 15u)) < 16777216.0f);
     if (in.depth < TGX_SVO_MIN_DEPTH || in.depth > TGX_SVO_MAX_DEPTH || bad_min || in.n_nodes == 0 ||
         in.n_nodes >= 0xFFFFFFu || hd.n_inner > in.n_nodes || in.n_leaves != in.n_nodes - hd.n_inner ||
-        hd.n_solid > (uint64_t)in.n_leaves * TGX_SVO_BLOCK_VOXELS || fsize < 0 || fixed != (uint64_t)fsize)
+        hd.n_solid > (uint64_t)in.n_leaves * TGX_SVO_BLOCK_VOXELS || hd.n_solid > 0xFFFFFFFFull || fsize < 0 || fixed != (uint64_t)fsize)
         return tgx_fail(ctx, TGX_ERR_INVALID_ARG, "%s: inconsistent SVO header or file size", path);
     if (hd.n_clusters != ctx->n_clusters || hd.n_luts != ctx->n_luts)
         return tgx_fail(ctx, TGX_ERR_INVALID_ARG, "%s was built from a scene of %u clusters and %u LUTs, not %u and %u",
