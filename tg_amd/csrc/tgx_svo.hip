@@ -187,8 +187,8 @@ __host__ __device__ static inline uint32_t node_word(uint32_t l)
 
 /* Counters of a build (u32): pairs of level l at l, then the summary the host
  * reads: first node of level l at SVO_CNT_BASE + l, all nodes after the last;
- * leaves that an update took over at SVO_CNT_REUSED; at SVO_CNT_MANY whether a
- * leaf is svo_leaf_mats_k's (leaf_few); at SVO_CNT_WRAP whether the leaves'
+ * leaves that an update took over at SVO_CNT_REUSED; at SVO_CNT_MANY the leaves
+ * that are svo_leaf_mats_k's (leaf_few); at SVO_CNT_WRAP whether the leaves'
  * solid voxels are more than the 32-bit material offsets hold. */
 #define SVO_CNT_BASE 16u
 #define SVO_CNT_REUSED 31u
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict
 #define LEAF_BLOCK 512u
 /* A launch holds less than 2^32 lanes along a dimension, and takes more modulo
  * 2^32 without an error: the leaves' workgroups lie in rows of LEAF_ROW leaves. */
-#define LEAF_ROW (1u << 20)
+#define LEAF_ROW (1u << 18)
 /* Bits: a leaf of few candidates leaves most of 512 lanes idle and is one chain
  * of dependent loads, so where the leaves have up to LEAF_SPARSE candidates on
  * average their workgroups are of LEAF_SPARSE_BLOCK lanes, four times as many at
@@ -521,7 +521,8 @@ __global__ __launch_bounds__(1024) void svo_offsets_k(const uint32_t* __restrict
  * limits of 8, 16 and 32 candidates measure the same; beyond 2048 voxels 256
  * lanes take longer than 2048 (646 leaves, limit 4096: 113 us against 71), and
  * fewer than LEAF_FEW_LEAVES leaves do not fill the chip with one workgroup each
- * (86 against 71). */
+ * (86 against 71). svo_leaf_k lists the others: with a launch over all leaves that
+ * returned for the few, one dense leaf among 449 thousand cost 1.7 ms. */
 #define LEAF_FEW 16u
 #define LEAF_FEW_SOLID 2048u
 #define LEAF_FEW_LEAVES 1024u
@@ -667,7 +668,8 @@ __global__ __launch_bounds__(kBlock) void svo_leaf_k(const svo_gnode* __restrict
                                                          const uint32_t* __restrict__ old_n,
                                                          const uint32_t* __restrict__ old_list_off,
                                                          const uint32_t* __restrict__ old_list,
-                                                         uint32_t few, uint32_t* __restrict__ n_many)
+                                                         uint32_t few, uint32_t* __restrict__ n_many,
+                                                         uint32_t* __restrict__ many)
 {
     constexpr uint32_t kStage = leaf_stage<kBlock>::kCount;
     const uint32_t leaf = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -693,7 +695,7 @@ __global__ __launch_bounds__(kBlock) void svo_leaf_k(const svo_gnode* __restrict
             nodes_rw[leaf_base + leaf].leaf_n = n;
             const uint32_t solid = old_off[j + 1] - old_off[j];
             leaf_solid[leaf] = solid;
-            if (!leaf_few(e - b, solid, few)) *n_many = 1u;
+            if (few && !leaf_few(e - b, solid, few)) many[atomicAdd(n_many, 1u)] = leaf;
         }
         return;
     }
@@ -772,7 +774,7 @@ __global__ __launch_bounds__(kBlock) void svo_leaf_k(const svo_gnode* __restrict
         leaf_n[leaf] = n_contrib;
         nodes_rw[leaf_base + leaf].leaf_n = n_contrib;
         leaf_solid[leaf] = total;
-        if (!leaf_few(e - b, total, few)) *n_many = 1u;
+        if (few && !leaf_few(e - b, total, few)) many[atomicAdd(n_many, 1u)] = leaf;
     }
 }
 
@@ -804,14 +806,15 @@ __global__ __launch_bounds__(LEAF_BLOCK) void svo_leaf_mats_k(const svo_gnode* _
                                                               uint16_t* __restrict__ pool,
                                                               const uint32_t* __restrict__ reuse,
                                                               const uint32_t* __restrict__ old_off,
-                                                              const uint16_t* __restrict__ old_pool, uint32_t few)
+                                                              const uint16_t* __restrict__ old_pool,
+                                                              const uint32_t* __restrict__ many, uint32_t n_many)
 {
-    const uint32_t leaf = blockIdx.y * (gridDim.x / LEAF_PARTS) + blockIdx.x / LEAF_PARTS, part = blockIdx.x % LEAF_PARTS;
+    const uint32_t i_many = blockIdx.y * (gridDim.x / LEAF_PARTS) + blockIdx.x / LEAF_PARTS, part = blockIdx.x % LEAF_PARTS;
     const uint32_t tid = threadIdx.x, wave = tid >> 6;
-    if (leaf >= n_leaves) return;
+    if (i_many >= n_many) return;
+    const uint32_t leaf = many ? many[i_many] : i_many; /* null: all leaves */
     const uint32_t b = leaf_first_pair[leaf];
     const uint32_t e = leaf + 1 < n_leaves ? leaf_first_pair[leaf + 1] : n_pairs;
-    if (leaf_few(e - b, mat_off[leaf + 1] - mat_off[leaf], few)) return;
     if (reuse && reuse[leaf] != SVO_NONE) {
         const uint32_t j = reuse[leaf];
         const uint32_t o = old_off[j], n = old_off[j + 1] - o, d = mat_off[leaf];
@@ -876,7 +879,7 @@ __global__ __launch_bounds__(LEAF_FEW_BLOCK) void svo_leaf_mats_few_k(
     float mnx, float mny, float mnz, uint32_t quirk, const uint32_t* __restrict__ leaf_bits,
     const uint16_t* __restrict__ wpre, const uint32_t* __restrict__ mat_off, uint16_t* __restrict__ pool,
     const uint32_t* __restrict__ reuse, const uint32_t* __restrict__ old_off, const uint16_t* __restrict__ old_pool,
-    uint32_t few)
+    const uint32_t* __restrict__, uint32_t few)
 {
     const uint32_t leaf = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x;
     if (leaf >= n_leaves) return;
@@ -1323,9 +1326,9 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_n, 4ull * nl, "svo leaf n")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_list_off, 4ull * (nl + 1), "svo list offsets")))
         return rc;
-    dbuf list_tmp, solid;
+    dbuf list_tmp, solid, many;
     if ((rc = dalloc(ctx, list_tmp, 4ull * (n_leaf_pairs ? n_leaf_pairs : 1), "svo list")) ||
-        (rc = dalloc(ctx, solid, 4ull * nl, "svo solid counts")))
+        (rc = dalloc(ctx, solid, 4ull * nl, "svo solid counts")) || (rc = dalloc(ctx, many, 4ull * nl, "svo leaves")))
         return rc;
     dbuf reuse;
     if (update && n_leaves) {
@@ -1343,15 +1346,15 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
     const uint32_t quirk = (flags & TGX_SVO_FLAG_REFERENCE_CORNER_QUIRK) ? 1u : 0u;
     const uint32_t* rz = update ? reuse.as<uint32_t>() : nullptr;
     const uint32_t few = n_leaves >= LEAF_FEW_LEAVES ? LEAF_FEW : 0u;
-    auto leaf_grid = [&](uint32_t per_leaf) {
-        const uint32_t row = n_leaves < LEAF_ROW ? n_leaves : LEAF_ROW;
-        return dim3(per_leaf * row, (n_leaves + row - 1u) / row);
+    auto leaf_grid = [](uint32_t n, uint32_t per_leaf) {
+        const uint32_t row = n < LEAF_ROW ? n : LEAF_ROW;
+        return dim3(per_leaf * row, (n + row - 1u) / row);
     };
     static_assert((uint64_t)LEAF_PARTS * LEAF_ROW * LEAF_BLOCK < 1ull << 32, "lanes of a row");
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_k");
         const bool sparse = n_leaf_pairs <= (uint64_t)LEAF_SPARSE * n_leaves;
-        hipLaunchKernelGGL(sparse ? svo_leaf_k<LEAF_SPARSE_BLOCK> : svo_leaf_k<LEAF_BLOCK>, leaf_grid(1u),
+        hipLaunchKernelGGL(sparse ? svo_leaf_k<LEAF_SPARSE_BLOCK> : svo_leaf_k<LEAF_BLOCK>, leaf_grid(n_leaves, 1u),
                            dim3(sparse ? LEAF_SPARSE_BLOCK : LEAF_BLOCK), 0, ctx->stream, nodes, leaf_base,
                            pair_cptr.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs,
                            n_leaves, frames, (const uint32_t*)ctx->bits.ptr, mn[0], mn[1], mn[2], quirk,
@@ -1360,7 +1363,7 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
                            (const uint32_t*)ctx->svo_old_bits.ptr, (const uint32_t*)ctx->svo_old_moff.ptr,
                            (const uint16_t*)ctx->svo_old_wpre.ptr, (const uint32_t*)ctx->svo_old_n.ptr,
                            (const uint32_t*)ctx->svo_old_list_off.ptr, (const uint32_t*)ctx->svo_old_list.ptr,
-                           few, cnt + SVO_CNT_MANY);
+                           few, cnt + SVO_CNT_MANY, many.as<uint32_t>());
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_k");
     /* material offsets and list offsets, their totals read back together */
@@ -1385,23 +1388,24 @@ static int svo_build(tgx_context* ctx, const float mn[3], uint32_t depth, uint32
         return tgx_fail(ctx, TGX_ERR_CAPACITY, "the SVO's leaves hold 2^32 solid voxels or more; the limit is 2^32 - 1");
     const uint32_t n_solid = h[0], n_list = h[1];
     ctx->svo_reused = h[2];
-    const bool many = h[3] != 0u;
+    const uint32_t n_many = few ? h[3] : n_leaves;
     if ((rc = tgx_buffer_reserve(ctx, &ctx->svo_leaf_mats, 2ull * (n_solid ? n_solid : 1), "svo leaf materials")) ||
         (rc = tgx_buffer_reserve(ctx, &ctx->svo_list, 4ull * (n_list ? n_list : 1), "svo list")))
         return rc;
     ctx->svo_n_solid = n_solid;
     if (n_leaves) {
         tgx_launch_scope s(ctx, "svo_leaf_mats_k");
-        auto mats = [&](auto kernel, dim3 blocks, uint32_t lanes) {
+        auto mats = [&](auto kernel, dim3 blocks, uint32_t lanes, uint32_t limit) {
             hipLaunchKernelGGL(kernel, blocks, dim3(lanes), 0, ctx->stream, nodes, leaf_base,
                                pair_cptr.as<uint32_t>(), first.as<uint32_t>(), n_leaf_pairs, n_leaves, frames,
                                (const uint32_t*)ctx->bits.ptr, tgx_scene_materials(ctx), mn[0], mn[1], mn[2], quirk,
                                (const uint32_t*)ctx->svo_leaf_bits.ptr, (const uint16_t*)ctx->svo_leaf_wpre.ptr,
                                (const uint32_t*)ctx->svo_leaf_moff.ptr, (uint16_t*)ctx->svo_leaf_mats.ptr, rz,
-                               (const uint32_t*)ctx->svo_old_moff.ptr, (const uint16_t*)ctx->svo_old_mats.ptr, few);
+                               (const uint32_t*)ctx->svo_old_moff.ptr, (const uint16_t*)ctx->svo_old_mats.ptr,
+                               few ? many.as<uint32_t>() : (uint32_t*)nullptr, limit);
         };
-        if (few) mats(svo_leaf_mats_few_k, leaf_grid(1u), LEAF_FEW_BLOCK);
-        if (many) mats(svo_leaf_mats_k, leaf_grid(LEAF_PARTS), LEAF_BLOCK);
+        if (n_many < n_leaves) mats(svo_leaf_mats_few_k, leaf_grid(n_leaves, 1u), LEAF_FEW_BLOCK, few);
+        if (n_many) mats(svo_leaf_mats_k, leaf_grid(n_many, LEAF_PARTS), LEAF_BLOCK, n_many);
     }
     TGX_LAUNCH_CHECK(ctx, "svo_leaf_mats_k");
     /* Lists; and the traversal layout: leaf brick masks and the leaf grid. */
